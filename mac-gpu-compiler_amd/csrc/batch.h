@@ -20,8 +20,8 @@ constexpr int kBatchMaxRuns = 32;
 // C[m][n] (=, +=) sum_k A'[m][k] W[n][k] for m < M, n < N; A' = A, or A x rowscale[m] x gain[k]
 // (an RMSNorm) when the launch asks for the norm. kGemmSiluPair: W rows 2i / 2i+1 are gate_i /
 // up_i and C[m][i] = silu(gate) * up. N even, K % 32 == 0, lda % 4 == 0.
-// Up to kGemmSkinnyMaxM rows run on the skinny kernel, which computes the norm's row scales
-// itself (rowscale unused, eps used); more rows need rowscale filled by launch_rownorm.
+// Up to kGemmSliceMaxM rows the k-sliced kernel computes the norm's row scales itself (rowscale
+// unused, eps used; K <= kGemmNormMaxK); more rows need rowscale filled by launch_rownorm.
 struct GemmParams {
   const float* A;
   uint32_t lda;
@@ -34,12 +34,12 @@ struct GemmParams {
   float eps;
 };
 
-constexpr uint32_t kGemmSkinnyMaxM = 32;
-// Between kGemmSkinnyMaxM and kGemmTileMinM rows, 64 x 64 tiles (k_gemm_lds). Above, up to
-// kGemmRowsMaxM rows (K a multiple of 64), the 64-row eight-wave kernel (k_gemm_rows8), then
-// 128-row tiles (k_gemm_tile): the faster at each size measured (128, 256, 512, 1024, 2048 rows).
-constexpr uint32_t kGemmTileMinM = 64;
+// Up to kGemmSliceMaxM rows every GEMM runs on k_gemm_kslice. Above, the norm and residual GEMMs of a
+// chunk take the 64-row eight-wave kernel (k_gemm_rows8) up to kGemmRowsMaxM rows (K a multiple of
+// 64), then 128-row tiles (k_gemm_tile): the faster at each size measured (128 .. 2048 rows).
+constexpr uint32_t kGemmSliceMaxM = 64;
 constexpr uint32_t kGemmRowsMaxM = 1024;
+constexpr int kGemmNormMaxK = 4096;
 
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
 // token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
@@ -89,9 +89,6 @@ struct BatchAttnParams {
 };
 
 hipError_t launch_rownorm(const float* x, uint32_t M, uint32_t K, float eps, float* s, hipStream_t st);
-// The L2 prefetch of W [N][K] for the unsplit skinny GEMM (M <= 16): workgroup j reads rows
-// 16 j .. 16 j + 15.
-L2Prefetch skinny_prefetch_target(const uint16_t* W, uint32_t N, uint32_t K);
 hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st);
 // K splits for a split GEMM: enough workgroups to fill the chip, each split a multiple of the
 // kernel's k step deep (1 when K does not split)

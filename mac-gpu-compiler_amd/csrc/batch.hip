@@ -19,31 +19,11 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "gemm_dma.h"
 #include "l2_prefetch.h"
 
 namespace qe {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// 8 floats -> (hi, lo) bf16x8 with hi = bf16(v), lo = bf16(v - hi), both rounded to nearest
-// even by the hardware pair conversion (v_cvt_pk_bf16_f32); hi + lo keeps ~16 mantissa bits
-__device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  u32x4 h, l;
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const uint32_t hb = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{v[2 * e], v[2 * e + 1]}), bf16x2));
-    const float r0 = v[2 * e] - __uint_as_float(hb << 16), r1 = v[2 * e + 1] - __uint_as_float(hb & 0xFFFF0000u);
-    h[e] = hb;
-    l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{r0, r1}), bf16x2));
-  }
-  hi = __builtin_bit_cast(bf16x8, h);
-  lo = __builtin_bit_cast(bf16x8, l);
-}
 
 // ---------------------------------------------------------------------------------------------
 // s[m] = 1 / sqrt(mean_k x[m][k]^2 + eps): one wave per row
@@ -60,219 +40,6 @@ __global__ __launch_bounds__(256) void k_rownorm(const float* __restrict__ x, ui
   }
   acc = wave_sum(acc);
   if (lane == 0) s[row] = 1.0f / sqrtf(acc / float(K) + eps);
-}
-
-// ---------------------------------------------------------------------------------------------
-// GEMM C = A' W^T on v_mfma_f32_16x16x32_bf16. Workgroup tile 64 (m) x 64 (n), 4 waves; wave w
-// owns rows [16w, 16w+16) of the tile and all four 16-column blocks. Per 32-wide k step, lane l
-// loads row (l % 16) of its A block at k = 8 (l / 16) .. +7 (two float4) and the same k range of
-// W rows n0 + 16 j + (l % 16) (one 16-byte load per block), all straight from global memory,
-// four k steps per iteration (the next iteration's loads are issued before this one's MFMAs);
-// A is split into hi + lo bf16 and
-// both halves multiply the same W fragment. Output lane layout: rows 4 (l / 16) + r, column l % 16.
-// Rows past M and columns past N are clamped on load and skipped on store.
-// ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI, int KU>
-__global__ __launch_bounds__(256) void k_gemm(GemmParams p) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kg = lane >> 4;
-  const uint32_t m0 = blockIdx.y * 64 + wave * 16, n0 = blockIdx.x * 64;
-  const uint32_t arow = min(m0 + uint32_t(li), p.M - 1);
-  const float* Ar = p.A + size_t(arow) * p.lda;
-  const float rs = NORM ? p.rowscale[arow] : 1.0f;
-  const uint16_t* Wr[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) Wr[j] = p.W + size_t(min(n0 + 16 * j + li, p.N - 1)) * p.K;  // rows past N clamped
-
-  f32x4 acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // KU k-steps of 32 per iteration, held in registers; the next iteration's are loaded before
-  // this one's MFMAs issue
-  float4 a0[KU], a1[KU];
-  uint4 g[KU], w[KU][4];
-  auto load = [&](uint32_t k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < KU; u++) {
-      const uint32_t k = k0 + 32 * u + 8 * kg;
-      a0[u] = *reinterpret_cast<const float4*>(Ar + k);
-      a1[u] = *reinterpret_cast<const float4*>(Ar + k + 4);
-      if constexpr (NORM) g[u] = *reinterpret_cast<const uint4*>(p.gain + k);
-#pragma unroll
-      for (int j = 0; j < 4; j++) w[u][j] = *reinterpret_cast<const uint4*>(Wr[j] + k);
-    }
-  };
-  load(0);
-  for (uint32_t k0 = 0; k0 < p.K; k0 += 32 * KU) {
-    bf16x8 hi[KU], lo[KU];
-    uint4 wc[KU][4];
-#pragma unroll
-    for (int u = 0; u < KU; u++) {
-      float v[8] = {a0[u].x, a0[u].y, a0[u].z, a0[u].w, a1[u].x, a1[u].y, a1[u].z, a1[u].w};
-      if constexpr (NORM) {
-        const uint32_t gg[4] = {g[u].x, g[u].y, g[u].z, g[u].w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          v[2 * e] = (v[2 * e] * rs) * __uint_as_float(gg[e] << 16);
-          v[2 * e + 1] = (v[2 * e + 1] * rs) * __uint_as_float(gg[e] & 0xFFFF0000u);
-        }
-      }
-      split8(v, hi[u], lo[u]);
-#pragma unroll
-      for (int j = 0; j < 4; j++) wc[u][j] = w[u][j];
-    }
-    if (k0 + 32 * KU < p.K) load(k0 + 32 * KU);
-#pragma unroll
-    for (int u = 0; u < KU; u++) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const bf16x8 b = __builtin_bit_cast(bf16x8, u32x4{wc[u][j].x, wc[u][j].y, wc[u][j].z, wc[u][j].w});
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[u], b, acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[u], b, acc[j], 0, 0, 0);
-      }
-    }
-  }
-
-  // epilogue: lane holds C[m0 + 4 kg + r][n0 + 16 j + li]
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint32_t n = n0 + 16 * j + li;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const uint32_t m = m0 + 4 * kg + r;
-      const float c = acc[j][r];
-      if constexpr (EPI == kGemmSiluPair) {
-        // columns 2i (gate) and 2i+1 (up) sit in neighbouring lanes (cpu_inference.rs:170)
-        const float up = __shfl_xor(c, 1);
-        if (m < p.M && n < p.N && (li & 1) == 0) p.C[size_t(m) * p.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-      } else if constexpr (EPI == kGemmResAdd) {
-        if (m < p.M && n < p.N) p.C[size_t(m) * p.ldc + n] += c;
-      } else {
-        if (m < p.M && n < p.N) p.C[size_t(m) * p.ldc + n] = c;
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Tiled GEMM, K % 64 == 0: workgroup tile 64 (m) x 64 (n), 4 waves; wave w owns rows
-// [16 w, 16 w + 16) and all four 16-column blocks. The W tile of each 64-deep stage is loaded
-// once per workgroup into LDS (three buffers, rows padded to 72 bf16 so that the 16 rows a
-// fragment read touches land in distinct banks) and shared by the four waves; each wave's A
-// rows go straight to registers, split hi + lo. Loads run two stages ahead of the MFMAs.
-// gridDim.z > 1 splits K: split z covers K / gridDim.z and writes
-// its partial sums (kGemmPartial) to C + z M ldc.
-// ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI>
-__global__ __launch_bounds__(256) void k_gemm_lds(GemmParams p) {
-  constexpr int BK = 64, WP = BK + 8;
-  __shared__ __align__(16) uint16_t ws[3][64][WP];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kg = lane >> 4;
-  const uint32_t m0 = blockIdx.y * 64 + wave * 16, n0 = blockIdx.x * 64;
-  const uint32_t kz = p.K / gridDim.z, kbeg = blockIdx.z * kz, nst = kz / BK;
-  const uint32_t arow = min(m0 + uint32_t(li), p.M - 1);
-  const float* Ar = p.A + size_t(arow) * p.lda + kbeg + 8 * kg;
-  const float rs = NORM ? p.rowscale[arow] : 1.0f;
-  const uint16_t* gp = NORM ? p.gain + kbeg + 8 * kg : nullptr;
-  // W stage: 64 rows x 8 chunks of 16 B; thread t moves chunks t and t + 256
-  const uint16_t* Wsrc[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int c = tid + 256 * i;
-    Wsrc[i] = p.W + size_t(min(n0 + uint32_t(c >> 3), p.N - 1)) * p.K + kbeg + 8 * (c & 7);
-  }
-  // one stage in registers: its W chunks (bound for LDS), A fragments and gains
-  struct Stage {
-    u32x4 w[2];
-    f32x4 a[2][2];
-    u32x4 g[2];
-  };
-  auto load = [&](Stage& r, uint32_t stg) __attribute__((always_inline)) {
-    const uint32_t k = stg * BK;
-#pragma unroll
-    for (int i = 0; i < 2; i++) r.w[i] = *reinterpret_cast<const u32x4*>(Wsrc[i] + k);
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      r.a[u][0] = *reinterpret_cast<const f32x4*>(Ar + k + 32 * u);
-      r.a[u][1] = *reinterpret_cast<const f32x4*>(Ar + k + 32 * u + 4);
-      if constexpr (NORM) r.g[u] = *reinterpret_cast<const u32x4*>(gp + k + 32 * u);
-    }
-  };
-  auto store_w = [&](const Stage& r, uint32_t buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int c = tid + 256 * i;
-      *reinterpret_cast<u32x4*>(&ws[buf][c >> 3][8 * (c & 7)]) = r.w[i];
-    }
-  };
-  f32x4 acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Software pipeline over three LDS buffers: at step s the W tile of stage s is in buffer
-  // s % 3, stage s + 1's W (loaded one step earlier) goes to buffer (s + 1) % 3, whose last
-  // readers were at step s - 2, and stage s + 2 is loaded into the registers stage s vacates.
-  auto step = [&](Stage& cur, Stage& nxt, uint32_t s) __attribute__((always_inline)) {
-    store_w(nxt, (s + 1) % 3);
-    bf16x8 hi[2], lo[2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      float v[8] = {cur.a[u][0][0], cur.a[u][0][1], cur.a[u][0][2], cur.a[u][0][3],
-                    cur.a[u][1][0], cur.a[u][1][1], cur.a[u][1][2], cur.a[u][1][3]};
-      if constexpr (NORM) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          v[2 * e] = (v[2 * e] * rs) * __uint_as_float(cur.g[u][e] << 16);
-          v[2 * e + 1] = (v[2 * e + 1] * rs) * __uint_as_float(cur.g[u][e] & 0xFFFF0000u);
-        }
-      }
-      split8(v, hi[u], lo[u]);
-    }
-    load(cur, min(s + 2, nst - 1));  // unconditional: the last stages reload the last one
-    if (s < nst) {                   // an odd stage count ends with one empty step
-      const uint32_t buf = s % 3;
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const bf16x8 b = *reinterpret_cast<const bf16x8*>(&ws[buf][16 * j + li][32 * u + 8 * kg]);
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[u], b, acc[j], 0, 0, 0);
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[u], b, acc[j], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
-  };
-  Stage r0, r1;
-  load(r0, 0);
-  load(r1, min(1u, nst - 1));
-  store_w(r0, 0);
-  __syncthreads();
-  for (uint32_t s = 0; s < nst; s += 2) {
-    step(r0, r1, s);
-    step(r1, r0, s + 1);
-  }
-
-  // epilogue: lane holds C[m0 + 4 kg + r][n0 + 16 j + li]
-  float* C = p.C + (EPI == kGemmPartial ? size_t(blockIdx.z) * p.M * p.ldc : 0);
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint32_t n = n0 + 16 * j + li;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const uint32_t m = m0 + 4 * kg + r;
-      const float c = acc[j][r];
-      if constexpr (EPI == kGemmSiluPair) {
-        const float up = __shfl_xor(c, 1);  // columns 2i (gate) and 2i+1 (up) in neighbouring lanes
-        if (m < p.M && n < p.N && (li & 1) == 0) C[size_t(m) * p.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-      } else if constexpr (EPI == kGemmResAdd) {
-        if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] += c;
-      } else {
-        if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] = c;
-      }
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -645,142 +412,6 @@ __global__ __launch_bounds__(256) void k_resadd_partials(float* __restrict__ x, 
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   if (tid == 0) s[m] = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / float(N) + eps);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Skinny GEMM for M <= 16 MT rows (verify, the last chunk of a prefill): the weights are the
-// whole cost, so the work is spread over K as well as N. Workgroup = NW waves on 16 columns
-// n0 .. n0+15 and the K range of split blockIdx.y (gridDim.y > 1: kGemmPartial sums to
-// C + split M ldc); wave w covers the k steps [w KPW, (w+1) KPW) with KPW = ceil(K / 32 / NW),
-// KMAX at a time with every load of the batch issued before any use (clamped to the last step;
-// steps past the range masked by a zero W fragment), MT m-tiles per W fragment, A split
-// hi + lo as in k_gemm. The NW partial tiles are summed in LDS in wave order. With the norm,
-// each lane also sums x^2 of its row over the steps it loads, so
-// C = s[m] sum_k (x g)[m][k] W[n][k] with s[m] = 1 / sqrt(mean x^2 + eps) (the scale applied
-// after the sum, a reassociation of the reference's f32 product).
-// ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI, int MT, int NW, int KMAX>
-__global__ __launch_bounds__(64 * NW) void k_gemm_skinny(GemmParams p) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kg = lane >> 4;
-  const uint32_t n0 = blockIdx.x * 16;
-  const uint32_t kz = p.K / gridDim.y, kbeg = blockIdx.y * kz;  // this split's k range
-  const uint32_t KS = kz / 32, KPW = (KS + NW - 1) / NW, s0 = uint32_t(wave) * KPW;
-  const uint16_t* Wr = p.W + size_t(min(n0 + uint32_t(li), p.N - 1)) * p.K + kbeg + 8 * kg;
-  const float* Ar[MT];
-#pragma unroll
-  for (int t = 0; t < MT; t++) Ar[t] = p.A + size_t(min(uint32_t(16 * t + li), p.M - 1)) * p.lda + kbeg + 8 * kg;
-  const uint16_t* gp = NORM ? p.gain + kbeg + 8 * kg : nullptr;
-
-  f32x4 acc[MT];
-  float ss[MT];
-#pragma unroll
-  for (int t = 0; t < MT; t++) {
-    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    ss[t] = 0.f;
-  }
-  for (uint32_t base = 0; base < KPW; base += KMAX) {
-    u32x4 w[KMAX], g[KMAX];
-    f32x4 a0[KMAX][MT], a1[KMAX][MT];
-#pragma unroll
-    for (int u = 0; u < KMAX; u++) {
-      const uint32_t k = 32 * min(s0 + base + uint32_t(u), KS - 1);
-      w[u] = *reinterpret_cast<const u32x4*>(Wr + k);
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        a0[u][t] = *reinterpret_cast<const f32x4*>(Ar[t] + k);
-        a1[u][t] = *reinterpret_cast<const f32x4*>(Ar[t] + k + 4);
-      }
-      if constexpr (NORM) g[u] = *reinterpret_cast<const u32x4*>(gp + k);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < KMAX; u++) {
-      const bool ok = base + u < KPW && s0 + base + u < KS;
-      const u32x4 wc = ok ? w[u] : u32x4{0u, 0u, 0u, 0u};
-      const bf16x8 b = __builtin_bit_cast(bf16x8, wc);
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        float v[8] = {a0[u][t][0], a0[u][t][1], a0[u][t][2], a0[u][t][3],
-                      a1[u][t][0], a1[u][t][1], a1[u][t][2], a1[u][t][3]};
-        if constexpr (NORM) {
-          float q = 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; e++) q += v[e] * v[e];
-          ss[t] += ok ? q : 0.f;
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            v[2 * e] *= __uint_as_float(g[u][e] << 16);
-            v[2 * e + 1] *= __uint_as_float(g[u][e] & 0xFFFF0000u);
-          }
-        }
-        bf16x8 hi, lo;
-        split8(v, hi, lo);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, b, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, b, acc[t], 0, 0, 0);
-      }
-    }
-  }
-
-  // partial tiles: lane holds rows 16 t + 4 kg + r, column li
-  __shared__ float part[NW][MT * 16][17];
-  __shared__ float ssp[NW][MT * 16];
-#pragma unroll
-  for (int t = 0; t < MT; t++) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) part[wave][16 * t + 4 * kg + r][li] = acc[t][r];
-    if constexpr (NORM) {
-      float q = ss[t];
-      q += __shfl_xor(q, 16);
-      q += __shfl_xor(q, 32);
-      if (kg == 0) ssp[wave][16 * t + li] = q;
-    }
-  }
-  __syncthreads();
-  float* C = p.C + (EPI == kGemmPartial ? size_t(blockIdx.y) * p.M * p.ldc : 0);
-  // MT * 256 outputs over the workgroup's threads; each pass covers whole waves
-  for (uint32_t o = uint32_t(tid); o < uint32_t(MT * 256); o += uint32_t(64 * NW)) {
-    const uint32_t row = o >> 4, col = o & 15;
-    float c = 0.f;
-#pragma unroll
-    for (int v = 0; v < NW; v++) c += part[v][row][col];
-    if constexpr (NORM) {
-      float q = 0.f;
-#pragma unroll
-      for (int v = 0; v < NW; v++) q += ssp[v][row];
-      c *= 1.0f / sqrtf(q / float(p.K) + p.eps);
-    }
-    const uint32_t m = row, n = n0 + col;
-    if constexpr (EPI == kGemmSiluPair) {
-      const float up = __shfl_xor(c, 1);  // column n ^ 1 of the same row
-      if (m < p.M && n < p.N && (col & 1) == 0) C[size_t(m) * p.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-    } else if constexpr (EPI == kGemmResAdd) {
-      if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] += c;
-    } else {
-      if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] = c;
-    }
-  }
-}
-
-// skinny launch: MT m-tiles, NW waves (4 when K is split over workgroups, else 8), and the
-// batch of k steps loaded at once sized to the steps per wave
-template <bool NORM, int EPI>
-void launch_skinny(const GemmParams& p, uint32_t splits, hipStream_t st) {
-  const uint32_t NW = splits > 1 ? 4 : 8, KPW = ceil_div(p.K / splits / 32, NW);
-  const dim3 grid(ceil_div(p.N, 16), splits);
-  const bool two = p.M > 16, wide_k = KPW > 4;
-#define QE_SK(MT, W, KM) hipLaunchKernelGGL((k_gemm_skinny<NORM, EPI, MT, W, KM>), grid, dim3(64 * W), 0, st, p)
-  // two m-tiles always load four steps at a time (eight do not fit their registers)
-  if (NW == 4) {
-    if (two) QE_SK(2, 4, 4);
-    else if (wide_k) QE_SK(1, 4, 8);
-    else QE_SK(1, 4, 4);
-  } else {
-    if (two) QE_SK(2, 8, 4);
-    else if (wide_k) QE_SK(1, 8, 8);
-    else QE_SK(1, 8, 4);
-  }
-#undef QE_SK
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1203,7 +834,7 @@ uint32_t tile_bn(uint32_t M, uint32_t N) { return ceil_div(M, 128) * ceil_div(N,
 constexpr int kTileDepth = 2;
 
 // k_gemm_rows8 serves M rows of a K-deep product
-bool rows_kernel(uint32_t M, uint32_t K) { return M > kGemmTileMinM && M <= kGemmRowsMaxM && K % 64 == 0; }
+bool rows_kernel(uint32_t M, uint32_t K) { return M > kGemmSliceMaxM && M <= kGemmRowsMaxM && K % 64 == 0; }
 
 // k_gemm_rows8 over `splits` K splits (K % (64 splits) == 0, checked by the callers)
 // Column tile of k_gemm_rows8 for an unsplit launch. The kernel is bound by what a CU pulls from
@@ -1709,110 +1340,127 @@ hipError_t launch_mv_rows(const MvRowsParams& p, bool norm, int epi, hipStream_t
   }
 }
 
-L2Prefetch skinny_prefetch_target(const uint16_t* W, uint32_t N, uint32_t K) {
-  return L2Prefetch{W, N * (K / 8), 16 * (K / 8), ceil_div(N, 16u)};
-}
-
 hipError_t launch_rownorm(const float* x, uint32_t M, uint32_t K, float eps, float* s, hipStream_t st) {
   if (M == 0 || K % 4) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_rownorm, dim3(ceil_div(M, 4)), dim3(256), 0, st, x, M, K, eps, s);
   return hipGetLastError();
 }
 
+namespace {
+
+// The tile of a k-sliced launch: the workgroups are dealt over 256 CUs, so its time goes with the
+// bytes the busiest CU loads (rounds of 256 x one workgroup's), plus what a workgroup costs besides
+// its loads, worth about 60 KB of them. Measured (us, M x N x K): 9 x 6144 x 1024 on 16 x 32 tiles
+// 3.5, 16 x 48 4.0; 64 x 6144 x 1024 on 32 x 48 5.8, 32 x 64 6.0, 16 x 32 7.3; 130 x 1024 x 3072 on
+// 32 x 32 7.5, 32 x 64 9.0, 16 x 32 9.5; 130 x 4096 x 1024 on 48 x 64 7.3, 64 x 64 7.9, 32 x 64 10.1;
+// 512 x 1024 x 3072 on 32 x 64 15.1, 48 x 64 17.6, 64 x 64 20.4.
+uint64_t tile_cost(const GemmParams& p, uint32_t bm, uint32_t bn) {
+  const uint64_t wgs = (uint64_t(p.M) + bm - 1) / bm * ((uint64_t(p.N) + bn - 1) / bn);
+  return (wgs + 255) / 256 * (uint64_t(4 * bm + 2 * bn) * p.K + 60 * 1024);
+}
+
+hipError_t check_grid(uint64_t wgs, uint32_t threads) {
+  return wgs * threads < (uint64_t(1) << 32) ? hipSuccess : hipErrorInvalidValue;
+}
+
+template <bool NORM, int EPI, int MT, int NT, int NW, int NS>
+hipError_t launch_kslice_t(const GemmParams& p, hipStream_t st) {
+  const uint64_t wgs = (uint64_t(p.M) + 16 * MT - 1) / (16 * MT) * ((uint64_t(p.N) + 16 * NT - 1) / (16 * NT));
+  if (hipError_t e = check_grid(wgs, 64 * NW)) return e;
+  hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
+  return hipGetLastError();
+}
+
+template <bool NORM, int EPI>
+hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
+  if (NORM && p.K > uint32_t(kGemmNormMaxK)) return hipErrorInvalidValue;
+  const uint32_t tile[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64}, {48, 64}, {64, 64}, {64, 128}};
+  int best = 0;
+  for (int i = 1; i < 8; i++)
+    if (tile_cost(p, tile[i][0], tile[i][1]) < tile_cost(p, tile[best][0], tile[best][1])) best = i;
+  switch (best) {
+    case 0: return launch_kslice_t<NORM, EPI, 1, 1, 8, 4>(p, st);
+    case 1: return launch_kslice_t<NORM, EPI, 1, 2, 8, 2>(p, st);
+    case 2: return launch_kslice_t<NORM, EPI, 2, 2, 8, 2>(p, st);
+    case 3: return launch_kslice_t<NORM, EPI, 2, 3, 8, 2>(p, st);
+    case 4: return launch_kslice_t<NORM, EPI, 2, 4, 8, 2>(p, st);
+    case 5: return launch_kslice_t<NORM, EPI, 3, 4, 8, 1>(p, st);
+    case 6: return launch_kslice_t<NORM, EPI, 4, 4, 8, 1>(p, st);
+    default: return launch_kslice_t<NORM, EPI, 4, 8, 4, 2>(p, st);
+  }
+}
+
+template <int EPI, int BM, int BN, int NS>
+hipError_t launch_wide_t(const GemmParams& p, hipStream_t st) {
+  const uint64_t wgs = (uint64_t(p.M) + BM - 1) / BM * ((uint64_t(p.N) + BN - 1) / BN);
+  if (hipError_t e = check_grid(wgs, 512)) return e;
+  hipLaunchKernelGGL((k_gemm_wide<EPI, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p);
+  return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t launch_wide(const GemmParams& p, hipStream_t st) {
+  const uint64_t c128 = tile_cost(p, 64, 128), c192 = tile_cost(p, 64, 192), c256 = tile_cost(p, 128, 256);
+  if (c256 < c128 && c256 < c192) return launch_wide_t<EPI, 128, 256, 2>(p, st);
+  if (c192 >= c128) return launch_wide_t<EPI, 64, 128, 2>(p, st);
+  // one workgroup per CU: three slots; more: two slots, two workgroups per CU
+  const uint64_t wgs = (uint64_t(p.M) + 63) / 64 * ((uint64_t(p.N) + 191) / 192);
+  return wgs <= 256 ? launch_wide_t<EPI, 64, 192, 3>(p, st) : launch_wide_t<EPI, 64, 192, 2>(p, st);
+}
+
+}  // namespace
+
 hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st) {
   if (p.M == 0 || p.N == 0 || p.N % 2 || p.K % 32 || p.K == 0 || p.lda % 4 || !p.A || !p.W || !p.C)
     return hipErrorInvalidValue;
   if (norm && !p.gain) return hipErrorInvalidValue;
-  if (p.M <= kGemmSkinnyMaxM) {
-    if (norm && epi == kGemmStore) launch_skinny<true, kGemmStore>(p, 1, st);
-    else if (norm && epi == kGemmSiluPair) launch_skinny<true, kGemmSiluPair>(p, 1, st);
-    else if (!norm && epi == kGemmStore) launch_skinny<false, kGemmStore>(p, 1, st);
-    else if (!norm && epi == kGemmResAdd) launch_skinny<false, kGemmResAdd>(p, 1, st);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+  if (p.M <= kGemmSliceMaxM) {
+    if (norm && epi == kGemmStore) return launch_kslice<true, kGemmStore>(p, st);
+    if (norm && epi == kGemmSiluPair) return launch_kslice<true, kGemmSiluPair>(p, st);
+    if (!norm && epi == kGemmResAdd) return launch_kslice<false, kGemmResAdd>(p, st);
+  }
+  if (!norm && epi == kGemmStore) {
+    // the k-sliced kernel up to two rounds of its smaller tiles, the wide one past that
+    uint64_t slice = ~uint64_t(0);
+    for (uint32_t bm : {32u, 48u, 64u}) slice = std::min(slice, tile_cost(p, bm, 64));
+    const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM &&
+                      std::min({tile_cost(p, 64, 128), tile_cost(p, 64, 192), tile_cost(p, 128, 256)}) < slice;
+    return wide ? launch_wide<kGemmStore>(p, st) : launch_kslice<false, kGemmStore>(p, st);
   }
   if (norm && !p.rowscale) return hipErrorInvalidValue;
   if (rows_kernel(p.M, p.K)) {
     if (norm && epi == kGemmStore) launch_rows<true, kGemmStore>(p, 1, st);
     else if (norm && epi == kGemmSiluPair) launch_rows<true, kGemmSiluPair>(p, 1, st);
-    else if (!norm && epi == kGemmStore) launch_rows<false, kGemmStore>(p, 1, st);
     else if (!norm && epi == kGemmResAdd) launch_rows<false, kGemmResAdd>(p, 1, st);
     else return hipErrorInvalidValue;
     return hipGetLastError();
   }
-  if (p.M > kGemmTileMinM) {
-    if (norm && epi == kGemmStore) launch_tile<true, kGemmStore>(p, 1, st);
-    else if (norm && epi == kGemmSiluPair) launch_tile<true, kGemmSiluPair>(p, 1, st);
-    else if (!norm && epi == kGemmStore) launch_tile<false, kGemmStore>(p, 1, st);
-    else if (!norm && epi == kGemmResAdd) launch_tile<false, kGemmResAdd>(p, 1, st);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-  }
-  const dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64));
-  if (p.K % 64 == 0) {
-    if (norm && epi == kGemmStore) hipLaunchKernelGGL((k_gemm_lds<true, kGemmStore>), grid, dim3(256), 0, st, p);
-    else if (norm && epi == kGemmSiluPair) hipLaunchKernelGGL((k_gemm_lds<true, kGemmSiluPair>), grid, dim3(256), 0, st, p);
-    else if (!norm && epi == kGemmStore) hipLaunchKernelGGL((k_gemm_lds<false, kGemmStore>), grid, dim3(256), 0, st, p);
-    else if (!norm && epi == kGemmResAdd) hipLaunchKernelGGL((k_gemm_lds<false, kGemmResAdd>), grid, dim3(256), 0, st, p);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-  }
-  // four 32-wide k steps per iteration when K allows, else one
-#define QE_GEMM(NRM, E)                                                                         \
-  do {                                                                                          \
-    if (p.K % 128 == 0) hipLaunchKernelGGL((k_gemm<NRM, E, 4>), grid, dim3(256), 0, st, p);     \
-    else hipLaunchKernelGGL((k_gemm<NRM, E, 1>), grid, dim3(256), 0, st, p);                    \
-  } while (0)
-  if (norm && epi == kGemmStore) QE_GEMM(true, kGemmStore);
-  else if (norm && epi == kGemmSiluPair) QE_GEMM(true, kGemmSiluPair);
-  else if (!norm && epi == kGemmStore) QE_GEMM(false, kGemmStore);
-  else if (!norm && epi == kGemmResAdd) QE_GEMM(false, kGemmResAdd);
+  if (norm && epi == kGemmStore) launch_tile<true, kGemmStore>(p, 1, st);
+  else if (norm && epi == kGemmSiluPair) launch_tile<true, kGemmSiluPair>(p, 1, st);
+  else if (!norm && epi == kGemmResAdd) launch_tile<false, kGemmResAdd>(p, 1, st);
   else return hipErrorInvalidValue;
-#undef QE_GEMM
   return hipGetLastError();
 }
 
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K) {
   // tiles of the kernel that runs M rows, and the depth one split must stay a multiple of
-  uint32_t tiles, unit;
-  if (M <= kGemmSkinnyMaxM) {
-    tiles = ceil_div(N, 16);
-    unit = 32;
-  } else if (M <= kGemmTileMinM) {
-    tiles = ceil_div(N, 64) * ceil_div(M, 64);
-    unit = 64;
-  } else if (rows_kernel(M, K)) {
-    tiles = ceil_div(N, 128) * ceil_div(M, 64);
-    unit = 64;
-  } else {
-    tiles = ceil_div(N, tile_bn(M, N)) * ceil_div(M, 128);
-    unit = 32;
-  }
+  const bool rows = rows_kernel(M, K);
+  const uint32_t tiles = rows ? ceil_div(N, 128) * ceil_div(M, 64) : ceil_div(N, tile_bn(M, N)) * ceil_div(M, 128);
+  const uint32_t unit = rows ? 64 : 32;
   uint32_t z = 1;
   while (z < 8 && tiles * z < 256 && K % (2 * unit * z) == 0) z *= 2;
   return z;
 }
 
 hipError_t launch_gemm_split(const GemmParams& p, uint32_t splits, hipStream_t st) {
-  if (p.M == 0 || p.N == 0 || p.N % 2 || p.lda % 4 || !p.A || !p.W || !p.C || splits == 0)
+  if (p.M <= kGemmSliceMaxM || p.N == 0 || p.N % 2 || p.lda % 4 || !p.A || !p.W || !p.C || splits == 0)
     return hipErrorInvalidValue;
-  if (p.M <= kGemmSkinnyMaxM) {
-    if (p.K % (32 * splits)) return hipErrorInvalidValue;
-    launch_skinny<false, kGemmPartial>(p, splits, st);
-    return hipGetLastError();
-  }
   if (rows_kernel(p.M, p.K) && p.K % (64 * splits) == 0) {
     launch_rows<false, kGemmPartial>(p, splits, st);
     return hipGetLastError();
   }
-  if (p.M > kGemmTileMinM) {
-    if (p.K % (32 * splits)) return hipErrorInvalidValue;
-    launch_tile<false, kGemmPartial>(p, splits, st);
-    return hipGetLastError();
-  }
-  if (p.K % (64 * splits)) return hipErrorInvalidValue;
-  const dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), splits);
-  hipLaunchKernelGGL((k_gemm_lds<false, kGemmPartial>), grid, dim3(256), 0, st, p);
+  if (p.K % (32 * splits)) return hipErrorInvalidValue;
+  launch_tile<false, kGemmPartial>(p, splits, st);
   return hipGetLastError();
 }
 

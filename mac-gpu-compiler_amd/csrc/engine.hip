@@ -986,14 +986,14 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   const size_t layer_kv = size_t(c.num_key_value_heads) * kv->max_seq * D * el;
   hipStream_t s = xb ? xb->stream : m->stream;
   const float eps = c.rms_norm_eps;
-  // Up to kGemmSkinnyMaxM rows the skinny GEMM computes each norm's row scales itself and adds
+  // Up to kGemmSliceMaxM rows the k-sliced GEMM computes each norm's row scales itself and adds
   // residuals in its epilogue. Past that, bs holds the row scales of the current norm input:
   // from a rownorm launch for layer 0, then from the reduction that finishes each split o_proj /
   // down (residual add + the next norm's scales in one pass).
   // Up to kMvRowsMaxM rows the projections are matvecs over the M token rows: each weight is
   // loaded once per pass, the norm is computed per row in the kernel and the residual is added in
   // its epilogue (the lm_head of a verify stays on the skinny GEMM).
-  const bool skinny = M <= qe::kGemmSkinnyMaxM;
+  const bool skinny = M <= qe::kGemmSliceMaxM;
   const bool mv = m->mv_rows && M <= qe::kMvRowsMaxM;
   auto gemm = [&](const float* A, uint32_t lda, const uint16_t* gain, const uint16_t* W, uint32_t N, uint32_t K,
                   float* C, uint32_t ldc, int epi) -> int {
@@ -1010,8 +1010,8 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   };
   // x += A W^T, then bs = the row scales of the updated x
   auto gemm_resadd = [&](const float* A, uint32_t lda, const uint16_t* W, uint32_t K) -> int {
-    if (mv || (skinny && qe::gemm_splits(M, H, K) == 1)) return gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd);
-    if (!skinny && K % 64) {  // no split: residual epilogue, then the row scales
+    if (mv || skinny) return gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd);
+    if (K % 64) {  // no split: residual epilogue, then the row scales
       if (int rc2 = gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd)) return rc2;
       HIP_TRY(qe::launch_rownorm(bx, M, H, eps, bs, s));
       return QE_OK;
@@ -1071,8 +1071,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
         // as in the decode step: the attention is latency-bound, so extra workgroups load this
         // layer's gate|up (the skinny GEMM's rows at 4 tokens, else the multi-row matvec's) and
         // down weights into the L2 of the XCDs that will read them
-        r.pf[0] = M >= 4 ? qe::skinny_prefetch_target(w.w_gu, 2 * I, H)
-                         : qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
+        if (M < 4) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
         r.pf[1] = qe::l2_prefetch_target(w.w_down, H, I, qe::kCopy, qe::kResAdd);
         r.pf_slots = qe::l2_prefetch_slots(r.pf, qe::kMaxPrefetch);
       }
@@ -1588,11 +1587,11 @@ int qe_prefill_batch(qe_model* model, const uint32_t* ids, uint64_t n, uint64_t 
     if (ids[i] >= model->cfg.vocab_size) return fail(QE_ERR_ARG, "token %u at %llu >= vocab", ids[i], (unsigned long long)i);
   int rc = ensure_batch(model, chunk, 0);
   if (rc) return rc;
-  // chunks of more than kGemmSkinnyMaxM tokens go round-robin over up to prefill_streams streams
+  // chunks of more than kGemmSliceMaxM tokens go round-robin over up to prefill_streams streams
   // and buffer sets: chunk i's layer-l attention waits for chunk i-1's layer-l K/V rows, and
   // otherwise the chunks' launches overlap (each chunk runs the same kernels as on one stream)
   const uint64_t n_chunks = (n + chunk - 1) / chunk;
-  const int S = chunk > qe::kGemmSkinnyMaxM ? int(std::min<uint64_t>(model->prefill_streams, n_chunks)) : 1;
+  const int S = chunk > qe::kGemmSliceMaxM ? int(std::min<uint64_t>(model->prefill_streams, n_chunks)) : 1;
   if (S > 1 && (rc = ensure_streams(model, chunk, S))) return rc;
   if ((rc = upload_ids(model, ids, n))) return rc;
   auto stream_of = [&](int set) { return set ? model->extra[set - 1].stream : model->stream; };

@@ -1,0 +1,51 @@
+"""The GEMMs that load their operands straight into LDS (qe_op_gemm_bf16) at the edges of their
+tiles: every k-sliced tile (16 x 16 .. 64 x 128) and every wide one (64 x 128, 64 x 192 with three
+and two slots, 128 x 256), ragged rows and columns, k of one 32-deep step, an odd number of steps,
+fewer 64-deep blocks than waves, and an output whose rows are not 16-byte aligned."""
+import numpy as np
+import pytest
+
+import qe
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # k-sliced: 16 x 16, 16 x 32, 32 x 32, 32 x 48, 32 x 64, 48 x 64, 64 x 64, 64 x 128
+    (1, 2, 32), (1, 6, 96), (16, 512, 64), (17, 514, 1056), (9, 6144, 1024), (33, 1026, 2048), (130, 1024, 3072),
+    (64, 6144, 1024), (333, 1022, 544), (511, 1024, 2048), (130, 4094, 1024), (257, 2048, 480), (200, 4096, 96),
+    # wide
+    (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 128), (1025, 6146, 320), (2047, 4098, 64),
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemm_tiles_match_float64(gpu, m, n, k, shift):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n + k)
+    a = torch.randn(m, k, generator=g, device="cuda")
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.05).bfloat16()
+    buf = torch.full((m * n + 8,), float("nan"), device="cuda")
+    c = buf[shift:shift + m * n].view(m, n)  # shift 1: 4-byte aligned only
+    qe.op_gemm_bf16(a, w, c)
+    torch.cuda.synchronize()
+    ref = a.double() @ w.double().T
+    # a is split into two bf16 halves (|error| <= 2^-17 |a|); f32 accumulation over k terms
+    bound = (2.0 ** -16 + k * 2.0 ** -24) * (a.abs().double() @ w.abs().double().T) + 1e-30
+    assert bool(((c.double() - ref).abs() <= bound).all())
+    assert bool(torch.isnan(buf[:shift]).all()) and bool(torch.isnan(buf[shift + m * n:]).all())  # nothing past it
+
+
+@pytest.mark.parametrize("m", [33, 48, 64])
+def test_verify_of_many_rows_matches_decode(gpu, tiny_ckpt, m):
+    """k tokens in one pass (norm, silu and residual epilogues of the k-sliced GEMM past 32 rows)
+    against the same tokens one by one"""
+    model = qe.Model.load_model(tiny_ckpt)
+    V = model.config().vocab_size
+    ids = qe.random_prompt(83, 20 + m, V)
+    c1, c2 = qe.KVCache(model, 20 + m), qe.KVCache(model, 20 + m)
+    model.prefill(ids[:20], 0, c1, want_logits=False)
+    model.prefill(ids[:20], 0, c2, want_logits=False)
+    rows = model.verify(ids[20:], 20, c1)
+    for i in range(m):
+        assert np.max(np.abs(rows[i] - model.forward(int(ids[20 + i]), 20 + i, c2))) < 1e-3, f"row {i}"
