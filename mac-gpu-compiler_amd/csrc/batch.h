@@ -12,38 +12,39 @@ namespace qe {
 // kGemmPartial: split over K; split z writes its partial sums to C + z M ldc (launch_gemm_split)
 // kGemmQkRope (launch_gemm_qk_rope): the q|k|v projection of a chunk with the per-head q/k
 // RMSNorm, RoPE and the K/V append of k_qk_rope in its epilogue
-enum GemmEpilogue { kGemmStore = 0, kGemmResAdd = 1, kGemmSiluPair = 2, kGemmPartial = 3, kGemmQkRope = 4 };
+// kGemmSiluSplit (launch_gemm_split_rows): kGemmSiluPair written as split rows
+enum GemmEpilogue {
+  kGemmStore = 0, kGemmResAdd = 1, kGemmSiluPair = 2, kGemmPartial = 3, kGemmQkRope = 4, kGemmSiluSplit = 5
+};
 
 // most key runs the causal attention of a chunk is split into (partials merged after)
 constexpr int kBatchMaxRuns = 32;
 
-// C[m][n] (=, +=) sum_k A'[m][k] W[n][k] for m < M, n < N; A' = A, or A x rowscale[m] x gain[k]
-// (an RMSNorm) when the launch asks for the norm. kGemmSiluPair: W rows 2i / 2i+1 are gate_i /
-// up_i and C[m][i] = silu(gate) * up. N even, K % 32 == 0, lda % 4 == 0.
-// Up to kGemmSliceMaxM rows the k-sliced kernel computes the norm's row scales itself (rowscale
-// unused, eps used; K <= kGemmNormMaxK); more rows need rowscale filled by launch_rownorm.
+// C[m][n] (=, +=) sum_k A'[m][k] W[n][k] for m < M, n < N; A' = A, or an RMSNorm of A's rows (gain,
+// eps; K <= kGemmNormMaxK) when the launch asks for the norm. kGemmSiluPair: W rows 2i / 2i+1 are
+// gate_i / up_i and C[m][i] = silu(gate) * up. N even, K % 32 == 0, lda % 4 == 0.
+// The launches of a chunk (launch_gemm_split, launch_gemm_silu_split, launch_gemm_qk_rope) take A as split rows:
+// every f32 value as hi + lo bf16, 8 hi then 8 lo (16 bytes each) per 8 values. K % 64 == 0.
 struct GemmParams {
   const float* A;
   uint32_t lda;
-  const float* rowscale;  // [M]
-  const uint16_t* gain;   // bf16 [K]
-  const uint16_t* W;      // bf16 [N][K]
+  const uint16_t* gain;  // bf16 [K]
+  const uint16_t* W;     // bf16 [N][K]
   uint32_t M, N, K;
   float* C;
   uint32_t ldc;
   float eps;
+  uint32_t kz;  // the depth of one K split (set by the launches)
 };
 
-// Up to kGemmSliceMaxM rows every GEMM runs on k_gemm_kslice. Above, the norm and residual GEMMs of a
-// chunk take the 64-row eight-wave kernel (k_gemm_rows8) up to kGemmRowsMaxM rows (K a multiple of
-// 64), then 128-row tiles (k_gemm_tile): the faster at each size measured (128 .. 2048 rows).
+// Verify passes and chunks of up to kGemmSliceMaxM rows run the projections on k_gemm_kslice over
+// f32 rows, norms and residuals within; longer chunks on k_gemm_wide over split rows.
 constexpr uint32_t kGemmSliceMaxM = 64;
-constexpr uint32_t kGemmRowsMaxM = 1024;
 constexpr int kGemmNormMaxK = 4096;
 
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
 // token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
-// own products and lane reductions to every wave of that matvec, so past 4 rows the skinny GEMM
+// own products and lane reductions to every wave of that matvec, so past 4 rows the k-sliced GEMM
 // on the matrix cores is faster (measured at 5, 8 and 9 rows).
 constexpr uint32_t kMvRowsMaxM = 4;
 struct MvRowsParams {
@@ -73,7 +74,7 @@ struct TilePrefetch {
 struct BatchAttnParams {
   const float* qkv;        // [M][n_heads + 2 n_kv][128] raw projections
   float* q;                // [M][n_heads][128] normalized + rotated q
-  float* att;              // [M][n_heads][128] attention output
+  float* att;              // [M][n_heads][128] attention output, as split rows with att_split
   float* part;             // [M][n_heads][runs][kPartStride] partials (several key runs)
   const uint16_t* q_norm;  // bf16 [128]
   const uint16_t* k_norm;
@@ -85,27 +86,29 @@ struct BatchAttnParams {
   float eps, scale;
   int kv_bf16;
   uint32_t runs;           // key runs (set by launch_attn_causal)
+  int att_split;
   TilePrefetch pf;         // launch_attn_causal: weights its launch also loads into L2
 };
 
-hipError_t launch_rownorm(const float* x, uint32_t M, uint32_t K, float eps, float* s, hipStream_t st);
 hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st);
-// K splits for a split GEMM: enough workgroups to fill the chip, each split a multiple of the
-// kernel's k step deep (1 when K does not split)
+// ---- a chunk's GEMMs: A as split rows (see GemmParams) ----
+// K splits for launch_gemm_split: enough workgroups to fill the chip (1 when K does not split)
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K);
-// partial sums of `splits` K ranges (no norm): C[z][m][n], z < splits, ldc = N
+// partial sums of `splits` K ranges: C[z][m][n], z < splits, ldc = N
 hipError_t launch_gemm_split(const GemmParams& p, uint32_t splits, hipStream_t st);
-// The prefetch target of the weights of launch_gemm / launch_gemm_qk_rope (epi) or
-// launch_gemm_split (kGemmPartial) at M rows on the 64-row kernel: column tile j, every row tile
-// and K split of which runs on XCD j % 8, reads W rows [bn j, bn (j + 1)). w = nullptr where
-// another kernel serves the shape or a column tile's workgroups do not stay on one XCD.
-L2Prefetch gemm_prefetch_target(const uint16_t* W, uint32_t M, uint32_t N, uint32_t K, int epi);
+// C[m] = split row of silu(gate) * up over the interleaved gate/up rows of W (ldc >= N / 2)
+hipError_t launch_gemm_silu_split(const GemmParams& p, hipStream_t st);
+// The prefetch target of the weights of launch_gemm_split at M rows: column tile j, every row tile
+// and K split of which runs on XCD j % 8, reads W rows [bn j, bn (j + 1)). w = nullptr where a
+// column tile's workgroups do not stay on one XCD.
+L2Prefetch gemm_prefetch_target(const uint16_t* W, uint32_t M, uint32_t N, uint32_t K);
 // the slots that cover these targets (at most 64)
 uint32_t tile_prefetch_slots(const L2Prefetch* pf, int n);
-// x[m][n] += sum_z part[z][m][n] (z in order), then s[m] = 1 / sqrt(mean_n x[m][n]^2 + eps):
-// the residual add of a split GEMM fused with the next RMSNorm's row scale. N % 4 == 0.
-hipError_t launch_resadd_partials(float* x, const float* part, uint32_t splits, uint32_t M, uint32_t N, float eps,
-                                  float* s, hipStream_t st);
+// x[m][n] += sum_z part[z][m][n] (z in order; splits = 0: x as it is), then, with a gain, out[m] =
+// RMSNorm(x[m]) x gain as a split row: the residual add of a split GEMM fused with the next norm.
+// N % 8 == 0.
+hipError_t launch_resadd_norm_split(float* x, const float* part, uint32_t splits, uint32_t M, uint32_t N, float eps,
+                                    const uint16_t* gain, float* out, hipStream_t st);
 // out[m][r] (=, +=) sum_c W[r][c] x'[m][c] for m < M (kGemmStore / kGemmResAdd), or
 // out[m][i] = silu(gate_i) * up_i over the interleaved gate/up rows (kGemmSiluPair, ldo >= rows/2);
 // x' = x, or RMSNorm(x_m) * gain with `norm`. f32 FMA on bf16 weights, as the decode matvec.
@@ -124,11 +127,9 @@ hipError_t launch_mv_rows_merge(const MvRowsParams& p, hipStream_t st);
 // token rows stay within 16
 bool mv_rows_merge_fits(uint32_t M, uint32_t splits);
 hipError_t launch_qk_rope(const BatchAttnParams& p, hipStream_t st);
-// The q|k|v GEMM of a chunk (A = x with the input RMSNorm, W = [q | k | v] rows, N = (n_heads +
+// The q|k|v GEMM of a chunk (A = the normalized x as split rows, W = [q | k | v] rows, N = (n_heads +
 // 2 n_kv) 128) with k_qk_rope's work in its epilogue: q rows normalized and rotated to a.q, k and
-// v rows (k normalized and rotated) appended to the cache at positions a.start + m. Returns
-// hipErrorNotSupported where the 64-row kernel does not serve the shape (the caller then runs
-// launch_gemm and launch_qk_rope).
+// v rows (k normalized and rotated) appended to the cache at positions a.start + m.
 hipError_t launch_gemm_qk_rope(const GemmParams& g, const BatchAttnParams& a, hipStream_t st);
 // causal attention of a chunk over `runs` (1..kBatchMaxRuns) key runs, merged into att; p.pf:
 // weights the launch also loads into L2 (whole planes of workgroups after the runs')

@@ -3,12 +3,11 @@
 // The reference runs its prompt one token at a time (metal_infrence_engine/src/bin/bench.rs:174-176
 // calls forward per position); these kernels run a chunk of M tokens through a layer at once, so
 // every weight is read once per chunk and the projections become GEMMs on the matrix cores:
-//   rownorm        s[m] = 1/sqrt(mean(x_m^2) + eps)                  (cpu_inference.rs:189-194)
-//   GEMMs          C[m][n] = sum_k A'[m][k] W[n][k], A' = f32 A (x s[m] x gain[k] with a norm),
-//                  split into hi + lo bf16 so the products keep ~16 mantissa bits; epilogues
-//                  store / residual add / silu(gate)*up / q-k norm + RoPE + K/V append
-//                  (cpu_inference.rs:225-257): k_gemm_skinny (<= 32 rows), k_gemm_lds / k_gemm (<= 64),
-//                  k_gemm_rows8 (<= 1024), k_gemm_tile (more); k_mv_rows (<= 4 rows, f32 FMA)
+//   GEMMs          C[m][n] = sum_k A'[m][k] W[n][k], A' = A or an RMSNorm of its rows, split into
+//                  hi + lo bf16 so the products keep ~16 mantissa bits (gemm_dma.h); epilogues store /
+//                  residual add / silu(gate)*up / q-k norm + RoPE + K/V append (cpu_inference.rs:225-257):
+//                  k_gemm_kslice (<= 64 rows), k_gemm_wide (more); k_mv_rows (<= 4 rows, f32 FMA)
+//   k_resadd_norm_split  residual add of a split GEMM, then the next norm, split for the next GEMM
 //   k_qk_rope      per token and head: q/k RMSNorm + RoPE, K/V append   (cpu_inference.rs:134-141)
 //   k_attn_causal_bf  token m attends positions 0..start+m, split bf16 MFMA (cpu_inference.rs:144-162)
 //   k_row_argmax_*    greedy token per logit row (main.rs:37-42)
@@ -25,393 +24,49 @@
 namespace qe {
 namespace {
 
-// ---------------------------------------------------------------------------------------------
-// s[m] = 1 / sqrt(mean_k x[m][k]^2 + eps): one wave per row
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_rownorm(const float* __restrict__ x, uint32_t M, uint32_t K, float eps,
-                                                 float* __restrict__ s) {
-  const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= M) return;
-  const float4* xr = reinterpret_cast<const float4*>(x + size_t(row) * K);
-  float acc = 0.f;
-  for (uint32_t i = lane; i < K / 4; i += 64) {
-    const float4 v = xr[i];
-    acc += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-  }
-  acc = wave_sum(acc);
-  if (lane == 0) s[row] = 1.0f / sqrtf(acc / float(K) + eps);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Tiled GEMM for M > 64: workgroup tile 128 (m) x BN (n), BN = 128 or 64, k stages of 32. Four
-// waves as 2 x 2: wave (wm, wn) owns rows 64 wm .. 64 wm + 63 and columns (BN / 2) wn .. + BN / 2
-// - 1, i.e. 4 x BN / 32 MFMA tiles of 16 x 16, so each fragment read from LDS feeds BN / 32 (A)
-// or 8 (W) MFMAs. Both operands are staged in LDS: the thread that loads an f32 A element
-// applies the norm scale and splits it into hi + lo bf16 once for the whole workgroup; W rows go
-// in as they are. Two LDS buffers and D register stages (stage t in register slot t % D): while
-// stage s is computed from one buffer, stage s + 1 goes from its slot to the other buffer and the
-// slot is refilled with stage s + 1 + D, so each load has D steps of MFMA work to arrive in (one
-// step is short next to the L2 / MALL latency). The stage count K / 32 (per split) is a multiple
-// of D (the launcher checks). gridDim.z > 1 splits K as in k_gemm_lds.
-// ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI, int BN, int D>
-__global__ __launch_bounds__(256) void k_gemm_tile(GemmParams p) {
-  constexpr int BM = 128, BK = 32, NT = BN / 32, KP = BK + 8;
-  constexpr int WCH = BN * BK / 8 / 256;  // 16-byte W chunks per thread per stage
-  static_assert(WCH >= 1 && NT >= 2, "tile");
-  __shared__ __align__(16) uint16_t as[2][2][BM][KP];  // [buffer][hi, lo][m][k]
-  __shared__ __align__(16) uint16_t bs[2][BN][KP];     // [buffer][n][k]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-  const uint32_t m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const uint32_t kz = p.K / gridDim.z, kbeg = blockIdx.z * kz, nst = kz / BK;
-  // A staging: float4 f = tid + 256 i (i < 4) is row tid / 8 + 32 i, k (tid % 8) * 4
-  const int ar = tid >> 3, ak = (tid & 7) * 4;
-  const float* Asrc[4];
-  float rs[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t row = min(m0 + uint32_t(ar + 32 * i), p.M - 1);
-    Asrc[i] = p.A + size_t(row) * p.lda + kbeg + ak;
-    rs[i] = NORM ? p.rowscale[row] : 1.0f;
-  }
-  const uint16_t* gsrc = NORM ? p.gain + kbeg + ak : nullptr;
-  // W staging: chunk c = tid + 256 i is row c / 4, k (c % 4) * 8
-  const uint16_t* Wsrc[WCH];
-#pragma unroll
-  for (int i = 0; i < WCH; i++) {
-    const int c = tid + 256 * i;
-    Wsrc[i] = p.W + size_t(min(n0 + uint32_t(c >> 2), p.N - 1)) * p.K + kbeg + 8 * (c & 3);
-  }
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  struct Stage {
-    f32x4 a[4];
-    u32x4 w[WCH];
-    u32x2 g;
-  };
-  auto load = [&](Stage& r, uint32_t stg) __attribute__((always_inline)) {
-    const uint32_t k = stg * BK;
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.a[i] = *reinterpret_cast<const f32x4*>(Asrc[i] + k);
-#pragma unroll
-    for (int i = 0; i < WCH; i++) r.w[i] = *reinterpret_cast<const u32x4*>(Wsrc[i] + k);
-    if constexpr (NORM) r.g = *reinterpret_cast<const u32x2*>(gsrc + k);
-  };
-  auto pk = [](float a, float b) __attribute__((always_inline)) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
-  };
-  auto store = [&](const Stage& r, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      float v[4] = {r.a[i][0], r.a[i][1], r.a[i][2], r.a[i][3]};
-      if constexpr (NORM) {
-        v[0] = (v[0] * rs[i]) * __uint_as_float(r.g[0] << 16);
-        v[1] = (v[1] * rs[i]) * __uint_as_float(r.g[0] & 0xFFFF0000u);
-        v[2] = (v[2] * rs[i]) * __uint_as_float(r.g[1] << 16);
-        v[3] = (v[3] * rs[i]) * __uint_as_float(r.g[1] & 0xFFFF0000u);
-      }
-      const uint32_t h0 = pk(v[0], v[1]), h1 = pk(v[2], v[3]);
-      const uint32_t l0 = pk(v[0] - __uint_as_float(h0 << 16), v[1] - __uint_as_float(h0 & 0xFFFF0000u));
-      const uint32_t l1 = pk(v[2] - __uint_as_float(h1 << 16), v[3] - __uint_as_float(h1 & 0xFFFF0000u));
-      *reinterpret_cast<u32x2*>(&as[buf][0][ar + 32 * i][ak]) = u32x2{h0, h1};
-      *reinterpret_cast<u32x2*>(&as[buf][1][ar + 32 * i][ak]) = u32x2{l0, l1};
-    }
-#pragma unroll
-    for (int i = 0; i < WCH; i++) {
-      const int c = tid + 256 * i;
-      *reinterpret_cast<u32x4*>(&bs[buf][c >> 2][8 * (c & 3)]) = r.w[i];
-    }
-  };
-  f32x4 acc[4][NT];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // All fragments of the stage are read before the first MFMA, so the LDS latency is paid once
-  // per stage; then the hi products, then the lo products (each accumulator still adds hi . w
-  // before lo . w).
-  auto compute = [&](int buf) __attribute__((always_inline)) {
-    bf16x8 b[NT], hi[4], lo[4];
-#pragma unroll
-    for (int j = 0; j < NT; j++)
-      b[j] = *reinterpret_cast<const bf16x8*>(&bs[buf][wn * (BN / 2) + 16 * j + li][8 * kg]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int row = wm * 64 + 16 * i + li;
-      hi[i] = *reinterpret_cast<const bf16x8*>(&as[buf][0][row][8 * kg]);
-      lo[i] = *reinterpret_cast<const bf16x8*>(&as[buf][1][row][8 * kg]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], b[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], b[j], acc[i][j], 0, 0, 0);
-  };
-  Stage r[D];
-#pragma unroll
-  for (int i = 0; i < D; i++) load(r[i], min(uint32_t(i), nst - 1));
-  store(r[0], 0);
-  load(r[0], min(uint32_t(D), nst - 1));
-  __syncthreads();
-  // Every step is unconditional: the loads past the last stage re-read the last stage (in
-  // bounds), and the last step's store goes to the buffer no later step reads.
-  for (uint32_t s0 = 0; s0 < nst; s0 += D) {
-#pragma unroll
-    for (int i = 0; i < D; i++) {
-      const uint32_t s = s0 + uint32_t(i);
-      compute(int(s & 1));
-      __builtin_amdgcn_sched_barrier(0);
-      store(r[(i + 1) % D], int((s + 1) & 1));
-      load(r[(i + 1) % D], min(s + 1 + D, nst - 1));
-      __syncthreads();
-    }
-  }
-
-  // epilogue: lane holds C[m0 + 64 wm + 16 i + 4 kg + r][n0 + (BN / 2) wn + 16 j + li]
-  float* C = p.C + (EPI == kGemmPartial ? size_t(blockIdx.z) * p.M * p.ldc : 0);
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-      const uint32_t n = n0 + uint32_t(wn * (BN / 2) + 16 * j + li);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const uint32_t m = m0 + uint32_t(wm * 64 + 16 * i + 4 * kg + r);
-        const float c = acc[i][j][r];
-        if constexpr (EPI == kGemmSiluPair) {
-          const float up = __shfl_xor(c, 1);  // columns 2i (gate) and 2i+1 (up) in neighbouring lanes
-          if (m < p.M && n < p.N && (li & 1) == 0) C[size_t(m) * p.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-        } else if constexpr (EPI == kGemmResAdd) {
-          if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] += c;
-        } else {
-          if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] = c;
-        }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Tiled GEMM for chunks of up to kGemmRowsMaxM rows, A straight to registers: workgroup tile 64
-// (m) x BN (n), k steps of 64, eight waves. Wave w owns the 16-row block w % 4 and the k half w / 4
-// of every step (k 64 s + 32 (w / 4) .. + 31). An A row belongs to one wave pair only, so each lane
-// loads its own f32 A fragment (row li of its block, k 8 kg .. 8 kg + 7), applies the norm scale
-// and splits it into hi + lo bf16 in registers; only the W tile, which all eight waves read, goes
-// through LDS (two buffers, rows staged 128 bytes = 64 k at a time). A 64 x 128 tile keeps the
-// bytes each CU pulls per MFMA lower than the 128-row tile does at these sizes, where the loads
-// from L2 and not the matrix cores set the pace, and still gives one tile per CU at 512 rows.
-// D steps in flight: A of step s + D is loaded as soon as step s is computed, W of step s + 1 + D
-// as soon as step s + 1 is in LDS. At the end the k-half-1 waves hand their sums to the k-half-0
-// waves through LDS: C = (sum over the even 32-k blocks) + (sum over the odd ones). The step
-// count K / 64 (per split) is a multiple of D. gridDim.z > 1 splits K as in k_gemm_lds.
-// ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI, int BN, int D>
-__global__ __launch_bounds__(512) void k_gemm_rows8(GemmParams p, BatchAttnParams qa) {
-  constexpr int BK = 64, KP = BK + 8, NT = BN / 16;
-  constexpr int WCH = BN * BK / 8 / 512;  // 16-byte W chunks per thread per step
-  static_assert(WCH >= 1, "tile");
-  static_assert(2 * BN * KP * 2 >= 4 * 64 * NT * 16, "the reduction reuses the W buffers");
-  __shared__ __align__(16) uint16_t bs[2][BN][KP];  // [buffer][n][k]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
-  const int wr = wave & 3, kh = wave >> 2;
-  const uint32_t m0 = blockIdx.y * 64 + uint32_t(wr) * 16, n0 = blockIdx.x * BN;
-  const uint32_t kz = p.K / gridDim.z, kbeg = blockIdx.z * kz, nst = kz / BK;
-  const uint32_t row = min(m0 + uint32_t(li), p.M - 1);
-  const float* Ar = p.A + size_t(row) * p.lda + kbeg + 32 * kh + 8 * kg;
-  const float rs = NORM ? p.rowscale[row] : 1.0f;
-  const uint16_t* gsrc = NORM ? p.gain + kbeg + 32 * kh + 8 * kg : nullptr;
-  // W staging: chunk c = tid + 512 i is row c / 8, k (c % 8) * 8
-  const uint16_t* Wsrc[WCH];
-#pragma unroll
-  for (int i = 0; i < WCH; i++) {
-    const int c = tid + 512 * i;
-    Wsrc[i] = p.W + size_t(min(n0 + uint32_t(c >> 3), p.N - 1)) * p.K + kbeg + 8 * (c & 7);
-  }
-  struct AStage {
-    f32x4 a[2];
-    u32x4 g;
-  };
-  struct WStage {
-    u32x4 w[WCH];
-  };
-  auto load_a = [&](AStage& r, uint32_t stg) __attribute__((always_inline)) {
-    const uint32_t k = stg * BK;
-    r.a[0] = *reinterpret_cast<const f32x4*>(Ar + k);
-    r.a[1] = *reinterpret_cast<const f32x4*>(Ar + k + 4);
-    if constexpr (NORM) r.g = *reinterpret_cast<const u32x4*>(gsrc + k);
-  };
-  auto load_w = [&](WStage& r, uint32_t stg) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < WCH; i++) r.w[i] = *reinterpret_cast<const u32x4*>(Wsrc[i] + stg * BK);
-  };
-  auto store_w = [&](const WStage& r, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < WCH; i++) {
-      const int c = tid + 512 * i;
-      *reinterpret_cast<u32x4*>(&bs[buf][c >> 3][8 * (c & 7)]) = r.w[i];
-    }
-  };
-  f32x4 acc[NT];
-#pragma unroll
-  for (int j = 0; j < NT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto compute = [&](const AStage& r, int buf) __attribute__((always_inline)) {
-    bf16x8 b[NT], hi, lo;
-#pragma unroll
-    for (int j = 0; j < NT; j++) b[j] = *reinterpret_cast<const bf16x8*>(&bs[buf][16 * j + li][32 * kh + 8 * kg]);
-    float v[8] = {r.a[0][0], r.a[0][1], r.a[0][2], r.a[0][3], r.a[1][0], r.a[1][1], r.a[1][2], r.a[1][3]};
-    if constexpr (NORM) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[2 * e] = (v[2 * e] * rs) * __uint_as_float(r.g[e] << 16);
-        v[2 * e + 1] = (v[2 * e + 1] * rs) * __uint_as_float(r.g[e] & 0xFFFF0000u);
-      }
-    }
-    split8(v, hi, lo);
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, b[j], acc[j], 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, b[j], acc[j], 0, 0, 0);
-  };
-  AStage ra[D];
-  WStage rw[D];
-#pragma unroll
-  for (int i = 0; i < D; i++) {
-    load_a(ra[i], min(uint32_t(i), nst - 1));
-    load_w(rw[i], min(uint32_t(i), nst - 1));
-  }
-  store_w(rw[0], 0);
-  load_w(rw[0], min(uint32_t(D), nst - 1));
-  __syncthreads();
-  // Every step is unconditional: loads past the last step re-read the last step (in bounds), and
-  // the last step's W store goes to the buffer no later step reads.
-  for (uint32_t s0 = 0; s0 < nst; s0 += D) {
-#pragma unroll
-    for (int i = 0; i < D; i++) {
-      const uint32_t s = s0 + uint32_t(i);
-      compute(ra[i], int(s & 1));
-      load_a(ra[i], min(s + D, nst - 1));
-      store_w(rw[(i + 1) % D], int((s + 1) & 1));
-      load_w(rw[(i + 1) % D], min(s + 1 + D, nst - 1));
-      __syncthreads();
-    }
-  }
-  // the k-half-1 waves' sums, lane-major per (row block, column block), through the W buffers
-  f32x4* red = reinterpret_cast<f32x4*>(&bs[0][0][0]);
-  if (kh == 1) {
-#pragma unroll
-    for (int j = 0; j < NT; j++) red[(wr * NT + j) * 64 + lane] = acc[j];
-  }
-  __syncthreads();
-  if (kh == 1) return;
-#pragma unroll
-  for (int j = 0; j < NT; j++) acc[j] += red[(wr * NT + j) * 64 + lane];
-
-  // epilogue: lane holds C[m0 + 4 kg + r][n0 + 16 j + li]
-  if constexpr (EPI == kGemmQkRope) {
-    // the tile's 128 columns are one head (BN == 128 == head_dim): head hh of [q | k | v]. A row's
-    // 128 values sit in the 16 lanes of its kg group (8 each), and the RoPE pair (d, d + 64) is
-    // (j, j + 4) of one lane (cpu_inference.rs:134-141, 189-215).
-    static_assert(BN == kHeadDim && NT == 8, "one head per tile");
-    const uint32_t hh = n0 / kHeadDim;
-    const bool isq = hh < qa.n_heads, isk = !isq && hh < qa.n_heads + qa.n_kv;
-    float gn[NT];
-    const uint16_t* gsrc = isq ? qa.q_norm : qa.k_norm;
-#pragma unroll
-    for (int j = 0; j < NT; j++) gn[j] = isq || isk ? bf16f(gsrc[16 * j + li]) : 1.0f;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const uint32_t m = m0 + uint32_t(4 * kg + r), pos = qa.start + min(m, p.M - 1);
-      float v[NT];
-#pragma unroll
-      for (int j = 0; j < NT; j++) v[j] = acc[j][r];
-      if (isq || isk) {  // uniform over the workgroup
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < NT; j++) ss += v[j] * v[j];
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
-        ss += __shfl_xor(ss, 8);
-        const float sc = 1.0f / sqrtf(ss / float(kHeadDim) + qa.eps);
-#pragma unroll
-        for (int j = 0; j < NT; j++) v[j] = v[j] * sc * gn[j];
-        const float2* rope = reinterpret_cast<const float2*>(qa.rope) + size_t(pos) * (kHeadDim / 2);
-#pragma unroll
-        for (int j = 0; j < NT / 2; j++) {
-          const float2 cs = rope[16 * j + li];
-          const float a = v[j], b = v[j + NT / 2];
-          v[j] = a * cs.x - b * cs.y;
-          v[j + NT / 2] = b * cs.x + a * cs.y;
-        }
-      }
-      if (m < p.M) {
-        if (isq) {
-          float* q = qa.q + (size_t(m) * qa.n_heads + hh) * kHeadDim;
-#pragma unroll
-          for (int j = 0; j < NT; j++) q[16 * j + li] = v[j];
-        } else {
-          const uint32_t kvh = isk ? hh - qa.n_heads : hh - qa.n_heads - qa.n_kv;
-          void* cache = isk ? qa.k_cache : qa.v_cache;
-          const size_t slot = (size_t(kvh) * qa.max_seq + pos) * kHeadDim;
-#pragma unroll
-          for (int j = 0; j < NT; j++) {
-            if (qa.kv_bf16) static_cast<uint16_t*>(cache)[slot + 16 * j + li] = f32_to_bf16(v[j]);
-            else static_cast<float*>(cache)[slot + 16 * j + li] = v[j];
-          }
-        }
-      }
-    }
-    return;
-  }
-  float* C = p.C + (EPI == kGemmPartial ? size_t(blockIdx.z) * p.M * p.ldc : 0);
-#pragma unroll
-  for (int j = 0; j < NT; j++) {
-    const uint32_t n = n0 + uint32_t(16 * j + li);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const uint32_t m = m0 + uint32_t(4 * kg + r);
-      const float c = acc[j][r];
-      if constexpr (EPI == kGemmSiluPair) {
-        const float up = __shfl_xor(c, 1);  // columns 2i (gate) and 2i+1 (up) in neighbouring lanes
-        if (m < p.M && n < p.N && (li & 1) == 0) C[size_t(m) * p.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-      } else if constexpr (EPI == kGemmResAdd) {
-        if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] += c;
-      } else {
-        if (m < p.M && n < p.N) C[size_t(m) * p.ldc + n] = c;
-      }
-    }
-  }
-}
-
-// x[m] += sum_z part[z][m] (in z order), then s[m] = 1 / sqrt(mean x[m]^2 + eps); one workgroup
-// per row, float4 per thread per pass
-__global__ __launch_bounds__(256) void k_resadd_partials(float* __restrict__ x, const float* __restrict__ part,
-                                                         uint32_t splits, uint32_t M, uint32_t N, float eps,
-                                                         float* __restrict__ s) {
+// x[m] += sum_z part[z][m] (in z order; none: x as it is), then out[m] = x[m] / sqrt(mean x[m]^2 +
+// eps) x gain as a split row (cpu_inference.rs:189-194); one workgroup per row, float4 per thread
+// per pass. The products that read the norm read it split, so it is computed and split once here.
+__global__ __launch_bounds__(256) void k_resadd_norm_split(float* __restrict__ x, const float* __restrict__ part,
+                                                           uint32_t splits, uint32_t M, uint32_t N, float eps,
+                                                           const uint16_t* __restrict__ gain,
+                                                           float* __restrict__ out) {
+  constexpr int U = 4;  // N <= 4096: a row is at most 4 float4 per thread
   __shared__ float red[4];
-  const uint32_t m = blockIdx.x, tid = threadIdx.x;
+  const uint32_t m = blockIdx.x, tid = threadIdx.x, n4 = N / 4;
+  float4 v[U];
   float ss = 0.f;
-  for (uint32_t c = tid; c < N / 4; c += 256) {
-    float4 acc = reinterpret_cast<const float4*>(part + size_t(m) * N)[c];
-    for (uint32_t z = 1; z < splits; z++) {
-      const float4 v = reinterpret_cast<const float4*>(part + (size_t(z) * M + m) * N)[c];
-      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-    }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const uint32_t c = tid + 256 * u;
+    if (c >= n4) break;
     float4* xr = reinterpret_cast<float4*>(x + size_t(m) * N) + c;
-    float4 xv = *xr;
-    xv.x += acc.x; xv.y += acc.y; xv.z += acc.z; xv.w += acc.w;
-    *xr = xv;
-    ss += (xv.x * xv.x + xv.y * xv.y) + (xv.z * xv.z + xv.w * xv.w);
+    v[u] = *xr;
+    if (splits) {
+      float4 acc = reinterpret_cast<const float4*>(part + size_t(m) * N)[c];
+      for (uint32_t z = 1; z < splits; z++) {
+        const float4 w = reinterpret_cast<const float4*>(part + (size_t(z) * M + m) * N)[c];
+        acc.x += w.x; acc.y += w.y; acc.z += w.z; acc.w += w.w;
+      }
+      v[u].x += acc.x; v[u].y += acc.y; v[u].z += acc.z; v[u].w += acc.w;
+      *xr = v[u];
+    }
+    ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
   }
+  if (!gain) return;
   ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
-  if (tid == 0) s[m] = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / float(N) + eps);
+  const float sc = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / float(N) + eps);
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const uint32_t c = tid + 256 * u;
+    if (c >= n4) break;
+    const uint2 g = reinterpret_cast<const uint2*>(gain)[c];
+    store_split4(out + size_t(m) * N, 4 * c, v[u].x * sc * __uint_as_float(g.x << 16),
+                 v[u].y * sc * __uint_as_float(g.x & 0xFFFF0000u), v[u].z * sc * __uint_as_float(g.y << 16),
+                 v[u].w * sc * __uint_as_float(g.y & 0xFFFF0000u));
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -699,11 +354,13 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
     const size_t vec = size_t(tok[b]) * p.n_heads + head[b];
     if (runs == 1) {
       const float inv = 1.0f / l_run[b];
-      float* out = p.att + vec * D + 4 * kg;
+      float* out = p.att + vec * D;
 #pragma unroll
-      for (int i = 0; i < 8; i++)
-        *reinterpret_cast<float4*>(out + 16 * i) =
-            make_float4(o[b][i][0] * inv, o[b][i][1] * inv, o[b][i][2] * inv, o[b][i][3] * inv);
+      for (int i = 0; i < 8; i++) {
+        const f32x4 v = o[b][i] * inv;
+        if (p.att_split) store_split4(out, 16 * i + 4 * kg, v[0], v[1], v[2], v[3]);
+        else *reinterpret_cast<f32x4*>(out + 16 * i + 4 * kg) = v;
+      }
     } else {
       float* out = p.part + (vec * runs + run) * kPartStride;
       if (kg == 0) {
@@ -718,34 +375,40 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
 }
 
 // att[v] = sum_s e_s acc_s / sum_s e_s l_s over the runs of query vector v = (token, head),
-// e_s = 2^(m_s - max m) (m in base-2 units); runs without a visible key (m = -inf) weigh 0. Two query vectors per
-// workgroup of 256 threads (one per dim); all U >= runs run loads are issued at once.
+// e_s = 2^(m_s - max m) (m in base-2 units); runs without a visible key (m = -inf) weigh 0. Eight
+// query vectors per workgroup of 256 threads (four dims each); all U >= runs run loads are issued
+// at once.
 template <int U>
 __global__ __launch_bounds__(256) void k_attn_merge_rows(const float* __restrict__ part, uint32_t runs,
-                                                         uint32_t n_vec, float* __restrict__ att) {
-  const size_t v = min(blockIdx.x * 2 + (threadIdx.x >> 7), n_vec - 1);  // odd count: the last one twice
-  const uint32_t d = threadIdx.x & (kHeadDim - 1);
+                                                         uint32_t n_vec, float* __restrict__ att, int split) {
+  const size_t v = min(blockIdx.x * 8 + (threadIdx.x >> 5), n_vec - 1);  // past the end: the last one again
+  const uint32_t d = 4 * (threadIdx.x & 31);
   const float* base = part + v * runs * kPartStride;
-  float mv[U], lv[U], av[U];
+  float2 ml[U];
+  f32x4 av[U];
 #pragma unroll
   for (int u = 0; u < U; u++) {
     const float* q = base + size_t(min(uint32_t(u), runs - 1)) * kPartStride;
-    mv[u] = q[0];
-    lv[u] = q[1];
-    av[u] = q[4 + d];
+    ml[u] = *reinterpret_cast<const float2*>(q);
+    av[u] = *reinterpret_cast<const f32x4*>(q + 4 + d);
   }
   __builtin_amdgcn_sched_barrier(0);
   float M = -INFINITY;
 #pragma unroll
-  for (int u = 0; u < U; u++) M = uint32_t(u) < runs ? fmaxf(M, mv[u]) : M;
-  float L = 0.f, A = 0.f;
+  for (int u = 0; u < U; u++) M = uint32_t(u) < runs ? fmaxf(M, ml[u].x) : M;
+  float L = 0.f;
+  f32x4 A = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < U; u++) {  // m in base-2 units (k_attn_causal_bf)
-    const float e = (uint32_t(u) < runs && mv[u] != -INFINITY) ? exp2f(mv[u] - M) : 0.f;
-    L += e * lv[u];
-    A += e * av[u];
+    const float e = (uint32_t(u) < runs && ml[u].x != -INFINITY) ? exp2f(ml[u].x - M) : 0.f;
+    L += e * ml[u].y;
+#pragma unroll
+    for (int r = 0; r < 4; r++) A[r] += e * av[u][r];
   }
-  att[v * kHeadDim + d] = A / L;
+#pragma unroll
+  for (int r = 0; r < 4; r++) A[r] /= L;
+  if (split) store_split4(att + v * kHeadDim, d, A[0], A[1], A[2], A[3]);
+  else *reinterpret_cast<f32x4*>(att + v * kHeadDim + d) = A;
 }
 
 // tokens[r] = the greedy token of logits row r by the reference's scan (bench.rs:98-103,
@@ -827,63 +490,6 @@ __global__ __launch_bounds__(256) void k_embed_rows_v(const uint16_t* __restrict
     x[size_t(m) * H + i] = bf16f(table[size_t(ids.id[m]) * H + i]);
 }
 
-// column tile of k_gemm_tile: 128 when that alone gives a tile per CU, else 64
-uint32_t tile_bn(uint32_t M, uint32_t N) { return ceil_div(M, 128) * ceil_div(N, 128) >= 256 ? 128 : 64; }
-
-// register prefetch depth of k_gemm_tile: stages in flight per thread
-constexpr int kTileDepth = 2;
-
-// k_gemm_rows8 serves M rows of a K-deep product
-bool rows_kernel(uint32_t M, uint32_t K) { return M > kGemmSliceMaxM && M <= kGemmRowsMaxM && K % 64 == 0; }
-
-// k_gemm_rows8 over `splits` K splits (K % (64 splits) == 0, checked by the callers)
-// Column tile of k_gemm_rows8 for an unsplit launch. The kernel is bound by what a CU pulls from
-// L2 (A 16 KB and W BN x 128 B per 64-deep step), so the tile is the one with the fewest bytes
-// on the busiest CU: rounds of 256 workgroups x bytes per step. For gate|up at 512 rows
-// (N = 6144) 192 columns give 256 workgroups at 40 KB a step against 384 at 32 KB (half the CUs
-// running two).
-uint32_t rows_bn(uint32_t M, uint32_t N, uint32_t splits) {
-  if (splits != 1 || N % 192) return 128;
-  const uint64_t rounds128 = ceil_div(ceil_div(N, 128) * ceil_div(M, 64), 256u);
-  const uint64_t rounds192 = ceil_div(ceil_div(N, 192) * ceil_div(M, 64), 256u);
-  return rounds192 * (16 + 24) < rounds128 * (16 + 16) ? 192 : 128;
-}
-
-template <bool NRM, int E>
-void launch_rows(const GemmParams& p, uint32_t splits, hipStream_t st) {
-  if constexpr (E == kGemmStore || E == kGemmSiluPair || E == kGemmResAdd) {
-    if (rows_bn(p.M, p.N, splits) == 192) {
-      // two steps in flight where the step count allows (-1% on the 2048-token prefill; the
-      // 128-column tile gains nothing from it)
-      const dim3 g(ceil_div(p.N, 192), ceil_div(p.M, 64), splits);
-      if ((p.K / splits / 64) % 2 == 0)
-        hipLaunchKernelGGL((k_gemm_rows8<NRM, E, 192, 2>), g, dim3(512), 0, st, p, BatchAttnParams{});
-      else
-        hipLaunchKernelGGL((k_gemm_rows8<NRM, E, 192, 1>), g, dim3(512), 0, st, p, BatchAttnParams{});
-      return;
-    }
-  }
-  const dim3 g(ceil_div(p.N, 128), ceil_div(p.M, 64), splits);
-  hipLaunchKernelGGL((k_gemm_rows8<NRM, E, 128, 1>), g, dim3(512), 0, st, p, BatchAttnParams{});
-}
-
-// k_gemm_tile over `splits` K splits (K % (32 splits) == 0, checked by the callers), with the
-// deepest register prefetch that divides the stage count
-template <bool NRM, int E>
-void launch_tile(const GemmParams& p, uint32_t splits, hipStream_t st) {
-  const uint32_t bn = tile_bn(p.M, p.N), nst = p.K / splits / 32;
-  const dim3 tg(ceil_div(p.N, bn), ceil_div(p.M, 128), splits);
-#define QE_TILE_D(D)                                                                             \
-  do {                                                                                           \
-    if (bn == 128) hipLaunchKernelGGL((k_gemm_tile<NRM, E, 128, D>), tg, dim3(256), 0, st, p);   \
-    else hipLaunchKernelGGL((k_gemm_tile<NRM, E, 64, D>), tg, dim3(256), 0, st, p);              \
-  } while (0)
-  if (nst % kTileDepth == 0) QE_TILE_D(kTileDepth);
-  else if (nst % 2 == 0) QE_TILE_D(2);
-  else QE_TILE_D(1);
-#undef QE_TILE_D
-}
-
 // ---------------------------------------------------------------------------------------------
 // Matvec over the NV = M token rows of a short verify pass or chunk (M <= kMvRowsMaxM): the
 // decode step's matvec layout. A row group of TPR threads covers one weight row in 8-column
@@ -893,7 +499,7 @@ void launch_tile(const GemmParams& p, uint32_t splits, hipStream_t st) {
 // chunks (which cover the row) and scales the dot products, s * sum_c W[r,c] (x_c * g_c)
 // (cpu_inference.rs:189-194, 225-257). All loads are issued before the first use. Each token row
 // costs every wave its own products and lane reductions, so past a few rows the matrix cores
-// (k_gemm_skinny) are faster.
+// (k_gemm_kslice) are faster.
 // ---------------------------------------------------------------------------------------------
 template <int TPR, int CPT, int RR, int NV, bool NORM, int EPI, int SM = 0>
 __global__ __launch_bounds__(256) void k_mv_rows(MvRowsParams p) {
@@ -1340,12 +946,6 @@ hipError_t launch_mv_rows(const MvRowsParams& p, bool norm, int epi, hipStream_t
   }
 }
 
-hipError_t launch_rownorm(const float* x, uint32_t M, uint32_t K, float eps, float* s, hipStream_t st) {
-  if (M == 0 || K % 4) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_rownorm, dim3(ceil_div(M, 4)), dim3(256), 0, st, x, M, K, eps, s);
-  return hipGetLastError();
-}
-
 namespace {
 
 // The tile of a k-sliced launch: the workgroups are dealt over 256 CUs, so its time goes with the
@@ -1390,22 +990,57 @@ hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
   }
 }
 
-template <int EPI, int BM, int BN, int NS>
-hipError_t launch_wide_t(const GemmParams& p, hipStream_t st) {
-  const uint64_t wgs = (uint64_t(p.M) + BM - 1) / BM * ((uint64_t(p.N) + BN - 1) / BN);
+// ---- k_gemm_wide: the tile ----
+struct WideTile {
+  uint32_t bm, bn;
+};
+constexpr WideTile kWideTiles[] = {{64, 128}, {64, 192}, {128, 128}, {128, 192}, {128, 256}};
+
+// Clocks of a launch over bm x bn tiles: rounds of 256 workgroups, each K / 32 phases of the longer
+// of its MFMAs (16 clocks each, per SIMD) and its LDS traffic (128 bytes a clock: the fragments four
+// waves read and the block that is written), plus what a workgroup costs besides (fill and drain).
+uint64_t wide_cost(uint32_t M, uint32_t N, uint32_t kz, uint32_t splits, uint32_t bm, uint32_t bn) {
+  const uint64_t wgs = uint64_t((uint64_t(M) + bm - 1) / bm) * ((uint64_t(N) + bn - 1) / bn) * splits;
+  const uint32_t mt = bm / 32, nt = bn / 32;
+  const uint32_t mfma = mt * nt * 2 * 16, lds = 32 * (2 * mt + nt) + bm + bn / 2;
+  return (wgs + 255) / 256 * (uint64_t(kz / 32) * std::max(mfma, lds) + 7000);
+}
+
+WideTile wide_tile(uint32_t M, uint32_t N, uint32_t kz, uint32_t splits, bool heads) {
+  WideTile best{};
+  uint64_t cost = ~uint64_t(0);
+  for (const WideTile& t : kWideTiles) {
+    if (heads && t.bn % kHeadDim) continue;
+    const uint64_t c = wide_cost(M, N, kz, splits, t.bm, t.bn);
+    if (c < cost) {
+      cost = c;
+      best = t;
+    }
+  }
+  return best;
+}
+
+template <int EPI, bool SPLIT, int BM, int BN, int NS>
+hipError_t launch_wide_t(const GemmParams& p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
+  const uint64_t wgs = (uint64_t(p.M) + BM - 1) / BM * ((uint64_t(p.N) + BN - 1) / BN) * splits;
   if (hipError_t e = check_grid(wgs, 512)) return e;
-  hipLaunchKernelGGL((k_gemm_wide<EPI, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p);
+  hipLaunchKernelGGL((k_gemm_wide<EPI, SPLIT, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p, qa);
   return hipGetLastError();
 }
 
-template <int EPI>
-hipError_t launch_wide(const GemmParams& p, hipStream_t st) {
-  const uint64_t c128 = tile_cost(p, 64, 128), c192 = tile_cost(p, 64, 192), c256 = tile_cost(p, 128, 256);
-  if (c256 < c128 && c256 < c192) return launch_wide_t<EPI, 128, 256, 2>(p, st);
-  if (c192 >= c128) return launch_wide_t<EPI, 64, 128, 2>(p, st);
-  // one workgroup per CU: three slots; more: two slots, two workgroups per CU
-  const uint64_t wgs = (uint64_t(p.M) + 63) / 64 * ((uint64_t(p.N) + 191) / 192);
-  return wgs <= 256 ? launch_wide_t<EPI, 64, 192, 3>(p, st) : launch_wide_t<EPI, 64, 192, 2>(p, st);
+template <int EPI, bool SPLIT>
+hipError_t launch_wide(GemmParams p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
+  if (splits == 0 || p.K % (64 * splits)) return hipErrorInvalidValue;
+  p.kz = p.K / splits;
+  const WideTile t = wide_tile(p.M, p.N, p.kz, splits, EPI == kGemmQkRope);
+  if (t.bm == 64 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 64, 128, 4>(p, splits, qa, st);
+  if (t.bm == 128 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 128, 128, 3>(p, splits, qa, st);
+  if (t.bm == 128 && t.bn == 256) return launch_wide_t<EPI, SPLIT, 128, 256, 2>(p, splits, qa, st);
+  if constexpr (EPI != kGemmQkRope) {  // (whole heads)
+    if (t.bm == 64 && t.bn == 192) return launch_wide_t<EPI, SPLIT, 64, 192, 3>(p, splits, qa, st);
+    if (t.bm == 128 && t.bn == 192) return launch_wide_t<EPI, SPLIT, 128, 192, 2>(p, splits, qa, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -1414,63 +1049,42 @@ hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st) 
   if (p.M == 0 || p.N == 0 || p.N % 2 || p.K % 32 || p.K == 0 || p.lda % 4 || !p.A || !p.W || !p.C)
     return hipErrorInvalidValue;
   if (norm && !p.gain) return hipErrorInvalidValue;
-  if (p.M <= kGemmSliceMaxM) {
-    if (norm && epi == kGemmStore) return launch_kslice<true, kGemmStore>(p, st);
-    if (norm && epi == kGemmSiluPair) return launch_kslice<true, kGemmSiluPair>(p, st);
-    if (!norm && epi == kGemmResAdd) return launch_kslice<false, kGemmResAdd>(p, st);
-  }
-  if (!norm && epi == kGemmStore) {
-    // the k-sliced kernel up to two rounds of its smaller tiles, the wide one past that
-    uint64_t slice = ~uint64_t(0);
-    for (uint32_t bm : {32u, 48u, 64u}) slice = std::min(slice, tile_cost(p, bm, 64));
-    const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM &&
-                      std::min({tile_cost(p, 64, 128), tile_cost(p, 64, 192), tile_cost(p, 128, 256)}) < slice;
-    return wide ? launch_wide<kGemmStore>(p, st) : launch_kslice<false, kGemmStore>(p, st);
-  }
-  if (norm && !p.rowscale) return hipErrorInvalidValue;
-  if (rows_kernel(p.M, p.K)) {
-    if (norm && epi == kGemmStore) launch_rows<true, kGemmStore>(p, 1, st);
-    else if (norm && epi == kGemmSiluPair) launch_rows<true, kGemmSiluPair>(p, 1, st);
-    else if (!norm && epi == kGemmResAdd) launch_rows<false, kGemmResAdd>(p, 1, st);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-  }
-  if (norm && epi == kGemmStore) launch_tile<true, kGemmStore>(p, 1, st);
-  else if (norm && epi == kGemmSiluPair) launch_tile<true, kGemmSiluPair>(p, 1, st);
-  else if (!norm && epi == kGemmResAdd) launch_tile<false, kGemmResAdd>(p, 1, st);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (norm && epi == kGemmStore) return launch_kslice<true, kGemmStore>(p, st);
+  if (norm && epi == kGemmSiluPair) return launch_kslice<true, kGemmSiluPair>(p, st);
+  if (!norm && epi == kGemmResAdd) return launch_kslice<false, kGemmResAdd>(p, st);
+  if (norm || epi != kGemmStore) return hipErrorInvalidValue;
+  // the k-sliced kernel up to two rounds of its smaller tiles, the wide one past that
+  uint64_t slice = ~uint64_t(0);
+  for (uint32_t bm : {32u, 48u, 64u}) slice = std::min(slice, tile_cost(p, bm, 64));
+  const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM &&
+                    std::min({tile_cost(p, 64, 128), tile_cost(p, 64, 192), tile_cost(p, 128, 256)}) < slice;
+  return wide ? launch_wide<kGemmStore, false>(p, 1, BatchAttnParams{}, st) : launch_kslice<false, kGemmStore>(p, st);
 }
 
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K) {
-  // tiles of the kernel that runs M rows, and the depth one split must stay a multiple of
-  const bool rows = rows_kernel(M, K);
-  const uint32_t tiles = rows ? ceil_div(N, 128) * ceil_div(M, 64) : ceil_div(N, tile_bn(M, N)) * ceil_div(M, 128);
-  const uint32_t unit = rows ? 64 : 32;
+  // 64 x 128 tiles: split while that leaves CUs without one
+  const uint32_t tiles = ceil_div(N, 128) * ceil_div(M, 64);
   uint32_t z = 1;
-  while (z < 8 && tiles * z < 256 && K % (2 * unit * z) == 0) z *= 2;
+  while (z < 8 && tiles * z < 256 && K % (128 * z) == 0) z *= 2;
   return z;
 }
 
 hipError_t launch_gemm_split(const GemmParams& p, uint32_t splits, hipStream_t st) {
-  if (p.M <= kGemmSliceMaxM || p.N == 0 || p.N % 2 || p.lda % 4 || !p.A || !p.W || !p.C || splits == 0)
-    return hipErrorInvalidValue;
-  if (rows_kernel(p.M, p.K) && p.K % (64 * splits) == 0) {
-    launch_rows<false, kGemmPartial>(p, splits, st);
-    return hipGetLastError();
-  }
-  if (p.K % (32 * splits)) return hipErrorInvalidValue;
-  launch_tile<false, kGemmPartial>(p, splits, st);
-  return hipGetLastError();
+  if (p.M == 0 || p.N == 0 || p.N % 2 || p.lda % 4 || !p.A || !p.W || !p.C) return hipErrorInvalidValue;
+  return launch_wide<kGemmPartial, true>(p, splits, BatchAttnParams{}, st);
 }
 
-L2Prefetch gemm_prefetch_target(const uint16_t* W, uint32_t M, uint32_t N, uint32_t K, int epi) {
-  if (!W || !rows_kernel(M, K)) return L2Prefetch{};
-  const uint32_t bn = epi == kGemmQkRope || epi == kGemmPartial ? 128 : rows_bn(M, N, 1);
-  const uint32_t tiles = ceil_div(N, bn);
-  // workgroup (j, y, z) runs on XCD (j + tiles (y + gridDim.y z)) % 8: j % 8 when tiles is a
-  // multiple of 8 or the grid is one row of tiles
-  if (tiles % 8 && (ceil_div(M, 64) > 1 || epi == kGemmPartial)) return L2Prefetch{};
+hipError_t launch_gemm_silu_split(const GemmParams& p, hipStream_t st) {
+  if (p.M == 0 || p.N == 0 || p.N % 16 || p.lda % 4 || p.ldc % 8 || !p.A || !p.W || !p.C) return hipErrorInvalidValue;
+  return launch_wide<kGemmSiluSplit, true>(p, 1, BatchAttnParams{}, st);
+}
+
+L2Prefetch gemm_prefetch_target(const uint16_t* W, uint32_t M, uint32_t N, uint32_t K) {
+  if (!W) return L2Prefetch{};
+  const uint32_t z = gemm_splits(M, N, K), bn = wide_tile(M, N, K / z, z, false).bn, tiles = ceil_div(N, bn);
+  // workgroup (j, y, z) runs on XCD (j + tiles (y + row tiles x z)) % 8: j % 8 when tiles is a
+  // multiple of 8
+  if (tiles % 8) return L2Prefetch{};
   return L2Prefetch{W, N * (K / 8), bn * (K / 8), tiles};
 }
 
@@ -1481,21 +1095,19 @@ uint32_t tile_prefetch_slots(const L2Prefetch* pf, int n) {
   return uint32_t(std::min<uint64_t>(64, (tot + 4095) / 4096));
 }
 
-hipError_t launch_resadd_partials(float* x, const float* part, uint32_t splits, uint32_t M, uint32_t N, float eps,
-                                  float* s, hipStream_t st) {
-  if (!M || N % 4 || !splits) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_resadd_partials, dim3(M), dim3(256), 0, st, x, part, splits, M, N, eps, s);
+hipError_t launch_resadd_norm_split(float* x, const float* part, uint32_t splits, uint32_t M, uint32_t N, float eps,
+                                    const uint16_t* gain, float* out, hipStream_t st) {
+  if (!M || N % 8 || N > 4096 || !x || (splits && !part) || (gain && !out)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_resadd_norm_split, dim3(M), dim3(256), 0, st, x, part, splits, M, N, eps, gain, out);
   return hipGetLastError();
 }
 
 hipError_t launch_gemm_qk_rope(const GemmParams& g, const BatchAttnParams& a, hipStream_t st) {
-  if (!rows_kernel(g.M, g.K) || g.M != a.M || g.N != (a.n_heads + 2 * a.n_kv) * kHeadDim || !g.rowscale || !g.gain ||
-      !a.q || !a.q_norm || !a.k_norm || !a.rope || !a.k_cache || !a.v_cache || g.lda % 4 || !g.A || !g.W)
-    return hipErrorNotSupported;
+  if (g.M == 0 || g.M != a.M || g.N != (a.n_heads + 2 * a.n_kv) * kHeadDim || !a.q || !a.q_norm || !a.k_norm ||
+      !a.rope || !a.k_cache || !a.v_cache || g.lda % 4 || !g.A || !g.W)
+    return hipErrorInvalidValue;
   if (uint64_t(a.start) + a.M > a.max_seq) return hipErrorInvalidValue;  // the K/V rows must fit the cache
-  const dim3 grid(g.N / 128, ceil_div(g.M, 64), 1);
-  hipLaunchKernelGGL((k_gemm_rows8<true, kGemmQkRope, 128, 1>), grid, dim3(512), 0, st, g, a);
-  return hipGetLastError();
+  return launch_wide<kGemmQkRope, true>(g, 1, a, st);
 }
 
 hipError_t launch_qk_rope(const BatchAttnParams& p, hipStream_t st) {
@@ -1539,11 +1151,11 @@ hipError_t launch_attn_causal(const BatchAttnParams& p, uint32_t runs, hipStream
 #undef QE_ATT
   if (e != hipSuccess || runs == 1) return e;
   const uint32_t n_vec = p.M * p.n_heads;
-  const dim3 mg(ceil_div(n_vec, 2));
-  if (runs <= 4) hipLaunchKernelGGL((k_attn_merge_rows<4>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att);
-  else if (runs <= 8) hipLaunchKernelGGL((k_attn_merge_rows<8>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att);
-  else if (runs <= 16) hipLaunchKernelGGL((k_attn_merge_rows<16>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att);
-  else hipLaunchKernelGGL((k_attn_merge_rows<32>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att);
+  const dim3 mg(ceil_div(n_vec, 8));
+  if (runs <= 4) hipLaunchKernelGGL((k_attn_merge_rows<4>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att, p.att_split);
+  else if (runs <= 8) hipLaunchKernelGGL((k_attn_merge_rows<8>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att, p.att_split);
+  else if (runs <= 16) hipLaunchKernelGGL((k_attn_merge_rows<16>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att, p.att_split);
+  else hipLaunchKernelGGL((k_attn_merge_rows<32>), mg, dim3(256), 0, st, p.part, runs, n_vec, p.att, p.att_split);
   return hipGetLastError();
 }
 

@@ -93,7 +93,7 @@ struct ChunkBufs {
   uint8_t* mem = nullptr;
   uint32_t cap = 0;
   hipStream_t stream = nullptr;
-  float *bx = nullptr, *bs = nullptr, *bqkv = nullptr, *bq = nullptr, *batt = nullptr, *bh = nullptr;
+  float *bx = nullptr, *bxs = nullptr, *bqkv = nullptr, *bq = nullptr, *batt = nullptr, *bh = nullptr;
   float *bpart = nullptr, *bsplit = nullptr;
   std::vector<hipEvent_t> kv_ev;
 };
@@ -172,7 +172,7 @@ struct qe_model {
   // decode attention launches also load the next weights into L2 (QE_L2_PREFETCH=0 turns it off)
   bool l2_prefetch = true;
   // verify passes and chunks of up to kMvRowsMaxM tokens run their projections as multi-row
-  // matvecs (QE_MV_ROWS=0: on the skinny GEMM)
+  // matvecs (QE_MV_ROWS=0: on the k-sliced GEMM)
   bool mv_rows = true;
   // passes of at most 8 / (q heads per KV head) tokens (a verify of up to 4 rows) attend on the
   // decode step's split kernel, all their q heads of a KV head sharing one read of its K/V
@@ -181,11 +181,11 @@ struct qe_model {
   // and their o_proj merges those runs in its prologue when they are few (QE_MV_MERGE=0: a
   // merge launch of its own)
   bool mv_merge = true;
-  // chunks on the 64-row GEMM: the causal attention launch also loads o_proj's weights into the
+  // chunks of more than 64 tokens: the causal attention launch also loads o_proj's weights into the
   // L2 of the XCDs that will read them (QE_PREFILL_PREFETCH=0 turns it off)
   bool prefill_prefetch = true;
   // ... and their lm_head is the decode step's matvec over all their rows, each row's logits
-  // equal to a decode step's (QE_LM_HEAD_ROWS=0: the skinny GEMM; a 2-row pass 0.83 -> 0.80 ms)
+  // equal to a decode step's (QE_LM_HEAD_ROWS=0: the k-sliced GEMM; a 2-row pass 0.83 -> 0.80 ms)
   bool lm_head_rows = true;
   // two-row verify passes through the two launches per layer (QE_VERIFY_FUSED=0: the batch path)
   bool verify_fused = true;
@@ -200,7 +200,7 @@ struct qe_model {
   // multi-token (chunked prefill / verify) buffers, grown on first use: up to batch_cap tokens
   uint8_t* batch_mem = nullptr;
   uint32_t batch_cap = 0, batch_logit_rows = 0;
-  float *bx = nullptr, *bs = nullptr, *bqkv = nullptr, *bq = nullptr, *batt = nullptr, *bh = nullptr;
+  float *bx = nullptr, *bxs = nullptr, *bqkv = nullptr, *bq = nullptr, *batt = nullptr, *bh = nullptr;
   float* bpart = nullptr;   // causal attention partials
   float* bsplit = nullptr;  // split GEMM partial sums [splits][cap][hidden]
   // a chunked prefill on prefill_streams streams (QE_PREFILL_STREAMS, 1 to 4): the extra streams
@@ -855,7 +855,7 @@ int ensure_batch(qe_model* m, uint32_t cap, uint32_t logit_rows) {
   const size_t QD = c.num_attention_heads * D, KD = c.num_key_value_heads * D;
   size_t off = 0;
   auto take = [&](size_t b) { size_t o = off; off = align_up(off + b, 256); return o; };
-  const size_t ox = take(cap * H * 4), os = take(cap * 4), oqkv = take(cap * (QD + 2 * KD) * 4),
+  const size_t ox = take(cap * H * 4), oxs = take(cap * H * 4), oqkv = take(cap * (QD + 2 * KD) * 4),
                oq = take(cap * QD * 4), oatt = take(cap * QD * 4), oh = take(cap * I * 4),
                ologit = take(size_t(logit_rows) * c.vocab_size * 4);
   // attention partials: the most (tokens x key runs) any chunk of up to cap tokens asks for
@@ -875,7 +875,7 @@ int ensure_batch(qe_model* m, uint32_t cap, uint32_t logit_rows) {
   m->batch_cap = cap;
   m->batch_logit_rows = logit_rows;
   m->bx = reinterpret_cast<float*>(m->batch_mem + ox);
-  m->bs = reinterpret_cast<float*>(m->batch_mem + os);
+  m->bxs = reinterpret_cast<float*>(m->batch_mem + oxs);
   m->bqkv = reinterpret_cast<float*>(m->batch_mem + oqkv);
   m->bq = reinterpret_cast<float*>(m->batch_mem + oq);
   m->batt = reinterpret_cast<float*>(m->batch_mem + oatt);
@@ -912,7 +912,7 @@ int ensure_streams(qe_model* m, uint32_t cap, int streams) {
     const uint32_t bcap = std::max(cap, b.cap);
     size_t off = 0;
     auto take = [&](size_t n) { size_t o = off; off = align_up(off + n, 256); return o; };
-    const size_t ox = take(bcap * H * 4), os = take(bcap * 4), oqkv = take(bcap * (QD + 2 * KD) * 4),
+    const size_t ox = take(bcap * H * 4), oxs = take(bcap * H * 4), oqkv = take(bcap * (QD + 2 * KD) * 4),
                  oq = take(bcap * QD * 4), oatt = take(bcap * QD * 4), oh = take(bcap * I * 4);
     size_t part_rows = 0;
     for (uint32_t M = 1; M <= bcap; M++)
@@ -927,7 +927,7 @@ int ensure_streams(qe_model* m, uint32_t cap, int streams) {
     HIP_TRY(hipMalloc(&b.mem, off));
     b.cap = bcap;
     b.bx = reinterpret_cast<float*>(b.mem + ox);
-    b.bs = reinterpret_cast<float*>(b.mem + os);
+    b.bxs = reinterpret_cast<float*>(b.mem + oxs);
     b.bqkv = reinterpret_cast<float*>(b.mem + oqkv);
     b.bq = reinterpret_cast<float*>(b.mem + oq);
     b.batt = reinterpret_cast<float*>(b.mem + oatt);
@@ -972,7 +972,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
                   const qe::TokenIds* ids_v = nullptr, const ChunkStream* cs = nullptr) {
   const ChunkBufs* xb = cs && cs->set > 0 ? &m->extra[cs->set - 1] : nullptr;
   float* const bx = xb ? xb->bx : m->bx;
-  float* const bs = xb ? xb->bs : m->bs;
+  float* const bxs = xb ? xb->bxs : m->bxs;
   float* const bqkv = xb ? xb->bqkv : m->bqkv;
   float* const bq = xb ? xb->bq : m->bq;
   float* const batt = xb ? xb->batt : m->batt;
@@ -986,48 +986,44 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   const size_t layer_kv = size_t(c.num_key_value_heads) * kv->max_seq * D * el;
   hipStream_t s = xb ? xb->stream : m->stream;
   const float eps = c.rms_norm_eps;
-  // Up to kGemmSliceMaxM rows the k-sliced GEMM computes each norm's row scales itself and adds
-  // residuals in its epilogue. Past that, bs holds the row scales of the current norm input:
-  // from a rownorm launch for layer 0, then from the reduction that finishes each split o_proj /
-  // down (residual add + the next norm's scales in one pass).
+  // Up to kGemmSliceMaxM rows (or widths that are no multiples of 64) the k-sliced GEMM computes each
+  // norm within and adds residuals in its epilogue. Past that, what the GEMMs read is written split
+  // into bf16 halves by whatever computes it: bxs holds the current norm of x, from the reduction
+  // that finishes each split o_proj / down (residual add + the next norm in one pass).
   // Up to kMvRowsMaxM rows the projections are matvecs over the M token rows: each weight is
   // loaded once per pass, the norm is computed per row in the kernel and the residual is added in
-  // its epilogue (the lm_head of a verify stays on the skinny GEMM).
-  const bool skinny = M <= qe::kGemmSliceMaxM;
+  // its epilogue (the lm_head of a verify stays on the k-sliced GEMM).
+  const bool wide = M > qe::kGemmSliceMaxM && H % 64 == 0 && I % 64 == 0 && QD % 64 == 0;
   const bool mv = m->mv_rows && M <= qe::kMvRowsMaxM;
   auto gemm = [&](const float* A, uint32_t lda, const uint16_t* gain, const uint16_t* W, uint32_t N, uint32_t K,
                   float* C, uint32_t ldc, int epi) -> int {
-    // gate|up (the widest projection) at 4 rows is faster on the skinny GEMM: 1.405 vs 1.431 ms
+    // gate|up (the widest projection) at 4 rows is faster on the k-sliced GEMM: 1.405 vs 1.431 ms
     // per k = 4 verify (at 3 rows the matvec still wins)
     if (mv && lda == K && W != m->lm_head && !(epi == qe::kGemmSiluPair && M >= 4)) {
       qe::MvRowsParams r{W, A, gain, C, M, N, K, ldc, eps};
       HIP_TRY(qe::launch_mv_rows(r, gain != nullptr, epi, s));
       return QE_OK;
     }
-    qe::GemmParams g{A, lda, bs, gain, W, M, N, K, C, ldc, eps};
+    qe::GemmParams g{A, lda, gain, W, M, N, K, C, ldc, eps, 0};
     HIP_TRY(qe::launch_gemm(g, gain != nullptr, epi, s));
     return QE_OK;
   };
-  // x += A W^T, then bs = the row scales of the updated x
-  auto gemm_resadd = [&](const float* A, uint32_t lda, const uint16_t* W, uint32_t K) -> int {
-    if (mv || skinny) return gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd);
-    if (K % 64) {  // no split: residual epilogue, then the row scales
-      if (int rc2 = gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd)) return rc2;
-      HIP_TRY(qe::launch_rownorm(bx, M, H, eps, bs, s));
-      return QE_OK;
-    }
+  // x += A W^T; in a chunk (A as split rows) also bxs = the next norm of x (gain; null: none) as split rows
+  auto gemm_resadd = [&](const float* A, uint32_t lda, const uint16_t* W, uint32_t K, const uint16_t* gain) -> int {
+    if (!wide) return gemm(A, lda, nullptr, W, H, K, bx, H, qe::kGemmResAdd);
     const uint32_t z = qe::gemm_splits(M, H, K);
-    qe::GemmParams g{A, lda, nullptr, nullptr, W, M, H, K, bsplit, H, eps};
+    qe::GemmParams g{A, lda, nullptr, W, M, H, K, bsplit, H, eps, 0};
     HIP_TRY(qe::launch_gemm_split(g, z, s));
-    HIP_TRY(qe::launch_resadd_partials(bx, bsplit, z, M, H, eps, bs, s));
+    HIP_TRY(qe::launch_resadd_norm_split(bx, bsplit, z, M, H, eps, gain, bxs, s));
     return QE_OK;
   };
   int rc;
   if (ids_v) HIP_TRY(qe::launch_embed_rows(m->embed, *ids_v, M, H, bx, s));
   else HIP_TRY(qe::launch_embed_rows(m->embed, ids, M, H, bx, s));
-  if (!skinny) HIP_TRY(qe::launch_rownorm(bx, M, H, eps, bs, s));
+  if (wide) HIP_TRY(qe::launch_resadd_norm_split(bx, nullptr, 0, M, H, eps, m->layers[0].w_in, bxs, s));
   for (uint64_t l = 0; l < c.num_hidden_layers; l++) {
     const Layer& w = m->layers[l];
+    const uint16_t* next_in = l + 1 < c.num_hidden_layers ? m->layers[l + 1].w_in : nullptr;
     // q/k norm + RoPE, K/V append, causal attention (cpu_inference.rs:134-162)
     qe::BatchAttnParams a{};
     a.qkv = bqkv; a.q = bq; a.att = batt; a.q_norm = w.q_norm; a.k_norm = w.k_norm; a.rope = kv->rope;
@@ -1036,15 +1032,12 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
     a.M = M; a.start = start; a.max_seq = uint32_t(kv->max_seq);
     a.n_heads = uint32_t(c.num_attention_heads); a.n_kv = uint32_t(c.num_key_value_heads);
     a.eps = eps; a.scale = 1.0f / sqrtf(float(D)); a.kv_bf16 = kv->dtype == QE_KV_BF16;
-    // input_layernorm + q|k|v (cpu_inference.rs:129-132); chunks on the 64-row GEMM do the q/k
-    // norm, RoPE and K/V append in its epilogue, the others in k_qk_rope
-    hipError_t fused = hipErrorNotSupported;
-    if (!mv && !skinny) {
-      const qe::GemmParams g{bx, H, bs, w.w_in, w.w_qkv, M, QD + 2 * KD, H, bqkv, QD + 2 * KD, eps};
-      fused = qe::launch_gemm_qk_rope(g, a, s);
-      if (fused != hipSuccess && fused != hipErrorNotSupported) HIP_TRY(fused);
-    }
-    if (fused != hipSuccess) {
+    // input_layernorm + q|k|v (cpu_inference.rs:129-132); long chunks do the q/k norm, RoPE and K/V
+    // append in the GEMM's epilogue, the others in k_qk_rope
+    if (wide) {
+      const qe::GemmParams g{bxs, H, nullptr, w.w_qkv, M, QD + 2 * KD, H, bqkv, QD + 2 * KD, eps, 0};
+      HIP_TRY(qe::launch_gemm_qk_rope(g, a, s));
+    } else {
       if ((rc = gemm(bx, H, w.w_in, w.w_qkv, QD + 2 * KD, H, bqkv, QD + 2 * KD, qe::kGemmStore))) return rc;
       HIP_TRY(qe::launch_qk_rope(a, s));
     }
@@ -1069,7 +1062,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       if (rows_per_kv == 8) r.row_split = 2;
       if (m->l2_prefetch && mv) {
         // as in the decode step: the attention is latency-bound, so extra workgroups load this
-        // layer's gate|up (the skinny GEMM's rows at 4 tokens, else the multi-row matvec's) and
+        // layer's gate|up (the k-sliced GEMM's rows at 4 tokens, else the multi-row matvec's) and
         // down weights into the L2 of the XCDs that will read them
         if (M < 4) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
         r.pf[1] = qe::l2_prefetch_target(w.w_down, H, I, qe::kCopy, qe::kResAdd);
@@ -1082,10 +1075,11 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       HIP_TRY(qe::launch_attention_rows(r, splits, merge_splits ? nullptr : batt, s));
     } else {
       a.part = bpart;
-      if (m->prefill_prefetch && !skinny) {
+      a.att_split = wide;
+      if (m->prefill_prefetch && wide) {
         // the attention is latency-bound: extra workgroups load o_proj's weights (a split GEMM)
         // into L2
-        a.pf.pf[0] = qe::gemm_prefetch_target(w.w_o, M, H, QD, qe::kGemmPartial);
+        a.pf.pf[0] = qe::gemm_prefetch_target(w.w_o, M, H, QD);
         a.pf.slots = qe::tile_prefetch_slots(a.pf.pf, qe::kMaxPrefetch);
       }
       HIP_TRY(qe::launch_attn_causal(a, qe::attn_causal_runs(M, start, a.n_heads, a.n_kv), s));
@@ -1095,12 +1089,17 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       qe::MvRowsParams r{w.w_o, nullptr, nullptr, bx, M, H, QD, H, eps};
       r.attn_part = bpart; r.attn_splits = merge_splits; r.tok_heads = a.n_heads / a.n_kv;
       HIP_TRY(qe::launch_mv_rows_merge(r, s));
-    } else if ((rc = gemm_resadd(batt, QD, w.w_o, QD))) {
+    } else if ((rc = gemm_resadd(batt, QD, w.w_o, QD, w.w_post))) {
       return rc;
     }
     // post_attention_layernorm + gate/up + silu*up, down + residual (cpu_inference.rs:167-172)
-    if ((rc = gemm(bx, H, w.w_post, w.w_gu, 2 * I, H, bh, I, qe::kGemmSiluPair))) return rc;
-    if ((rc = gemm_resadd(bh, I, w.w_down, I))) return rc;
+    if (wide) {
+      const qe::GemmParams g{bxs, H, nullptr, w.w_gu, M, 2 * I, H, bh, I, eps, 0};
+      HIP_TRY(qe::launch_gemm_silu_split(g, s));
+    } else if ((rc = gemm(bx, H, w.w_post, w.w_gu, 2 * I, H, bh, I, qe::kGemmSiluPair))) {
+      return rc;
+    }
+    if ((rc = gemm_resadd(bh, I, w.w_down, I, next_in))) return rc;
   }
   // final norm + lm_head (cpu_inference.rs:175-178)
   if (logits == kAllLogits) {
@@ -2052,8 +2051,8 @@ int qe_op_gemm_bf16(const float* a, const void* w, float* c, uint64_t m, uint64_
     return fail(QE_ERR_ARG, "need m > 0, n even, k a multiple of 32");
   if (reinterpret_cast<uintptr_t>(a) % 16 || reinterpret_cast<uintptr_t>(w) % 16)
     return fail(QE_ERR_ARG, "a and w must be 16-byte aligned");
-  qe::GemmParams g{a, uint32_t(k), nullptr, nullptr, static_cast<const uint16_t*>(w), uint32_t(m), uint32_t(n),
-                   uint32_t(k), c, uint32_t(n), 0.f};
+  qe::GemmParams g{a, uint32_t(k), nullptr, static_cast<const uint16_t*>(w), uint32_t(m), uint32_t(n),
+                   uint32_t(k), c, uint32_t(n), 0.f, 0};
   HIP_TRY(qe::launch_gemm(g, false, qe::kGemmStore, static_cast<hipStream_t>(stream)));
   return QE_OK;
 }

@@ -37,6 +37,33 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8& hi, bf16x8& 
   lo = __builtin_bit_cast(bf16x8, l);
 }
 
+// Split rows: a row of n floats (n a multiple of 8) held as its two bf16 halves in the same n x 4
+// bytes, per 8 values the 8 hi then the 8 lo. A producer that writes them saves every reader the
+// split, and the halves of 8 consecutive k are the 16-byte pieces an MFMA operand wants.
+// store_split2 / 4: elements i, i + 1 (i even) / i .. i + 3 (i a multiple of 4) of the row at `row`.
+__device__ __forceinline__ uint32_t split_pair(float a, float b, uint32_t& lo) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+  const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xFFFF0000u);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
+  return hi;
+}
+__device__ __forceinline__ void store_split2(float* row, uint32_t i, float a, float b) {
+  uint32_t* o = reinterpret_cast<uint32_t*>(row) + (i >> 3) * 8 + ((i & 7) >> 1);
+  uint32_t lo;
+  o[0] = split_pair(a, b, lo);
+  o[4] = lo;
+}
+__device__ __forceinline__ void store_split4(float* row, uint32_t i, float a, float b, float c, float d) {
+  uint2* o = reinterpret_cast<uint2*>(row) + (i >> 3) * 4 + ((i & 7) >> 2);
+  uint2 hi, lo;
+  hi.x = split_pair(a, b, lo.x);
+  hi.y = split_pair(c, d, lo.y);
+  o[0] = hi;
+  o[2] = lo;
+}
+
 // One direct-to-LDS load of a wave: lane l's 16 bytes at `src` go to LDS byte address lds + 16 l.
 // The compiler does not count it: a reader waits with wait_dma first. (No output registers.)
 __device__ __forceinline__ void dma16(uint32_t lds, const void* src) {
@@ -65,13 +92,17 @@ __device__ __forceinline__ void wait_steps(uint32_t steps) {
 
 // Writes columns n .. n + 3 (n a multiple of 4, N even) of row m < M; vec: C and its rows are
 // aligned for 16-byte stores. kGemmSiluPair: columns 2i / 2i + 1 are gate_i / up_i
-// (cpu_inference.rs:170).
+// (cpu_inference.rs:170); kGemmSiluSplit: the same as a split row (N a multiple of 4).
 template <int EPI>
 __device__ __forceinline__ void emit4(const GemmParams& p, uint32_t m, uint32_t n, f32x4 v, bool vec) {
   if constexpr (EPI == kGemmSiluPair) {
     float* c = p.C + size_t(m) * p.ldc + (n >> 1);
     if (n < p.N) c[0] = v[0] / (1.0f + expf(-v[0])) * v[1];
     if (n + 2 < p.N) c[1] = v[2] / (1.0f + expf(-v[2])) * v[3];
+  } else if constexpr (EPI == kGemmSiluSplit) {
+    if (n < p.N)
+      store_split2(p.C + size_t(m) * p.ldc, n >> 1, v[0] / (1.0f + expf(-v[0])) * v[1],
+                   v[2] / (1.0f + expf(-v[2])) * v[3]);
   } else {
     float* c = p.C + size_t(m) * p.ldc + n;
     if (vec && n + 3 < p.N) {
@@ -246,49 +277,65 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_kslice(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// GEMM for many rows: tile BM (m) x BN (n), eight waves as 2 x 2 (a quarter of the tile each) x
-// the two 32-deep halves of every 64-deep stage; K a multiple of 64. The stages of both operands
-// are loaded straight into a ring of NS LDS slots, NS - 1 ahead, one barrier per stage: A rows of 256 bytes (64
-// f32, chunk c at place (c & 8) | ((c ^ row) & 7)), then W rows of 128 bytes (chunk c at place
-// c ^ (row & 7)). The two waves of a quarter hand each other half of their blocks at the end:
-// C = (sum over the even 32-k blocks) + (sum over the odd ones), or the other way round.
+// GEMM for many rows: tile BM (m) x BN (n), K a multiple of 64, eight waves as 2 x 2 (a quarter of the
+// tile each) x the two 32-deep halves of every 64-deep stage. The stages of both operands are loaded
+// straight into a ring of NS LDS slots, NS - 1 ahead, one barrier per stage, in whole 128-byte lines
+// (with every CU loading, L2 gives a CU 115 B/ns in lines and 70 in halves of them): A rows of 256
+// bytes (chunk c of 16 bytes at place (c & 8) | ((c ^ row) & 7)), then W rows of 128 bytes (chunk c at
+// place c ^ (row & 7)).
+// SPLIT: A rows are split rows, whose lanes read hi and lo where an f32 row's hold their eight
+// floats; otherwise A is f32 and split here.
+// C = (sum over the even 32-k blocks) + (sum over the odd ones), or the other way round: the two
+// waves of a quarter hand each other half of their rows at the end.
+// kGemmQkRope: a tile holds whole heads; the columns of a wave are dims d and d + 64 of its head(s).
+// Bound: 25 us per 1024 of K at 2048 x 4096 are 1375 TFLOP/s of MFMAs, against 1590 of a large plain
+// library product and 2055 of MFMAs alone on random operands (2430 on zeros: the clock gives way to
+// power). Two other schedules of the same tiles (the two halves in antiphase; fragments read a stage
+// ahead) ran at the same rate per stage and started 0.6 - 1.1 us later.
 // ---------------------------------------------------------------------------------------------
-template <int EPI, int BM, int BN, int NS>
-__global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p) {
-  constexpr int NW = 8, MT = BM / 32, NT = BN / 32;
-  constexpr int AI = BM / 4 / NW, WI = BN / 8 / NW;  // loads per wave per stage
-  static_assert(AI * 4 * NW == BM && WI * 8 * NW == BN && MT % 2 == 0, "tile");
+template <int EPI, bool SPLIT, int BM, int BN, int NS>
+__global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p, BatchAttnParams qa) {
+  constexpr int MT = BM / 32, NT = BN / 32;
+  constexpr int AI = BM / 32, WI = BN / 64;  // loads per wave and stage
+  static_assert(AI * 32 == BM && WI * 64 == BN && MT % 2 == 0, "tile");
   constexpr uint32_t ABYTES = BM * 256, SBYTES = ABYTES + BN * 128;
   static_assert(uint32_t(BM) * BN * 4 <= NS * SBYTES, "the sums meet over the ring");
+  constexpr bool HALF_HEADS = EPI == kGemmQkRope && BN == kHeadDim;  // two waves share a head
+  static_assert(EPI != kGemmQkRope || BN == kHeadDim || BN == 2 * kHeadDim, "whole heads");
   __shared__ __align__(16) uint8_t smem[NS * SBYTES];
+  __shared__ float squares[HALF_HEADS ? 2 * BM : 1];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kh = wave >> 2, pr = wave & 3, wm = pr & 1, wn = pr >> 1;
-  const uint32_t ncol = ceil_div(p.N, uint32_t(BN));
-  const uint32_t m0 = blockIdx.x / ncol * BM, n0 = blockIdx.x % ncol * BN;
-  const uint32_t nst = p.K / 64, lds0 = lds_address(smem);
+  const int grp = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
+  const uint32_t ncol = ceil_div(p.N, uint32_t(BN)), tiles = ncol * ceil_div(p.M, uint32_t(BM));
+  const uint32_t z = blockIdx.x / tiles, t = blockIdx.x % tiles, m0 = t / ncol * BM, n0 = t % ncol * BN;
+  const uint32_t nst = p.kz / 64, lds0 = lds_address(smem);
+  // tile column of fragment j's first column
+  auto col = [&](int j) __attribute__((always_inline)) {
+    return HALF_HEADS ? 64 * (j / (NT / 2)) + 32 * wn + 16 * (j % (NT / 2)) : 16 * (wn * NT + j);
+  };
 
   const uint8_t *asrc[AI], *wsrc[WI];  // of the next stage to load (rows past M or N: the last one)
 #pragma unroll
   for (int i = 0; i < AI; i++) {
-    const uint32_t r = 4 * (wave + NW * i) + (lane >> 4), c = lane & 15, lc = (c & 8) | ((c ^ r) & 7);
-    asrc[i] = reinterpret_cast<const uint8_t*>(p.A + size_t(min(m0 + r, p.M - 1)) * p.lda) + lc * 16;
+    const uint32_t r = 4 * (wave + 8 * i) + (lane >> 4), c = lane & 15, lc = (c & 8) | ((c ^ r) & 7);
+    asrc[i] = reinterpret_cast<const uint8_t*>(p.A + size_t(min(m0 + r, p.M - 1)) * p.lda + size_t(z) * p.kz) + lc * 16;
   }
 #pragma unroll
   for (int i = 0; i < WI; i++) {
-    const uint32_t r = 8 * (wave + NW * i) + (lane >> 3), lc = (lane & 7) ^ (r & 7);
-    wsrc[i] = reinterpret_cast<const uint8_t*>(p.W + size_t(min(n0 + r, p.N - 1)) * p.K) + lc * 16;
+    const uint32_t r = 8 * (wave + 8 * i) + (lane >> 3), lc = (lane & 7) ^ (r & 7);
+    wsrc[i] = reinterpret_cast<const uint8_t*>(p.W + size_t(min(n0 + r, p.N - 1)) * p.K + size_t(z) * p.kz) + lc * 16;
   }
   auto issue = [&](uint32_t slot) __attribute__((always_inline)) {
     const uint32_t l = lds0 + slot * SBYTES;
 #pragma unroll
     for (int i = 0; i < AI; i++) {
-      dma16(l + uint32_t(wave + NW * i) * 1024, asrc[i]);
+      dma16(l + uint32_t(wave + 8 * i) * 1024, asrc[i]);
       asrc[i] += 256;
     }
 #pragma unroll
     for (int i = 0; i < WI; i++) {
-      dma16(l + ABYTES + uint32_t(wave + NW * i) * 1024, wsrc[i]);
+      dma16(l + ABYTES + uint32_t(wave + 8 * i) * 1024, wsrc[i]);
       wsrc[i] += 128;
     }
   };
@@ -298,9 +345,9 @@ __global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p) {
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint32_t ar = (16 * wm * MT + li) * 256 + kh * 128, ws = ABYTES + (16 * wn * NT + li) * 128;
+  const uint32_t ar = (16 * wm * MT + li) * 256 + grp * 128;
   const uint32_t a0 = ar + ((2 * kg) ^ (li & 7)) * 16, a1 = ar + ((2 * kg + 1) ^ (li & 7)) * 16;
-  const uint32_t w0 = ws + ((4 * kh + kg) ^ (li & 7)) * 16;
+  const uint32_t w0 = ABYTES + li * 128 + ((4 * grp + kg) ^ (li & 7)) * 16;
 #pragma unroll
   for (int i = 0; i < NS - 1; i++)
     if (uint32_t(i) < nst) issue(i);
@@ -321,13 +368,18 @@ __global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p) {
       y[i] = *reinterpret_cast<const f32x4*>(sp + a1 + i * 4096);
     }
 #pragma unroll
-    for (int j = 0; j < NT; j++) w[j] = *reinterpret_cast<const bf16x8*>(sp + w0 + j * 2048);
+    for (int j = 0; j < NT; j++) w[j] = *reinterpret_cast<const bf16x8*>(sp + w0 + col(j) * 128);
     if (s + NS - 1 < nst) issue(slot == 0 ? NS - 1 : slot - 1);
 #pragma unroll
     for (int i = 0; i < MT; i++) {
-      const float v[8] = {x[i][0], x[i][1], x[i][2], x[i][3], y[i][0], y[i][1], y[i][2], y[i][3]};
       bf16x8 hi, lo;
-      split8(v, hi, lo);
+      if constexpr (SPLIT) {
+        hi = __builtin_bit_cast(bf16x8, x[i]);
+        lo = __builtin_bit_cast(bf16x8, y[i]);
+      } else {
+        const float v[8] = {x[i][0], x[i][1], x[i][2], x[i][3], y[i][0], y[i][1], y[i][2], y[i][3]};
+        split8(v, hi, lo);
+      }
 #pragma unroll
       for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], hi, acc[i][j], 0, 0, 0);
 #pragma unroll
@@ -337,6 +389,7 @@ __global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p) {
   }
 
   f32x4* red = reinterpret_cast<f32x4*>(smem);
+  const int pr = wave & 3;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < MT / 2; i++)
@@ -347,21 +400,88 @@ __global__ __launch_bounds__(512) void k_gemm_wide(GemmParams p) {
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const float a = acc[i][j][r], b = acc[i + MT / 2][j][r];
-        give[r] = kh ? a : b;
-        keep[r] = kh ? b : a;
+        give[r] = grp ? a : b;
+        keep[r] = grp ? b : a;
       }
-      red[((kh * 4 + pr) * (MT / 2 * NT) + i * NT + j) * 64 + lane] = give;
+      red[((grp * 4 + pr) * (MT / 2 * NT) + i * NT + j) * 64 + lane] = give;
       acc[i][j] = keep;
     }
   __syncthreads();
-  const bool vec = p.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(p.C) % 16 == 0;
 #pragma unroll
-  for (int i = 0; i < MT / 2; i++) {
-    const uint32_t m = m0 + uint32_t(16 * (wm * MT + i + kh * (MT / 2)) + li);
+  for (int i = 0; i < MT / 2; i++)
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
-      const f32x4 s = acc[i][j] + red[(((1 - kh) * 4 + pr) * (MT / 2 * NT) + i * NT + j) * 64 + lane];
-      if (m < p.M) emit4<EPI>(p, m, n0 + uint32_t(16 * (wn * NT + j) + 4 * kg), s, vec);
+    for (int j = 0; j < NT; j++) acc[i][j] += red[(((1 - grp) * 4 + pr) * (MT / 2 * NT) + i * NT + j) * 64 + lane];
+  const uint32_t mrow = 16 * (wm * MT + grp * (MT / 2)) + li;  // tile row of acc[0]
+  if constexpr (EPI == kGemmQkRope) {
+    // per-head q/k RMSNorm, RoPE and the K/V append (cpu_inference.rs:134-141, 189-215)
+    const uint32_t hh = (n0 + (HALF_HEADS ? 0 : wn * kHeadDim)) / kHeadDim;  // head of [q | k | v]
+    const bool isq = hh < qa.n_heads, isk = !isq && hh < qa.n_heads + qa.n_kv, isv = !isq && !isk;
+    constexpr int NH = NT / 2;
+    auto dim = [&](int j) __attribute__((always_inline)) { return (HALF_HEADS ? col(j) : 16 * j) + 4 * kg; };
+    float q[MT / 2];
+#pragma unroll
+    for (int i = 0; i < MT / 2; i++) {
+      q[i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) q[i] += acc[i][j][r] * acc[i][j][r];
+      q[i] += __shfl_xor(q[i], 16);
+      q[i] += __shfl_xor(q[i], 32);
+      if (HALF_HEADS && kg == 0) squares[wn * BM + mrow + 16 * i] = q[i];
+    }
+    if constexpr (HALF_HEADS) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < MT / 2; i++) q[i] = squares[mrow + 16 * i] + squares[BM + mrow + 16 * i];
+    }
+#pragma unroll
+    for (int i = 0; i < MT / 2; i++) {
+      const uint32_t m = m0 + mrow + 16 * i, pos = qa.start + min(m, p.M - 1);
+      if (!isv) {
+        const uint16_t* gain = isq ? qa.q_norm : qa.k_norm;
+        const float sc = 1.0f / sqrtf(q[i] / float(kHeadDim) + qa.eps);
+        const float* rope = qa.rope + size_t(pos) * kHeadDim;  // (cos, sin) of dims 0 .. 63
+#pragma unroll
+        for (int j = 0; j < NH; j++) {
+          const f32x4 c01 = *reinterpret_cast<const f32x4*>(rope + 2 * dim(j));
+          const f32x4 c23 = *reinterpret_cast<const f32x4*>(rope + 2 * dim(j) + 4);
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float cs = r < 2 ? c01[2 * r] : c23[2 * r - 4], sn = r < 2 ? c01[2 * r + 1] : c23[2 * r - 3];
+            const float a = acc[i][j][r] * sc * bf16f(gain[dim(j) + r]);
+            const float b = acc[i][j + NH][r] * sc * bf16f(gain[dim(j + NH) + r]);
+            acc[i][j][r] = a * cs - b * sn;
+            acc[i][j + NH][r] = b * cs + a * sn;
+          }
+        }
+      }
+      if (m >= p.M || hh >= qa.n_heads + 2 * qa.n_kv) continue;  // (a tile's second head may lie past N)
+      const uint32_t kvh = isk ? hh - qa.n_heads : hh - qa.n_heads - qa.n_kv;
+      const size_t slot = isq ? (size_t(m) * qa.n_heads + hh) * kHeadDim : (size_t(kvh) * qa.max_seq + pos) * kHeadDim;
+      void* out = isq ? qa.q : isk ? qa.k_cache : qa.v_cache;
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        if (!isq && qa.kv_bf16) {
+          uint16_t* o = static_cast<uint16_t*>(out) + slot + dim(j);
+          const uint32_t lo = f32_to_bf16(acc[i][j][0]) | uint32_t(f32_to_bf16(acc[i][j][1])) << 16;
+          const uint32_t hi = f32_to_bf16(acc[i][j][2]) | uint32_t(f32_to_bf16(acc[i][j][3])) << 16;
+          *reinterpret_cast<uint2*>(o) = make_uint2(lo, hi);
+        } else {
+          *reinterpret_cast<f32x4*>(static_cast<float*>(out) + slot + dim(j)) = acc[i][j];
+        }
+      }
+    }
+  } else {
+    GemmParams q = p;
+    if (EPI == kGemmPartial) q.C += size_t(z) * p.M * p.ldc;
+    const bool vec = p.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(p.C) % 16 == 0;
+#pragma unroll
+    for (int i = 0; i < MT / 2; i++) {
+      const uint32_t m = m0 + mrow + 16 * i;
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+        if (m < p.M) emit4<EPI>(q, m, n0 + uint32_t(col(j) + 4 * kg), acc[i][j], vec);
     }
   }
 }

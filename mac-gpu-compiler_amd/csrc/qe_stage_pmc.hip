@@ -18,8 +18,8 @@
 //                         from one launch to the next
 //   qe_stage_pmc --gemm   the chunked prefill's GEMM instead (launch_gemm, no norm, plain store),
 //                         3 launches at each of M x N x K = 2048 x 4096 x 1024 (q|k|v of a
-//                         2048-token chunk: k_gemm_tile), 512 x 6144 x 1024 and 512 x 4096 x 1024
-//                         (gate|up and q|k|v of a 512-token chunk: k_gemm_rows8), for the
+//                         2048-token chunk: k_gemm_wide), 512 x 6144 x 1024 and 512 x 4096 x 1024
+//                         (gate|up and q|k|v of a 512-token chunk: k_gemm_wide), for the
 //                         matrix-core counters (SQ_INSTS_MFMA, SQ_VALU_MFMA_BUSY_CYCLES, ...);
 //                         --reps R launches per shape instead of 3, --random fills A and W with
 //                         hashed values in [-1, 1) and [-1/64, 1/64) instead of constants (the
@@ -183,7 +183,7 @@ int main(int argc, char** argv) {
         // bf16 pairs (0, 0.0078125): any finite values give the same matrix-core work
         k_fill_f32<<<1024, 256, 0, gs>>>(reinterpret_cast<float*>(W), size_t(N) * K / 2, 0.0078125f);
       }
-      const qe::GemmParams g{A, K, nullptr, nullptr, W, M, N, K, C, N, 1e-6f};
+      const qe::GemmParams g{A, K, nullptr, W, M, N, K, C, N, 1e-6f, 0};
       for (int r = 0; r < reps; r++) CK(qe::launch_gemm(g, false, qe::kGemmStore, gs));
       CK(hipStreamSynchronize(gs));
       CK(hipFree(A));

@@ -1,0 +1,35 @@
+"""Chunks of more than 64 tokens: their GEMMs on split rows (norm, attention and SwiGLU outputs held
+as bf16 halves) against the same prompt token by token, at ragged rows, odd numbers of 64-deep
+stages, a last column tile that holds one of its two heads, and widths that are no multiple of 64
+(the k-sliced GEMMs at any number of rows)."""
+import numpy as np
+import pytest
+
+import qe
+
+pytestmark = pytest.mark.gpu
+
+CONFIGS = {
+    "tiny": qe.Config(256, 512, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999),
+    "odd_stages": qe.Config(320, 448, 2, 4, 4, 128, 1000, 1e-6, 1e6, 999),
+    "half_stage": qe.Config(288, 480, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999),
+    "93_heads": qe.Config(256, 512, 1, 31, 31, 128, 1000, 1e-6, 1e6, 999),
+}
+
+
+@pytest.mark.parametrize("name,n,kv", [("tiny", 65, "f32"), ("tiny", 129, "bf16"), ("tiny", 1025, "f32"),
+                                       ("odd_stages", 200, "f32"), ("half_stage", 150, "f32"),
+                                       ("93_heads", 2001, "f32")])
+def test_chunk_matches_token_by_token(gpu, tmp_path, name, n, kv):
+    model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 7, CONFIGS[name]))
+    dtype = qe.QE_KV_BF16 if kv == "bf16" else qe.QE_KV_F32
+    ids = qe.random_prompt(5, n, 1000)
+    a, b = qe.KVCache(model, n + 4, dtype), qe.KVCache(model, n + 4, dtype)
+    got, ref = model.prefill_batch(ids, 0, a, chunk=2048), model.prefill(ids, 0, b)
+    # 16-bit mantissas in the products against f32 ones, as the other chunk tests; a bf16 cache's
+    # rows next to a rounding boundary fall to either side (2^-8 of a value, averaged over n keys)
+    tol = 1e-3 if kv == "f32" else 1e-2
+    assert np.max(np.abs(got - ref)) < tol
+    for i in range(2):  # the K/V rows of every position are what the next steps attend to
+        d = np.max(np.abs(model.forward(int(ids[i]), n + i, a) - model.forward(int(ids[i]), n + i, b)))
+        assert d < tol, f"step {i}: {d}"
