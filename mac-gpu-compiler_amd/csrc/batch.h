@@ -132,10 +132,11 @@ hipError_t launch_qk_rope(const BatchAttnParams& p, hipStream_t st);
 // v rows (k normalized and rotated) appended to the cache at positions a.start + m.
 hipError_t launch_gemm_qk_rope(const GemmParams& g, const BatchAttnParams& a, hipStream_t st);
 // causal attention of a chunk over `runs` (1..kBatchMaxRuns) key runs, merged into att; p.pf:
-// weights the launch also loads into L2 (whole planes of workgroups after the runs')
-hipError_t launch_attn_causal(const BatchAttnParams& p, uint32_t runs, hipStream_t st);
-// key runs for a chunk of M tokens at positions start.. : at least 4, more while the chunk has
-// under 512 workgroups, and at most one per 128 keys
+// weights the launch also loads into L2 (whole planes of workgroups after the runs'). rope: q, k and
+// v are the raw rows of p.qkv; the launch normalizes and rotates them and appends K/V (k_qk_rope's work)
+hipError_t launch_attn_causal(const BatchAttnParams& p, bool rope, uint32_t runs, hipStream_t st);
+// key runs for a chunk of M tokens at positions start.. : what fits one workgroup per CU, at most one
+// per 128 keys (64 for short passes)
 uint32_t attn_causal_runs(uint32_t M, uint32_t start, uint32_t n_heads, uint32_t n_kv);
 // tokens[r] = greedy token of row r of logits [rows][V] (the decode step's argmax rule);
 // cand: rows * kArgParts candidates of scratch (device memory); rows <= 65535; err_in / err_out

@@ -116,28 +116,37 @@ __global__ __launch_bounds__(256) void k_qk_rope(BatchAttnParams p) {
 // in LDS), and each product keeps the hi*hi, hi*lo and lo*hi terms (lo*lo is below 2^-16 of the
 // product); a bf16 cache is exact in hi, so its tiles take two terms.
 // Workgroup (KV head g, block of TOK = 64 RB / G tokens, key run s) serves 64 RB query rows,
-// row r = token mb + r / G of head g G + r % G; wave w owns RB blocks of 16 rows (rows 16 (RB w
-// + b) .. + 15) and lane l the row l % 16 of each. Keys come in LDS tiles of 64 positions (the
-// next tile's K is loaded into registers during this tile's scores, its V during P V), and every fragment a wave reads
-// from LDS feeds the MFMAs of all its RB row blocks. Per tile a wave computes the transposed
-// scores S^T[key][row] (A = K rows: lane has key 16 j + l % 16, dims 32 s + 8 kg .. +7 with
-// kg = l / 16; B = q of row l % 16, same dims). In the 16 x 16 output layout a lane then holds
-// keys 16 j + 4 kg + r (j, r < 4) of its own row, so the online softmax (max, rescale, sum)
-// stays in the lane plus two shuffles across kg, with no LDS round trip for P. Next
-// O^T[d][row] += V^T P^T, with the k index of a 32-key step mapped so that lane kg's eight B
-// values are its own probabilities for keys 4 kg + r and 16 + 4 kg + r (r < 4); the A side
-// reads those keys from a transposed V tile whose key slots are permuted to match (Vt[d][slot],
-// key 32 s + 16 h + 4 kg + r in slot 32 s + 8 kg + 4 h + r), so a lane's eight keys are one
-// 16-byte read, and O^T's column is again the lane's row. Rows with no visible key in the run keep m = -inf,
-// l = 0. One run: normalized output to att [M][n_heads][128]; several: (m, l, acc) partials to
-// part [M][n_heads][runs][kPartStride], combined by k_attn_merge_rows.
+// row r = token mb + r / G of head g G + r % G, with eight waves: wave w owns RB blocks of 16 rows
+// (rows 16 (RB (w % 4) + b) .. + 15), lane l the row l % 16 of each, and the keys of half w / 4 of
+// every tile; the two halves' sums meet in LDS at the end. Keys come in LDS tiles of 64 positions,
+// and every fragment a wave reads from LDS feeds the MFMAs of all its RB row blocks. Per tile a wave
+// computes the transposed scores S^T[key][row] of its 32 keys (A = K rows: lane has key 16 j + l %
+// 16, dims 32 s + 8 kg .. +7 with kg = l / 16; B = q of row l % 16, same dims). In the 16 x 16 output
+// layout a lane then holds keys 16 j + 4 kg + r (j < 2, r < 4) of its own row, so the online softmax
+// stays in the lane plus two shuffles across kg, with no LDS round trip for P. Next O^T[d][row] +=
+// V^T P^T, with the k index mapped so that lane kg's eight B values are its own probabilities for
+// keys 4 kg + r and 16 + 4 kg + r (r < 4); the A side reads those keys from a transposed V tile whose
+// key slots are permuted to match (Vt[d][slot], key 32 s + 16 h + 4 kg + r in slot 32 s + 8 kg + 4 h +
+// r), so a lane's eight keys are one 16-byte read, and O^T's column is again the lane's row. Rows with
+// no visible key in the run keep m = -inf, l = 0. One run: normalized output to att [M][n_heads][128];
+// several: (m, l, acc) partials to part [M][n_heads][runs][kPartStride], combined by
+// k_attn_merge_rows.
+// ROPE (short passes): q, k and v are the raw projections in qkv; the workgroup applies the q/k
+// RMSNorm and RoPE to the rows it reads and appends the pass's K/V rows, so that no launch of its own
+// has to.
+// Bound: per SIMD and tile 96 MFMAs (1536 clocks) a wave beside ~230 VALU instructions (920); with
+// both waves of a SIMD in one phase they add up (3.7 us per tile of 128 rows), a phase apart they
+// overlap (2.9 us; four waves of all 64 keys, staged between two barriers, took 5). 512 rows at
+// position 1536: 46 -> 34 us.
 // ---------------------------------------------------------------------------------------------
-template <int G, bool KV_BF16, int RB>
-__global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
+template <int G, bool KV_BF16, int RB, bool ROPE>
+__global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
   constexpr int D = kHeadDim, BK = 64, TOK = 64 * RB / G, KP = D + 8, VP = BK + 8, NL = KV_BF16 ? 1 : 2;
-  __shared__ __align__(16) uint16_t ks[NL][BK][KP];  // [hi, lo][key][dim]
-  __shared__ __align__(16) uint16_t vt[NL][D][VP];   // [hi, lo][dim][key slot]
+  constexpr int KS = NL * BK * KP, TILE = KS + NL * D * VP;        // u16s: K [hi, lo][key][dim], V [hi, lo][dim][key slot]
+  constexpr int MERGE = 4 * RB * (8 * 64 * 8 + 16 * 4);            // ... of the halves' merge
+  __shared__ __align__(16) uint16_t smem[2 * TILE > MERGE ? 2 * TILE : MERGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
+  const int rw = wave & 3, kh = wave >> 2;
   const uint32_t g = blockIdx.x, mb = blockIdx.y * TOK, run = blockIdx.z, runs = p.runs;
   if (run >= runs) {  // a prefetch workgroup (whole workgroup, before any load)
     l2_prefetch_tiles(p.pf.pf, (run - runs) * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + g,
@@ -147,7 +156,7 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
   uint32_t tok[RB], head[RB], my_pos[RB];
 #pragma unroll
   for (int b = 0; b < RB; b++) {
-    const uint32_t row = uint32_t(wave * RB + b) * 16 + uint32_t(li);
+    const uint32_t row = uint32_t(rw * RB + b) * 16 + uint32_t(li);
     tok[b] = mb + row / G;
     head[b] = g * G + row % G;
     my_pos[b] = p.start + min(tok[b], p.M - 1);
@@ -155,52 +164,59 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
   const uint32_t last = p.start + min(mb + TOK - 1, p.M - 1);  // positions 0..last are needed
   const uint32_t k_begin = run * p.key_run;
   const uint32_t k_end = min(last + 1, k_begin + p.key_run);  // this run: positions [k_begin, k_end)
-  // scores in base-2 units: softmax weights are 2^(s log2(e) scale - m), m and the partials' m
-  // in the same units
+  // scores in base-2 units (q carries the factor): softmax weights are 2^(s - m), the partials' m in
+  // the same units
   const float sl2 = p.scale * 1.44269504088896341f;
 
-  bf16x8 qh[RB][4], ql[RB][4];
+  const uint32_t heads = ROPE ? p.n_heads + 2 * p.n_kv : p.n_heads;  // heads of a token's row of q
+  float4 qv[RB][4][2];
 #pragma unroll
   for (int b = 0; b < RB; b++) {
-    const float* qp = p.q + (size_t(min(tok[b], p.M - 1)) * p.n_heads + head[b]) * D + 8 * kg;
+    const float* qp = (ROPE ? p.qkv : p.q) + (size_t(min(tok[b], p.M - 1)) * heads + head[b]) * D + 8 * kg;
 #pragma unroll
     for (int st = 0; st < 4; st++) {
-      const float4 x = *reinterpret_cast<const float4*>(qp + 32 * st);
-      const float4 y = *reinterpret_cast<const float4*>(qp + 32 * st + 4);
-      const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-      split8(v, qh[b][st], ql[b][st]);
+      qv[b][st][0] = *reinterpret_cast<const float4*>(qp + 32 * st);
+      qv[b][st][1] = *reinterpret_cast<const float4*>(qp + 32 * st + 4);
     }
   }
-  f32x4 o[RB][8];
-  float m_run[RB], l_run[RB];
+  float4 q_rope[RB][2][4];  // ROPE: (cos, sin) of dims 32 st + 8 kg .. + 7 and the gains
+  uint4 q_gain[4];
+  if constexpr (ROPE) {
 #pragma unroll
-  for (int b = 0; b < RB; b++) {
+    for (int st = 0; st < 4; st++) q_gain[st] = *reinterpret_cast<const uint4*>(p.q_norm + 32 * st + 8 * kg);
 #pragma unroll
-    for (int i = 0; i < 8; i++) o[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m_run[b] = -INFINITY;
-    l_run[b] = 0.f;
+    for (int b = 0; b < RB; b++)
+#pragma unroll
+      for (int st = 0; st < 2; st++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+          q_rope[b][st][c] =
+              *reinterpret_cast<const float4*>(p.rope + size_t(my_pos[b]) * D + 2 * (32 * st + 8 * kg) + 4 * c);
   }
 
-  // staging: K rows lr + 8 i (i < 8) at dims ld .. ld + 3 (coalesced rows); V key pair
-  // 2 vk, 2 vk + 1 at dims 4 vb + 32 i .. +3 (i < 4), so that Vt gets (key, key + 1) words
+  // staging: K rows lr + 16 i (i < 4) at dims ld .. ld + 3; V key pair 2 vk, 2 vk + 1 at dims
+  // vd + 64 i .. +3 (i < 2), so that Vt gets (key, key + 1) words; 8 lanes on one row
   const size_t hbase = size_t(g) * p.max_seq * D;
-  const int lr = tid >> 5, ld = (tid & 31) * 4, vk = tid & 31, vb = tid >> 5;
+  const int lr = tid >> 5, ld = (tid & 31) * 4, vk = (tid >> 3) & 31, vd = 4 * (tid & 7) + 32 * (tid >> 8);
   // Vt slot of keys 2 vk, 2 vk + 1 (adjacent slots): key 32 s + 16 h + 4 c + r -> 32 s + 8 c + 4 h + r
   const int vslot = (2 * vk & 32) | ((2 * vk >> 2) & 3) << 3 | ((2 * vk >> 4) & 1) << 2 | (2 * vk & 3);
   using Pre = typename std::conditional<KV_BF16, uint2, float4>::type;
-  Pre kp[8], vp[8];
+  Pre kp[4], vp[4];
+  auto k_row = [&](int i) __attribute__((always_inline)) { return uint32_t(lr + 16 * i); };
+  auto v_row = [&](int i) __attribute__((always_inline)) { return uint32_t(2 * vk + (i & 1)); };
+  auto v_dim = [&](int i) __attribute__((always_inline)) { return vd + 64 * (i >> 1); };
   auto load_k = [&](uint32_t t0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const size_t ko = hbase + size_t(min(t0 + uint32_t(lr + 8 * i), k_end - 1)) * D + ld;
+    for (int i = 0; i < 4; i++) {
+      const size_t ko = hbase + size_t(min(t0 + k_row(i), k_end - 1)) * D + ld;
       if constexpr (KV_BF16) kp[i] = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.k_cache) + ko);
       else kp[i] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.k_cache) + ko);
     }
   };
   auto load_v = [&](uint32_t t0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const size_t vo = hbase + size_t(min(t0 + uint32_t(2 * vk + (i & 1)), k_end - 1)) * D + 4 * vb + 32 * (i >> 1);
+    for (int i = 0; i < 4; i++) {
+      const size_t vo = hbase + size_t(min(t0 + v_row(i), k_end - 1)) * D + v_dim(i);
       if constexpr (KV_BF16) vp[i] = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p.v_cache) + vo);
       else vp[i] = *reinterpret_cast<const float4*>(static_cast<const float*>(p.v_cache) + vo);
     }
@@ -210,150 +226,311 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
   auto pk = [](float x, float y) __attribute__((always_inline)) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), bf16x2));
   };
-  auto store_k = [&]() __attribute__((always_inline)) {
+  auto store_k = [&](uint16_t* ks) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < 4; i++) {
+      uint16_t* at = ks + k_row(i) * KP + ld;
       if constexpr (KV_BF16) {
-        *reinterpret_cast<uint2*>(&ks[0][lr + 8 * i][ld]) = kp[i];
+        *reinterpret_cast<uint2*>(at) = kp[i];
       } else {
         const float4 v = kp[i];
         const uint32_t h0 = pk(v.x, v.y), h1 = pk(v.z, v.w);
-        *reinterpret_cast<uint2*>(&ks[0][lr + 8 * i][ld]) = make_uint2(h0, h1);
-        *reinterpret_cast<uint2*>(&ks[NL - 1][lr + 8 * i][ld]) =
+        *reinterpret_cast<uint2*>(at) = make_uint2(h0, h1);
+        *reinterpret_cast<uint2*>(at + BK * KP) =
             make_uint2(pk(v.x - __uint_as_float(h0 << 16), v.y - __uint_as_float(h0 & 0xFFFF0000u)),
                        pk(v.z - __uint_as_float(h1 << 16), v.w - __uint_as_float(h1 & 0xFFFF0000u)));
       }
     }
   };
-  auto store_v = [&]() __attribute__((always_inline)) {
+  auto store_v = [&](uint16_t* vt) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) {  // vp[i]: key 2 vk, vp[i + 1]: key 2 vk + 1, dims 4 vb + 16 i ..
-      const int d0 = 4 * vb + 16 * i;
+    for (int i = 0; i < 4; i += 2) {  // vp[i]: key 2 vk, vp[i + 1]: key 2 vk + 1
+      uint16_t* at = vt + v_dim(i) * VP + vslot;
       if constexpr (KV_BF16) {
         const uint2 x = vp[i], y = vp[i + 1];
         const uint32_t w[4] = {(x.x & 0xFFFFu) | (y.x << 16), (x.x >> 16) | (y.x & 0xFFFF0000u),
                                (x.y & 0xFFFFu) | (y.y << 16), (x.y >> 16) | (y.y & 0xFFFF0000u)};
 #pragma unroll
-        for (int c = 0; c < 4; c++) *reinterpret_cast<uint32_t*>(&vt[0][d0 + c][vslot]) = w[c];
+        for (int c = 0; c < 4; c++) *reinterpret_cast<uint32_t*>(at + c * VP) = w[c];
       } else {
         const float x[4] = {vp[i].x, vp[i].y, vp[i].z, vp[i].w};
         const float y[4] = {vp[i + 1].x, vp[i + 1].y, vp[i + 1].z, vp[i + 1].w};
 #pragma unroll
         for (int c = 0; c < 4; c++) {
           const uint32_t h = pk(x[c], y[c]);
-          *reinterpret_cast<uint32_t*>(&vt[0][d0 + c][vslot]) = h;
-          *reinterpret_cast<uint32_t*>(&vt[NL - 1][d0 + c][vslot]) =
+          *reinterpret_cast<uint32_t*>(at + c * VP) = h;
+          *reinterpret_cast<uint32_t*>(at + (D + c) * VP) =
               pk(x[c] - __uint_as_float(h << 16), y[c] - __uint_as_float(h & 0xFFFF0000u));
         }
       }
     }
   };
-  // K and V of the next tile are staged apart, each into its LDS tile as soon as the current
-  // tile's last read of it is done (after the scores; after P V), so only one of them is held in
-  // registers at a time (-5% against both held across the whole tile)
+  // ROPE: the rows of this pass's own tokens come from its raw projections instead of the cache: k
+  // normalized and rotated (a row sits in 32 lanes, its dims d and d + 64 in lanes 16 apart), in the
+  // cache's type, and appended to the cache by the last token block, which sees all of them. All
+  // loads come before the first use: one latency, not one per row.
+  const bool append = ROPE && blockIdx.y == gridDim.y - 1;
+  auto has_new = [&](uint32_t t0) __attribute__((always_inline)) {
+    return ROPE && t0 + BK > p.start && k_end > p.start;
+  };
+  auto new_pos = [&](uint32_t t) __attribute__((always_inline)) { return max(min(t, k_end - 1), p.start); };
+  auto to_cache = [&](float4 x) __attribute__((always_inline)) {
+    if constexpr (KV_BF16)
+      return make_uint2(f32_to_bf16(x.x) | uint32_t(f32_to_bf16(x.y)) << 16,
+                        f32_to_bf16(x.z) | uint32_t(f32_to_bf16(x.w)) << 16);
+    else return x;
+  };
+  auto pick = [](bool c, Pre x, Pre y) __attribute__((always_inline)) {  // component-wise (see k_gemm_wide's end)
+    if constexpr (KV_BF16) return make_uint2(c ? x.x : y.x, c ? x.y : y.y);
+    else return make_float4(c ? x.x : y.x, c ? x.y : y.y, c ? x.z : y.z, c ? x.w : y.w);
+  };
+  auto put = [&](void* cache, uint32_t t, int d, Pre x) __attribute__((always_inline)) {
+    if (!append || t < p.start || t >= k_end) return;
+    const size_t slot = hbase + size_t(t) * D + d;
+    if constexpr (KV_BF16) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(cache) + slot) = x;
+    else *reinterpret_cast<float4*>(static_cast<float*>(cache) + slot) = x;
+  };
+  float4 x[4], r0[4], r1[4], y[4];  // k, (cos, sin) of its four dims, v
+  uint2 gn;
+  auto load_new = [&](uint32_t t0) __attribute__((always_inline)) {
+    if (!has_new(t0)) return;
+    gn = *reinterpret_cast<const uint2*>(p.k_norm + ld);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t tk = new_pos(t0 + k_row(i)), tv = new_pos(t0 + v_row(i));
+      x[i] = *reinterpret_cast<const float4*>(p.qkv + (size_t(tk - p.start) * heads + p.n_heads + g) * D + ld);
+      const float4* rp = reinterpret_cast<const float4*>(p.rope + size_t(tk) * D + 2 * (ld & 63));
+      r0[i] = rp[0];
+      r1[i] = rp[1];
+      y[i] = *reinterpret_cast<const float4*>(p.qkv + (size_t(tv - p.start) * heads + p.n_heads + p.n_kv + g) * D +
+                                              v_dim(i));
+    }
+  };
+  auto apply_new = [&](uint32_t t0) __attribute__((always_inline)) {
+    if (!has_new(t0)) return;
+    float ss[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) ss[i] = (x[i].x * x[i].x + x[i].y * x[i].y) + (x[i].z * x[i].z + x[i].w * x[i].w);
+#pragma unroll
+    for (int m = 1; m < 32; m <<= 1)
+#pragma unroll
+      for (int i = 0; i < 4; i++) ss[i] += __shfl_xor(ss[i], m);
+    const float s = ld < 64 ? -1.f : 1.f;  // a cos - b sin, b cos + a sin
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float sc = 1.0f / sqrtf(ss[i] / float(D) + p.eps);
+      const float4 v =
+          make_float4(x[i].x * sc * __uint_as_float(gn.x << 16), x[i].y * sc * __uint_as_float(gn.x & 0xFFFF0000u),
+                      x[i].z * sc * __uint_as_float(gn.y << 16), x[i].w * sc * __uint_as_float(gn.y & 0xFFFF0000u));
+      const float4 w = make_float4(s * __shfl_xor(v.x, 16), s * __shfl_xor(v.y, 16), s * __shfl_xor(v.z, 16),
+                                   s * __shfl_xor(v.w, 16));
+      const Pre nk = to_cache(make_float4(v.x * r0[i].x + w.x * r0[i].y, v.y * r0[i].z + w.y * r0[i].w,
+                                          v.z * r1[i].x + w.z * r1[i].y, v.w * r1[i].z + w.w * r1[i].w));
+      const Pre nv = to_cache(y[i]);
+      // (rows past k_end hold row k_end - 1, which may be a new one: finite either way)
+      kp[i] = pick(min(t0 + k_row(i), k_end - 1) >= p.start, nk, kp[i]);
+      vp[i] = pick(min(t0 + v_row(i), k_end - 1) >= p.start, nv, vp[i]);
+      put(p.k_cache, t0 + k_row(i), ld, nk);
+      put(p.v_cache, t0 + v_row(i), v_dim(i), nv);
+    }
+  };
+  // the first tile's K and V are in flight before q is used: a short pass's runs are one tile, and
+  // its time is these loads' latency
   if (k_begin < k_end) {
     load_k(k_begin);
-    store_k();
     load_v(k_begin);
-    store_v();
+    load_new(k_begin);
   }
+  __builtin_amdgcn_sched_barrier(0);
+  bf16x8 qh[RB][4], ql[RB][4];
+  f32x4 o[RB][8];
+  float m_run[RB], l_run[RB];
+#pragma unroll
+  for (int b = 0; b < RB; b++) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) o[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[b] = -INFINITY;
+    l_run[b] = 0.f;
+    float v[4][8];
+#pragma unroll
+    for (int st = 0; st < 4; st++) {
+      const float4 x = qv[b][st][0], y = qv[b][st][1];
+      const float u[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[st][e] = u[e];
+    }
+    if constexpr (ROPE) {  // q RMSNorm + RoPE (cpu_inference.rs:134-141): dims d, d + 64 in one lane
+      float ss = 0.f;
+#pragma unroll
+      for (int st = 0; st < 4; st++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) ss += v[st][e] * v[st][e];
+      ss += __shfl_xor(ss, 16);
+      ss += __shfl_xor(ss, 32);
+      const float sc = 1.0f / sqrtf(ss / float(D) + p.eps);
+#pragma unroll
+      for (int st = 0; st < 2; st++) {
+        const uint32_t ga[4] = {q_gain[st].x, q_gain[st].y, q_gain[st].z, q_gain[st].w};
+        const uint32_t gb[4] = {q_gain[st + 2].x, q_gain[st + 2].y, q_gain[st + 2].z, q_gain[st + 2].w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float a = v[st][e] * sc * __uint_as_float(e & 1 ? ga[e / 2] & 0xFFFF0000u : ga[e / 2] << 16);
+          const float c = v[st + 2][e] * sc * __uint_as_float(e & 1 ? gb[e / 2] & 0xFFFF0000u : gb[e / 2] << 16);
+          const float4 r = q_rope[b][st][e / 2];
+          const float cs = e & 1 ? r.z : r.x, sn = e & 1 ? r.w : r.y;
+          v[st][e] = a * cs - c * sn;
+          v[st + 2][e] = c * cs + a * sn;
+        }
+      }
+    }
+#pragma unroll
+    for (int st = 0; st < 4; st++) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[st][e] *= sl2;
+      split8(v[st], qh[b][st], ql[b][st]);
+    }
+  }
+  auto load_tile = [&](uint32_t t0) __attribute__((always_inline)) {
+    if (t0 >= k_end) return;
+    load_k(t0);
+    load_v(t0);
+  };
+  auto store_tile = [&](uint16_t* at) __attribute__((always_inline)) {
+    store_k(at);
+    store_v(at + KS);
+  };
+  if (k_begin < k_end) {
+    apply_new(k_begin);
+    store_tile(smem);
+  }
+  load_tile(k_begin + BK);
+  // Two LDS tiles, one barrier per tile: the next tile waits in registers and goes to the other LDS
+  // tile before this one's products in the waves of key half 1, after them in those of key half 0.
+  // The two waves of a SIMD are so in different phases: one's MFMAs run beside the other's staging
+  // and softmax.
+  uint32_t cur = 0;
   for (uint32_t t0 = k_begin; t0 < k_end; t0 += BK) {
     const bool more = t0 + BK < k_end;
-    __syncthreads();  // K and V of this tile are in LDS
-    if (more) load_k(t0 + BK);
+    __syncthreads();  // this tile is in LDS; every wave is done with the other one
+    auto stage = [&]() __attribute__((always_inline)) {
+      load_new(t0 + BK);
+      apply_new(t0 + BK);
+      store_tile(smem + (cur ^ 1) * TILE);
+      load_tile(t0 + 2 * BK);
+    };
+    if (kh == 1 && more) stage();
+    const uint16_t* ks = smem + cur * TILE + 32 * kh * KP;
+    const uint16_t* vt = smem + cur * TILE + KS + 32 * kh;
 
-    f32x4 s[RB][4];
+    f32x4 s[RB][2];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < 2; j++) {
 #pragma unroll
       for (int b = 0; b < RB; b++) s[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int st = 0; st < 4; st++) {
-        const bf16x8 kh = *reinterpret_cast<const bf16x8*>(&ks[0][16 * j + li][32 * st + 8 * kg]);
-        bf16x8 kl;
-        if constexpr (!KV_BF16) kl = *reinterpret_cast<const bf16x8*>(&ks[NL - 1][16 * j + li][32 * st + 8 * kg]);
+        const uint16_t* at = ks + (16 * j + li) * KP + 32 * st + 8 * kg;
+        const bf16x8 hi = *reinterpret_cast<const bf16x8*>(at);
+        bf16x8 lo;
+        if constexpr (!KV_BF16) lo = *reinterpret_cast<const bf16x8*>(at + BK * KP);
 #pragma unroll
-        for (int b = 0; b < RB; b++) {
-          s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh[b][st], s[b][j], 0, 0, 0);
-          s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql[b][st], s[b][j], 0, 0, 0);
-          if constexpr (!KV_BF16) s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh[b][st], s[b][j], 0, 0, 0);
+        for (int b = 0; b < RB; b++) s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, qh[b][st], s[b][j], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < RB; b++) s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, ql[b][st], s[b][j], 0, 0, 0);
+        if constexpr (!KV_BF16) {
+#pragma unroll
+          for (int b = 0; b < RB; b++)
+            s[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, qh[b][st], s[b][j], 0, 0, 0);
         }
       }
     }
-    bf16x8 ph[RB][2], pl[RB][2];
+    // every key of the tile is visible to every row
+    const bool all_seen = t0 + BK <= k_end && t0 + BK <= p.start + mb + 1;
+    bf16x8 ph[RB], pl[RB];
 #pragma unroll
     for (int b = 0; b < RB; b++) {
-      float mx = -INFINITY;
+      if (!all_seen) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < 2; j++) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const uint32_t t = t0 + uint32_t(16 * j + 4 * kg + r);
-          const float v = t <= my_pos[b] && t < k_end ? s[b][j][r] * sl2 : -INFINITY;
-          s[b][j][r] = v;
-          mx = fmaxf(mx, v);
+          for (int r = 0; r < 4; r++) {
+            const uint32_t t = t0 + uint32_t(32 * kh + 16 * j + 4 * kg + r);
+            s[b][j][r] = t <= my_pos[b] && t < k_end ? s[b][j][r] : -INFINITY;
+          }
         }
       }
+      float mx = s[b][0][0];
+#pragma unroll
+      for (int e = 1; e < 8; e++) mx = fmaxf(mx, s[b][e / 4][e % 4]);
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float m_new = fmaxf(m_run[b], mx);  // -inf while no key of the run is visible to this row
-      // 2^(-inf) = 0 on the hardware exp2: masked keys and a first visible tile weigh 0 with no
-      // test per key; m_use keeps -inf - -inf out while nothing is visible
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float corr = __builtin_amdgcn_exp2f(m_run[b] - m_use);
-      float sum = 0.f;
+      // m only has to keep 2^(s - m) in range: it moves when a row's maximum passes it by 8 (weights up
+      // to 2^8), and the rows are rescaled only then. -inf while no key of the run is visible to the
+      // row; m_use keeps -inf - -inf out, and 2^(-inf) = 0 needs no test per masked key.
+      if (__any(mx > m_run[b] + 8.f)) {
+        const float m_new = mx > m_run[b] + 8.f ? mx : m_run[b];
+        const float corr = __builtin_amdgcn_exp2f(m_run[b] - (m_new == -INFINITY ? 0.f : m_new));
+        l_run[b] *= corr;
+        m_run[b] = m_new;
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float e = __builtin_amdgcn_exp2f(s[b][j][r] - m_use);
-          s[b][j][r] = e;
-          sum += e;
-        }
+        for (int i = 0; i < 8; i++) o[b][i] *= corr;
       }
-      sum += __shfl_xor(sum, 16);
-      sum += __shfl_xor(sum, 32);
-      l_run[b] = l_run[b] * corr + sum;
-      m_run[b] = m_new;
+      const float m_use = m_run[b] == -INFINITY ? 0.f : m_run[b];
+      float pv[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) o[b][i] *= corr;
-#pragma unroll
-      for (int st = 0; st < 2; st++) {
-        const float pv[8] = {s[b][2 * st][0], s[b][2 * st][1], s[b][2 * st][2], s[b][2 * st][3],
-                             s[b][2 * st + 1][0], s[b][2 * st + 1][1], s[b][2 * st + 1][2], s[b][2 * st + 1][3]};
-        split8(pv, ph[b][st], pl[b][st]);
-      }
-    }
-    __syncthreads();  // every wave's reads of ks are done
-    if (more) {
-      store_k();
-      load_v(t0 + BK);
+      for (int e = 0; e < 8; e++) pv[e] = __builtin_amdgcn_exp2f(s[b][e / 4][e % 4] - m_use);
+      l_run[b] += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+      split8(pv, ph[b], pl[b]);
     }
 #pragma unroll
-    for (int st = 0; st < 2; st++) {
+    for (int i = 0; i < 8; i++) {
+      const uint16_t* at = vt + (16 * i + li) * VP + 8 * kg;
+      const bf16x8 hi = *reinterpret_cast<const bf16x8*>(at);
+      bf16x8 lo;
+      if constexpr (!KV_BF16) lo = *reinterpret_cast<const bf16x8*>(at + D * VP);
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const bf16x8 vh = *reinterpret_cast<const bf16x8*>(&vt[0][16 * i + li][32 * st + 8 * kg]);
-        bf16x8 vl;
-        if constexpr (!KV_BF16) vl = *reinterpret_cast<const bf16x8*>(&vt[NL - 1][16 * i + li][32 * st + 8 * kg]);
+      for (int b = 0; b < RB; b++) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, ph[b], o[b][i], 0, 0, 0);
 #pragma unroll
-        for (int b = 0; b < RB; b++) {
-          o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph[b][st], o[b][i], 0, 0, 0);
-          o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pl[b][st], o[b][i], 0, 0, 0);
-          if constexpr (!KV_BF16) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vl, ph[b][st], o[b][i], 0, 0, 0);
-        }
+      for (int b = 0; b < RB; b++) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, pl[b], o[b][i], 0, 0, 0);
+      if constexpr (!KV_BF16) {
+#pragma unroll
+        for (int b = 0; b < RB; b++) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, ph[b], o[b][i], 0, 0, 0);
       }
     }
-    __syncthreads();  // every wave's reads of vt are done
-    if (more) store_v();
+    if (kh == 0 && more) stage();
+    cur ^= 1;
   }
-  // lane holds O^T[16 i + 4 kg + r][row], r < 4
+#pragma unroll
+  for (int b = 0; b < RB; b++) {  // a lane's sum is over its own keys so far
+    l_run[b] += __shfl_xor(l_run[b], 16);
+    l_run[b] += __shfl_xor(l_run[b], 32);
+  }
+  // the two key halves of a row block meet in LDS; lane holds O^T[16 i + 4 kg + r][row], r < 4
+  f32x4* ro = reinterpret_cast<f32x4*>(smem);
+  float2* rml = reinterpret_cast<float2*>(ro + 4 * RB * 8 * 64);
+  __syncthreads();
+  if (kh == 1) {
+#pragma unroll
+    for (int b = 0; b < RB; b++) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) ro[((rw * RB + b) * 8 + i) * 64 + lane] = o[b][i];
+      if (kg == 0) rml[(rw * RB + b) * 16 + li] = make_float2(m_run[b], l_run[b]);
+    }
+  }
+  __syncthreads();
+  if (kh == 1) return;
 #pragma unroll
   for (int b = 0; b < RB; b++) {
     if (tok[b] >= p.M) continue;
+    const float2 ml = rml[(rw * RB + b) * 16 + li];
+    const float m = fmaxf(m_run[b], ml.x), m_use = m == -INFINITY ? 0.f : m;
+    const float e0 = __builtin_amdgcn_exp2f(m_run[b] - m_use), e1 = __builtin_amdgcn_exp2f(ml.x - m_use);
+    const float l = l_run[b] * e0 + ml.y * e1;
+#pragma unroll
+    for (int i = 0; i < 8; i++) o[b][i] = o[b][i] * e0 + ro[((rw * RB + b) * 8 + i) * 64 + lane] * e1;
     const size_t vec = size_t(tok[b]) * p.n_heads + head[b];
     if (runs == 1) {
-      const float inv = 1.0f / l_run[b];
+      const float inv = 1.0f / l;
       float* out = p.att + vec * D;
 #pragma unroll
       for (int i = 0; i < 8; i++) {
@@ -364,12 +541,11 @@ __global__ __launch_bounds__(256) void k_attn_causal_bf(BatchAttnParams p) {
     } else {
       float* out = p.part + (vec * runs + run) * kPartStride;
       if (kg == 0) {
-        out[0] = m_run[b];
-        out[1] = l_run[b];
+        out[0] = m;
+        out[1] = l;
       }
 #pragma unroll
-      for (int i = 0; i < 8; i++)
-        *reinterpret_cast<float4*>(out + 4 + 16 * i + 4 * kg) = make_float4(o[b][i][0], o[b][i][1], o[b][i][2], o[b][i][3]);
+      for (int i = 0; i < 8; i++) *reinterpret_cast<f32x4*>(out + 4 + 16 * i + 4 * kg) = o[b][i];
     }
   }
 }
@@ -1116,12 +1292,24 @@ hipError_t launch_qk_rope(const BatchAttnParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Row blocks per wave of k_attn_causal_bf. One: at 2048 tokens in chunks of 512, two (half the
-// workgroups, each LDS fragment feeding twice the MFMAs) took 15.1 ms against 13.9, and eight
-// waves of one block (twice the LDS reads per tile) 14.6.
-constexpr uint32_t kAttnCausalRB = 1;
+// Row blocks per wave of k_attn_causal_bf: two (each LDS fragment feeds twice the MFMAs, each staged
+// tile twice the rows) once that leaves a workgroup for every second CU. 2048 tokens in one chunk 7.62 ms
+// with two, 7.89 with one; in chunks of 512 9.47 and 9.29; 333 tokens 2.35 and 2.26.
+uint32_t attn_row_blocks(uint32_t M) { return M >= 1024 ? 2 : 1; }
 
-hipError_t launch_attn_causal(const BatchAttnParams& p, uint32_t runs, hipStream_t st) {
+template <int G, int RB>
+hipError_t launch_attn_causal_t(const BatchAttnParams& p, bool rope, dim3 grid, hipStream_t st) {
+  auto* k = p.kv_bf16 ? &k_attn_causal_bf<G, true, RB, false> : &k_attn_causal_bf<G, false, RB, false>;
+  if constexpr (RB == 1) {
+    if (rope) k = p.kv_bf16 ? &k_attn_causal_bf<G, true, RB, true> : &k_attn_causal_bf<G, false, RB, true>;
+  }
+  hipLaunchKernelGGL(k, grid, dim3(512), 0, st, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_attn_causal(const BatchAttnParams& p, bool rope, uint32_t runs, hipStream_t st) {
+  if (rope && (!p.qkv || !p.q_norm || !p.k_norm || !p.rope || uint64_t(p.start) + p.M > p.max_seq))
+    return hipErrorInvalidValue;
   if (!p.n_kv || p.n_heads % p.n_kv || runs == 0 || runs > uint32_t(kBatchMaxRuns) || (runs > 1 && !p.part))
     return hipErrorInvalidValue;
   const uint32_t G = p.n_heads / p.n_kv;
@@ -1132,23 +1320,16 @@ hipError_t launch_attn_causal(const BatchAttnParams& p, uint32_t runs, hipStream
   q.key_run = 64 * per_run;
   q.runs = runs;
   if (q.pf.slots > 64) return hipErrorInvalidValue;
-  constexpr uint32_t RB = kAttnCausalRB;
+  const uint32_t RB = rope ? 1 : attn_row_blocks(p.M);
   const uint32_t gy = ceil_div(p.M, 64 * RB / G);
   // prefetch workgroups: whole planes after the runs' (8 x slots of them at consecutive ids)
   const uint32_t planes = q.pf.slots ? ceil_div(8 * q.pf.slots, p.n_kv * gy) : 0;
   const dim3 grid(p.n_kv, gy, runs + planes);
   hipError_t e = hipErrorInvalidValue;
-#define QE_ATT(GG)                                                                                         \
-  if (G == GG) {                                                                                           \
-    if (p.kv_bf16) hipLaunchKernelGGL((k_attn_causal_bf<GG, true, RB>), grid, dim3(256), 0, st, q);        \
-    else hipLaunchKernelGGL((k_attn_causal_bf<GG, false, RB>), grid, dim3(256), 0, st, q);                 \
-    e = hipGetLastError();                                                                                 \
-  }
-  QE_ATT(1)
-  QE_ATT(2)
-  QE_ATT(4)
-  QE_ATT(8)
-#undef QE_ATT
+  if (G == 1) e = RB == 2 ? launch_attn_causal_t<1, 2>(q, rope, grid, st) : launch_attn_causal_t<1, 1>(q, rope, grid, st);
+  if (G == 2) e = RB == 2 ? launch_attn_causal_t<2, 2>(q, rope, grid, st) : launch_attn_causal_t<2, 1>(q, rope, grid, st);
+  if (G == 4) e = RB == 2 ? launch_attn_causal_t<4, 2>(q, rope, grid, st) : launch_attn_causal_t<4, 1>(q, rope, grid, st);
+  if (G == 8) e = RB == 2 ? launch_attn_causal_t<8, 2>(q, rope, grid, st) : launch_attn_causal_t<8, 1>(q, rope, grid, st);
   if (e != hipSuccess || runs == 1) return e;
   const uint32_t n_vec = p.M * p.n_heads;
   const dim3 mg(ceil_div(n_vec, 8));
@@ -1161,11 +1342,14 @@ hipError_t launch_attn_causal(const BatchAttnParams& p, uint32_t runs, hipStream
 
 uint32_t attn_causal_runs(uint32_t M, uint32_t start, uint32_t n_heads, uint32_t n_kv) {
   if (!M || !n_kv || n_heads % n_kv || n_heads / n_kv > 16) return 1;
-  const uint32_t wgs = n_kv * ceil_div(M, 64 * kAttnCausalRB / (n_heads / n_kv));
-  // at least 4 runs, more while that leaves under 512 workgroups (measured: 4 runs beat 2 and 8
-  // at M = 512 and 1 and 2 at M = 2048); at most kBatchMaxRuns
-  uint32_t runs = std::min(std::max(ceil_div(512, wgs), 4u), uint32_t(kBatchMaxRuns));
-  return std::max(1u, std::min(runs, ceil_div(start + M, 128)));
+  // what fits one workgroup per CU (two f32 tiles are 140 KB of LDS): a second round or more partials
+  // cost more than longer runs (2048 tokens in chunks of 512: 1, 2 and 4 runs 9.68, 9.29, 10.46 ms; in
+  // one chunk of 2048: 1 and 2 runs 7.62, 8.09)
+  const uint32_t wgs = n_kv * ceil_div(M, 64 * attn_row_blocks(M) / (n_heads / n_kv));
+  const uint32_t runs = std::min(std::max(256 / wgs, 1u), uint32_t(kBatchMaxRuns));
+  // a short pass is a few workgroups whose time is one tile's latency after the other: runs of one tile
+  const uint32_t least = M <= kGemmSliceMaxM ? 64 : 128;
+  return std::max(1u, std::min(runs, ceil_div(start + M, least)));
 }
 
 hipError_t launch_row_argmax(const float* logits, uint32_t rows, uint32_t V, uint32_t* tokens, ArgCand* cand,

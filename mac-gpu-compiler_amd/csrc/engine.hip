@@ -1032,24 +1032,28 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
     a.M = M; a.start = start; a.max_seq = uint32_t(kv->max_seq);
     a.n_heads = uint32_t(c.num_attention_heads); a.n_kv = uint32_t(c.num_key_value_heads);
     a.eps = eps; a.scale = 1.0f / sqrtf(float(D)); a.kv_bf16 = kv->dtype == QE_KV_BF16;
+    const uint32_t rows_per_kv = (a.n_heads / a.n_kv) * M;
+    const bool split_attn =
+        m->rows_split_attn && (rows_per_kv == 1 || rows_per_kv == 2 || rows_per_kv == 4 || rows_per_kv == 8);
     // input_layernorm + q|k|v (cpu_inference.rs:129-132); long chunks do the q/k norm, RoPE and K/V
-    // append in the GEMM's epilogue, the others in k_qk_rope
+    // append in the GEMM's epilogue, the others in the attention launch (or k_qk_rope before the
+    // split kernel)
     if (wide) {
       const qe::GemmParams g{bxs, H, nullptr, w.w_qkv, M, QD + 2 * KD, H, bqkv, QD + 2 * KD, eps, 0};
       HIP_TRY(qe::launch_gemm_qk_rope(g, a, s));
     } else {
       if ((rc = gemm(bx, H, w.w_in, w.w_qkv, QD + 2 * KD, H, bqkv, QD + 2 * KD, qe::kGemmStore))) return rc;
-      HIP_TRY(qe::launch_qk_rope(a, s));
+      if (split_attn) HIP_TRY(qe::launch_qk_rope(a, s));
     }
     // multi-stream prefill: the attention reads the previous chunks' K/V rows of this layer,
     // appended on other streams. The event is recorded after this chunk's own wait, so that it
     // stands for the K/V rows of this chunk and of every chunk before it (chunk i waits for
     // chunk i-1 only, whatever the number of streams).
     if (cs && cs->wait_kv) HIP_TRY(hipStreamWaitEvent(s, cs->wait_kv[l], 0));
-    if (cs && cs->kv_done) HIP_TRY(hipEventRecord(cs->kv_done[l], s));
-    const uint32_t rows_per_kv = (a.n_heads / a.n_kv) * M;
+    const bool attn_appends = !wide && !split_attn;  // the attention launch itself appends the K/V rows
+    if (cs && cs->kv_done && !attn_appends) HIP_TRY(hipEventRecord(cs->kv_done[l], s));
     uint32_t merge_splits = 0;  // > 0: o_proj merges this many attention runs in its prologue
-    if (m->rows_split_attn && (rows_per_kv == 1 || rows_per_kv == 2 || rows_per_kv == 4 || rows_per_kv == 8)) {
+    if (split_attn) {
       // few tokens: the split kernel, the q heads of all M tokens of a KV head over one read of
       // its K/V, each token causal (positions up to its own), runs of 64 positions
       AttnParams r{};
@@ -1082,7 +1086,8 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
         a.pf.pf[0] = qe::gemm_prefetch_target(w.w_o, M, H, QD);
         a.pf.slots = qe::tile_prefetch_slots(a.pf.pf, qe::kMaxPrefetch);
       }
-      HIP_TRY(qe::launch_attn_causal(a, qe::attn_causal_runs(M, start, a.n_heads, a.n_kv), s));
+      HIP_TRY(qe::launch_attn_causal(a, attn_appends, qe::attn_causal_runs(M, start, a.n_heads, a.n_kv), s));
+      if (cs && cs->kv_done && attn_appends) HIP_TRY(hipEventRecord(cs->kv_done[l], s));
     }
     // o_proj + residual (cpu_inference.rs:163-164)
     if (merge_splits) {
