@@ -144,7 +144,8 @@ __global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
   constexpr int D = kHeadDim, BK = 64, TOK = 64 * RB / G, KP = D + 8, VP = BK + 8, NL = KV_BF16 ? 1 : 2;
   constexpr int KS = NL * BK * KP, TILE = KS + NL * D * VP;        // u16s: K [hi, lo][key][dim], V [hi, lo][dim][key slot]
   constexpr int MERGE = 4 * RB * (8 * 64 * 8 + 16 * 4);            // ... of the halves' merge
-  __shared__ __align__(16) uint16_t smem[2 * TILE > MERGE ? 2 * TILE : MERGE];
+  constexpr int NB = ROPE ? 1 : 2;                                 // LDS tiles
+  __shared__ __align__(16) uint16_t smem[NB * TILE > MERGE ? NB * TILE : MERGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
   const int rw = wave & 3, kh = wave >> 2;
   const uint32_t g = blockIdx.x, mb = blockIdx.y * TOK, run = blockIdx.z, runs = p.runs;
@@ -415,10 +416,10 @@ __global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
     auto stage = [&]() __attribute__((always_inline)) {
       load_new(t0 + BK);
       apply_new(t0 + BK);
-      store_tile(smem + (cur ^ 1) * TILE);
+      store_tile(smem + (NB == 2 ? cur ^ 1 : 0) * TILE);
       load_tile(t0 + 2 * BK);
     };
-    if (kh == 1 && more) stage();
+    if (NB == 2 && kh == 1 && more) stage();
     const uint16_t* ks = smem + cur * TILE + 32 * kh * KP;
     const uint16_t* vt = smem + cur * TILE + KS + 32 * kh;
 
@@ -497,8 +498,9 @@ __global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
         for (int b = 0; b < RB; b++) o[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, ph[b], o[b][i], 0, 0, 0);
       }
     }
-    if (kh == 0 && more) stage();
-    cur ^= 1;
+    if (NB == 1) __syncthreads();  // every wave is done with this tile
+    if ((NB == 1 || kh == 0) && more) stage();
+    if (NB == 2) cur ^= 1;
   }
 #pragma unroll
   for (int b = 0; b < RB; b++) {  // a lane's sum is over its own keys so far
@@ -1129,10 +1131,14 @@ namespace {
 // its loads, worth about 60 KB of them. Measured (us, M x N x K): 9 x 6144 x 1024 on 16 x 32 tiles
 // 3.5, 16 x 48 4.0; 64 x 6144 x 1024 on 32 x 48 5.8, 32 x 64 6.0, 16 x 32 7.3; 130 x 1024 x 3072 on
 // 32 x 32 7.5, 32 x 64 9.0, 16 x 32 9.5; 130 x 4096 x 1024 on 48 x 64 7.3, 64 x 64 7.9, 32 x 64 10.1;
-// 512 x 1024 x 3072 on 32 x 64 15.1, 48 x 64 17.6, 64 x 64 20.4.
+// 512 x 1024 x 3072 on 32 x 64 15.1, 48 x 64 17.6, 64 x 64 20.4. N = 151936, K = 1024 (an lm_head): 5 rows
+// on 16 x 128 54.7, 64 x 128 76.5; 12 rows 56.6 and 77.9; 24 rows on 32 x 128 67.1, 64 x 128 79.7; 40 rows on
+// 48 x 128 80.7, 64 x 128 84.8. Deeper rings (all of a wave's steps in flight) were slower: down of 5 rows
+// 7.3 against 6.2 traced.
 uint64_t tile_cost(const GemmParams& p, uint32_t bm, uint32_t bn) {
   const uint64_t wgs = (uint64_t(p.M) + bm - 1) / bm * ((uint64_t(p.N) + bn - 1) / bn);
-  return (wgs + 255) / 256 * (uint64_t(4 * bm + 2 * bn) * p.K + 60 * 1024);
+  const uint32_t rows = bm == 16 && p.M <= 8 ? 8 : bm;  // (HALF)
+  return (wgs + 255) / 256 * (uint64_t(4 * rows + 2 * bn) * p.K + 60 * 1024);
 }
 
 hipError_t check_grid(uint64_t wgs, uint32_t threads) {
@@ -1143,16 +1149,24 @@ template <bool NORM, int EPI, int MT, int NT, int NW, int NS>
 hipError_t launch_kslice_t(const GemmParams& p, hipStream_t st) {
   const uint64_t wgs = (uint64_t(p.M) + 16 * MT - 1) / (16 * MT) * ((uint64_t(p.N) + 16 * NT - 1) / (16 * NT));
   if (hipError_t e = check_grid(wgs, 64 * NW)) return e;
-  hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
+  if constexpr (MT == 1) {
+    if (p.M <= 8) {
+      hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, true>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, false>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
   return hipGetLastError();
 }
 
 template <bool NORM, int EPI>
 hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
   if (NORM && p.K > uint32_t(kGemmNormMaxK)) return hipErrorInvalidValue;
-  const uint32_t tile[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64}, {48, 64}, {64, 64}, {64, 128}};
+  // (the last four: many columns, as an lm_head's, where a wide tile has fewer bytes of A beside its W)
+  const uint32_t tile[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64},  {48, 64},
+                              {64, 64}, {16, 128}, {32, 128}, {48, 128}, {64, 128}};
   int best = 0;
-  for (int i = 1; i < 8; i++)
+  for (int i = 1; i < 11; i++)
     if (tile_cost(p, tile[i][0], tile[i][1]) < tile_cost(p, tile[best][0], tile[best][1])) best = i;
   switch (best) {
     case 0: return launch_kslice_t<NORM, EPI, 1, 1, 8, 4>(p, st);
@@ -1162,6 +1176,9 @@ hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
     case 4: return launch_kslice_t<NORM, EPI, 2, 4, 8, 2>(p, st);
     case 5: return launch_kslice_t<NORM, EPI, 3, 4, 8, 1>(p, st);
     case 6: return launch_kslice_t<NORM, EPI, 4, 4, 8, 1>(p, st);
+    case 7: return launch_kslice_t<NORM, EPI, 1, 8, 4, 2>(p, st);
+    case 8: return launch_kslice_t<NORM, EPI, 2, 8, 4, 2>(p, st);
+    case 9: return launch_kslice_t<NORM, EPI, 3, 8, 4, 2>(p, st);
     default: return launch_kslice_t<NORM, EPI, 4, 8, 4, 2>(p, st);
   }
 }

@@ -997,9 +997,10 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   const bool mv = m->mv_rows && M <= qe::kMvRowsMaxM;
   auto gemm = [&](const float* A, uint32_t lda, const uint16_t* gain, const uint16_t* W, uint32_t N, uint32_t K,
                   float* C, uint32_t ldc, int epi) -> int {
-    // gate|up (the widest projection) at 4 rows is faster on the k-sliced GEMM: 1.405 vs 1.431 ms
-    // per k = 4 verify (at 3 rows the matvec still wins)
-    if (mv && lda == K && W != m->lm_head && !(epi == qe::kGemmSiluPair && M >= 4)) {
+    // q|k|v and gate|up (many rows of W, few columns) are faster on the k-sliced GEMM from 3 rows: 1.324
+    // ms vs 1.366 per k = 4 verify at 2048, 1.164 vs 1.200 at 3 rows and 700; o_proj and down are not
+    // (1.448 at 4 rows)
+    if (mv && lda == K && W != m->lm_head && !(gain && M >= 3)) {
       qe::MvRowsParams r{W, A, gain, C, M, N, K, ldc, eps};
       HIP_TRY(qe::launch_mv_rows(r, gain != nullptr, epi, s));
       return QE_OK;
@@ -1066,9 +1067,9 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       if (rows_per_kv == 8) r.row_split = 2;
       if (m->l2_prefetch && mv) {
         // as in the decode step: the attention is latency-bound, so extra workgroups load this
-        // layer's gate|up (the k-sliced GEMM's rows at 4 tokens, else the multi-row matvec's) and
+        // layer's gate|up (up to 2 tokens: as the multi-row matvec reads it) and
         // down weights into the L2 of the XCDs that will read them
-        if (M < 4) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
+        if (M < 3) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
         r.pf[1] = qe::l2_prefetch_target(w.w_down, H, I, qe::kCopy, qe::kResAdd);
         r.pf_slots = qe::l2_prefetch_slots(r.pf, qe::kMaxPrefetch);
       }

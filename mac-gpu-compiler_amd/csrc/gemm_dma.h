@@ -130,14 +130,17 @@ __device__ __forceinline__ void emit4(const GemmParams& p, uint32_t m, uint32_t 
 // NORM: A' = A x gain[k], C scaled by s[m] = 1 / sqrt(mean_k A^2 + eps), the squares summed over
 // the same slices (s applied after the sum, a reassociation of the reference's f32 product,
 // cpu_inference.rs:189-194).
+// HALF (M <= 8): rows 8 .. 15 of the A tile are not loaded and have no place in the slot. Their lanes
+// multiply what lies there (W), which reaches only the sums of those rows, and those are not written.
 // Bound: at these sizes the bytes each CU pulls from L2 (about 50 B/ns with all CUs loading); the
 // tile is the one with the fewest on the busiest CU (launch_kslice).
 // ---------------------------------------------------------------------------------------------
-template <bool NORM, int EPI, int MT, int NT, int NW, int NS>
+template <bool NORM, int EPI, int MT, int NT, int NW, int NS, bool HALF>
 __global__ __launch_bounds__(64 * NW) void k_gemm_kslice(GemmParams p) {
   constexpr int BM = 16 * MT, BN = 16 * NT;
-  constexpr int AI = 2 * MT, WI = NT, X = AI + WI;  // loads per step
-  constexpr uint32_t ABYTES = BM * 128, SBYTES = ABYTES + BN * 64;
+  constexpr int AI = HALF ? 1 : 2 * MT, WI = NT, X = AI + WI;  // loads per step
+  static_assert(!HALF || MT == 1, "HALF: rows 8 .. 15 of the only row block are not there");
+  constexpr uint32_t ABYTES = AI * 1024, SBYTES = ABYTES + BN * 64;
   constexpr uint32_t RING = NW * NS * SBYTES, SUMS = MT * NT * NW * 1024, TOP = RING > SUMS ? RING : SUMS;
   // the rings, later the sums
   __shared__ __align__(16) uint8_t smem[TOP];

@@ -13,6 +13,10 @@ SHAPES = [
     # k-sliced: 16 x 16, 16 x 32, 32 x 32, 32 x 48, 32 x 64, 48 x 64, 64 x 64, 64 x 128
     (1, 2, 32), (1, 6, 96), (16, 512, 64), (17, 514, 1056), (9, 6144, 1024), (33, 1026, 2048), (130, 1024, 3072),
     (64, 6144, 1024), (333, 1022, 544), (511, 1024, 2048), (130, 4094, 1024), (257, 2048, 480), (200, 4096, 96),
+    # k-sliced, up to 8 rows (half an A tile) on 16 x 16, 16 x 32 and 16 x 128, the last on ragged columns
+    (8, 1024, 3072), (3, 1022, 96), (7, 6146, 1056), (5, 80002, 288), (8, 65538, 32),
+    # k-sliced over many columns: 16 x 128, 32 x 128, 48 x 128, 64 x 128
+    (12, 70002, 288), (24, 40002, 96), (40, 40002, 96), (64, 40002, 64),
     # wide
     (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 128), (1025, 6146, 320), (2047, 4098, 64),
 ]
