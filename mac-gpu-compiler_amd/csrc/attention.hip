@@ -9,6 +9,7 @@
 // k_attn_merge.
 #include "kernels.h"
 
+#include <algorithm>
 #include <cmath>
 
 #include "attn_tile.h"
@@ -324,6 +325,125 @@ __global__ __launch_bounds__(8 * DW) void k_attn_merge(const float* __restrict__
   out[o + d] = AA / LL;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Attention of one token over at most 64 PASS positions in one launch: workgroup (g, dq) computes the
+// scores of all G q heads of KV head g over every position (K is read once per workgroup, by the four
+// workgroups of g from one L2 when n_kv is a multiple of 8), and the output's dims 32 dq .. + 31. No
+// partials, no merge. Wave w's lanes hold rows 64 i + 8 w + lane / 8, 8 lanes a row: neighbouring
+// lanes read one 128-byte line, and a row's products meet through three DPP steps.
+// Bound: the bytes of K through one CU (64 KB of K and 16 of V per 128 positions) behind one load
+// latency: all loads are issued before any is used. Rows past n_pos read the last one and weigh 0.
+// ---------------------------------------------------------------------------------------------
+template <int G, int PASS>
+__global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q_in, const float* __restrict__ k_in,
+                                                    const float* __restrict__ v_in, float* __restrict__ out, uint32_t n,
+                                                    uint32_t max_seq, float scale) {
+  constexpr int D = kHeadDim;
+  __shared__ float sc[G][64 * PASS];
+  __shared__ __align__(16) float red[8][G][32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dc = lane & 7;
+  const uint32_t g = blockIdx.x, dq = blockIdx.y;
+  const uint32_t row0 = 8 * wave + (lane >> 3);
+  const size_t base = size_t(g) * max_seq * D;
+  const float* K = k_in + base + 4 * dc;
+  const float* V = v_in + base + 32 * dq + 4 * dc;
+  float4 q[G][4], k[PASS][4], v[PASS];
+#pragma unroll
+  for (int j = 0; j < G; j++)
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      q[j][c] = *reinterpret_cast<const float4*>(q_in + size_t(g * G + j) * D + 32 * c + 4 * dc);
+#pragma unroll
+  for (int i = 0; i < PASS; i++)
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      k[i][c] = *reinterpret_cast<const float4*>(K + size_t(min(row0 + 64 * i, n - 1)) * D + 32 * c);
+#pragma unroll
+  for (int i = 0; i < PASS; i++) v[i] = *reinterpret_cast<const float4*>(V + size_t(min(row0 + 64 * i, n - 1)) * D);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < PASS; i++) {  // (a weight of 0 does not cancel an infinity)
+    const bool in = row0 + 64 * i < n;
+    v[i] = make_float4(in ? v[i].x : 0.f, in ? v[i].y : 0.f, in ? v[i].z : 0.f, in ? v[i].w : 0.f);
+  }
+#pragma unroll
+  for (int i = 0; i < PASS; i++) {
+#pragma unroll
+    for (int j = 0; j < G; j++) {
+      float a = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        a = fmaf(q[j][c].x, k[i][c].x, a);
+        a = fmaf(q[j][c].y, k[i][c].y, a);
+        a = fmaf(q[j][c].z, k[i][c].z, a);
+        a = fmaf(q[j][c].w, k[i][c].w, a);
+      }
+      a = sum8(a) * scale;
+      if (dc == 0) sc[j][row0 + 64 * i] = row0 + 64 * i < n ? a : -INFINITY;
+    }
+  }
+  __syncthreads();
+  // every wave: the maximum and the sum of all weights, then its own rows' weights
+  float4 acc[G];
+  float total[G];
+#pragma unroll
+  for (int j = 0; j < G; j++) {
+    float x[PASS], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < PASS; i++) {
+      x[i] = sc[j][lane + 64 * i];
+      m = fmaxf(m, x[i]);
+    }
+    m = wave_max(m);
+#pragma unroll
+    for (int i = 0; i < PASS; i++) l += x[i] == -INFINITY ? 0.f : expf(x[i] - m);
+    total[j] = wave_sum(l);
+    acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < PASS; i++) {
+      const float s = sc[j][row0 + 64 * i], e = s == -INFINITY ? 0.f : expf(s - m);
+      acc[j].x = fmaf(e, v[i].x, acc[j].x);
+      acc[j].y = fmaf(e, v[i].y, acc[j].y);
+      acc[j].z = fmaf(e, v[i].z, acc[j].z);
+      acc[j].w = fmaf(e, v[i].w, acc[j].w);
+    }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) {
+      acc[j].x += __shfl_xor(acc[j].x, o);
+      acc[j].y += __shfl_xor(acc[j].y, o);
+      acc[j].z += __shfl_xor(acc[j].z, o);
+      acc[j].w += __shfl_xor(acc[j].w, o);
+    }
+    if (lane < 8) *reinterpret_cast<float4*>(&red[wave][j][4 * lane]) = acc[j];
+  }
+  __syncthreads();
+  if (tid < 32 * G) {
+    const int j = tid >> 5, d = tid & 31;
+    float a = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; w++) a += red[w][j][d];
+    float l = total[0];
+#pragma unroll
+    for (int h = 1; h < G; h++) l = j == h ? total[h] : l;
+    out[size_t(g * G + j) * D + 32 * dq + d] = a / l;
+  }
+}
+
+// Positions up to which one launch of k_attn_short beats runs and their merge, up to 2 q heads per KV
+// head (more hold too many q rows in registers). 16 over 8 heads (us, one launch / two): 64 positions
+// 3.9 / 6.6, 128 4.2 / 6.6, 197 5.4 / 6.5, 256 5.3 / 6.5, but 300 (eight passes) 7.9 / 6.6.
+constexpr uint32_t kAttnShortMax = 256;
+
+template <int G>
+hipError_t launch_short(const AttnParams& p, float* out, hipStream_t s) {
+  const dim3 grid(p.n_kv, 4);
+  const uint32_t passes = ceil_div(p.n_pos_fixed, 64u);
+  auto* k = passes <= 1 ? &k_attn_short<G, 1> : passes <= 2 ? &k_attn_short<G, 2> : &k_attn_short<G, 4>;
+  hipLaunchKernelGGL(k, grid, dim3(512), 0, s, p.qkv, static_cast<const float*>(p.k_cache),
+                     static_cast<const float*>(p.v_cache), out, p.n_pos_fixed, p.max_seq, p.scale);
+  return hipGetLastError();
+}
+
 // shapes the kernels support; the runs [s*chunk, (s+1)*chunk) must cover positions 0..n-1
 bool attn_args_ok(const AttnParams& p, uint32_t splits, uint32_t chunk, uint32_t n) {
   if (!p.n_kv || p.n_heads % p.n_kv || !p.qkv || !p.k_cache || !p.v_cache || !p.partial || p.max_seq == 0)
@@ -394,11 +514,17 @@ hipError_t launch_attention_merge(const AttnParams& p, uint32_t splits, float* o
   return launch_merge(p, splits, out, 0u, 0u, s);
 }
 
-hipError_t launch_attention_op(const AttnParams& p, uint32_t splits, float* out, hipStream_t s) {
+hipError_t launch_attention_op(const AttnParams& p, uint32_t n_splits, float* out, hipStream_t s) {
+  const uint32_t splits = n_splits ? n_splits : std::min(ceil_div(p.n_pos_fixed, 64), uint32_t(kAttnMaxSplits));
   if (p.n_pos_fixed == 0 || p.n_pos_fixed > p.max_seq || splits == 0 || splits > uint32_t(kAttnMaxSplits) || !out)
     return hipErrorInvalidValue;
   const uint32_t chunk = ceil_div(p.n_pos_fixed, splits);
   if (!attn_args_ok(p, splits, chunk, p.n_pos_fixed) || p.kv_bf16 || p.row_split > 1) return hipErrorInvalidValue;
+  // (workgroups read q while others write out: only apart)
+  const float* q_end = p.qkv + size_t(p.n_heads) * kHeadDim;
+  const bool apart = out >= q_end || out + size_t(p.n_heads) * kHeadDim <= p.qkv;
+  if (n_splits == 0 && p.n_pos_fixed <= kAttnShortMax && p.n_heads <= 2 * p.n_kv && apart)
+    return p.n_heads == p.n_kv ? launch_short<1>(p, out, s) : launch_short<2>(p, out, s);
   hipError_t e = launch_split<false>(p, splits, chunk, s);
   if (e != hipSuccess) return e;
   return launch_merge(p, splits, out, 0u, 0u, s);

@@ -2114,10 +2114,7 @@ int qe_op_attention(const float* q, const float* k, const float* v, float* out, 
   a.partial = static_cast<float*>(work);
   a.n_heads = uint32_t(n_heads); a.n_kv = uint32_t(n_kv_heads); a.max_seq = uint32_t(kv_stride);
   a.scale = 1.0f / sqrtf(float(qe::kHeadDim)); a.n_pos_fixed = uint32_t(n_pos);
-  // default: runs of 64 positions (one tile each), at most kAttnMaxSplits of them
-  uint64_t splits = n_splits ? n_splits : (n_pos + 63) / 64;
-  splits = std::min<uint64_t>(std::max<uint64_t>(splits, 1), qe::kAttnMaxSplits);
-  HIP_TRY(qe::launch_attention_op(a, uint32_t(splits), out, static_cast<hipStream_t>(stream)));
+  HIP_TRY(qe::launch_attention_op(a, n_splits, out, static_cast<hipStream_t>(stream)));
   return QE_OK;
 }
 

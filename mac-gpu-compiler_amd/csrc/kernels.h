@@ -128,8 +128,9 @@ L2Prefetch l2_prefetch_target(const uint16_t* w, uint32_t rows, uint32_t cols, i
 // Prefetch workgroups per XCD for these targets (each loads at most 16 chunks per thread).
 uint32_t l2_prefetch_slots(const L2Prefetch* pf, int n);
 // The isolated op: final q [n_heads][D], complete K/V [n_kv][max_seq][D] (f32), positions
-// 0..n_pos_fixed-1 in `splits` runs (<= kAttnMaxSplits), partials merged into out [n_heads][D].
-hipError_t launch_attention_op(const AttnParams& p, uint32_t splits, float* out, hipStream_t s);
+// 0..n_pos_fixed-1 in `n_splits` runs (<= kAttnMaxSplits), partials merged into out [n_heads][D].
+// n_splits = 0: one launch over a short context, else runs of 64 positions, at most kAttnMaxSplits.
+hipError_t launch_attention_op(const AttnParams& p, uint32_t n_splits, float* out, hipStream_t s);
 // Attention of T tokens at positions n_pos_fixed - T .. n_pos_fixed - 1 over positions
 // 0..n_pos_fixed-1 of a cache that already holds their K/V (f32 or bf16), causal among them, with
 // the same kernels: q [T][heads][128] final (normalized, rotated), out [T][heads][128]. The T

@@ -77,7 +77,7 @@ extern "C" int qe_op_attention_static(const float* q, const float* k, const floa
   a.max_seq = uint32_t(kv_stride);
   a.scale = 1.0f / sqrtf(float(qe::kHeadDim));
   a.n_pos_fixed = uint32_t(n_pos);
-  const hipError_t e = qe::launch_attention_op(a, uint32_t(splits), out, static_cast<hipStream_t>(stream));
+  const hipError_t e = qe::launch_attention_op(a, n_splits, out, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return qe::set_error(QE_ERR_HIP, "attention launch failed: %s", hipGetErrorString(e));
   return QE_OK;
 }
