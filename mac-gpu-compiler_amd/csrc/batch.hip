@@ -140,7 +140,15 @@ __global__ __launch_bounds__(256) void k_qk_rope(BatchAttnParams p) {
 // position 1536: 46 -> 34 us.
 // ---------------------------------------------------------------------------------------------
 template <int G, bool KV_BF16, int RB, bool ROPE>
-__global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
+__global__ __launch_bounds__(512) void k_attn_causal_bf(const float* q_in, const void* k_cache, const void* v_cache,
+                                                        uint32_t start, uint32_t M, uint32_t max_seq,
+                                                        uint32_t key_run, uint32_t runs, uint32_t n_heads,
+                                                        uint32_t n_kv, BatchAttnParams p) {
+  // what the first loads need comes first, as plain values (in scalar registers when a wave starts)
+  if constexpr (ROPE) p.qkv = q_in;
+  else p.q = const_cast<float*>(q_in);
+  p.k_cache = const_cast<void*>(k_cache), p.v_cache = const_cast<void*>(v_cache);
+  p.start = start, p.M = M, p.max_seq = max_seq, p.key_run = key_run, p.n_heads = n_heads, p.n_kv = n_kv;
   constexpr int D = kHeadDim, BK = 64, TOK = 64 * RB / G, KP = D + 8, VP = BK + 8, NL = KV_BF16 ? 1 : 2;
   constexpr int KS = NL * BK * KP, TILE = KS + NL * D * VP;        // u16s: K [hi, lo][key][dim], V [hi, lo][dim][key slot]
   constexpr int MERGE = 4 * RB * (8 * 64 * 8 + 16 * 4);            // ... of the halves' merge
@@ -148,7 +156,7 @@ __global__ __launch_bounds__(512) void k_attn_causal_bf(BatchAttnParams p) {
   __shared__ __align__(16) uint16_t smem[NB * TILE > MERGE ? NB * TILE : MERGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
   const int rw = wave & 3, kh = wave >> 2;
-  const uint32_t g = blockIdx.x, mb = blockIdx.y * TOK, run = blockIdx.z, runs = p.runs;
+  const uint32_t g = blockIdx.x, mb = blockIdx.y * TOK, run = blockIdx.z;
   if (run >= runs) {  // a prefetch workgroup (whole workgroup, before any load)
     l2_prefetch_tiles(p.pf.pf, (run - runs) * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + g,
                       reinterpret_cast<uint32_t*>(p.att));
@@ -1151,11 +1159,13 @@ hipError_t launch_kslice_t(const GemmParams& p, hipStream_t st) {
   if (hipError_t e = check_grid(wgs, 64 * NW)) return e;
   if constexpr (MT == 1) {
     if (p.M <= 8) {
-      hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, true>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
+      hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, true>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p.A, p.W,
+                         p.gain, p.C, p.lda, p.M, p.N, p.K, p.ldc, p.eps);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, false>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p);
+  hipLaunchKernelGGL((k_gemm_kslice<NORM, EPI, MT, NT, NW, NS, false>), dim3(uint32_t(wgs)), dim3(64 * NW), 0, st, p.A, p.W,
+                     p.gain, p.C, p.lda, p.M, p.N, p.K, p.ldc, p.eps);
   return hipGetLastError();
 }
 
@@ -1217,7 +1227,8 @@ template <int EPI, bool SPLIT, int BM, int BN, int NS>
 hipError_t launch_wide_t(const GemmParams& p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
   const uint64_t wgs = (uint64_t(p.M) + BM - 1) / BM * ((uint64_t(p.N) + BN - 1) / BN) * splits;
   if (hipError_t e = check_grid(wgs, 512)) return e;
-  hipLaunchKernelGGL((k_gemm_wide<EPI, SPLIT, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p, qa);
+  hipLaunchKernelGGL((k_gemm_wide<EPI, SPLIT, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p.A, p.W, p.gain, p.C,
+                     p.lda, p.M, p.N, p.K, p.ldc, p.kz, qa);
   return hipGetLastError();
 }
 
@@ -1320,7 +1331,8 @@ hipError_t launch_attn_causal_t(const BatchAttnParams& p, bool rope, dim3 grid, 
   if constexpr (RB == 1) {
     if (rope) k = p.kv_bf16 ? &k_attn_causal_bf<G, true, RB, true> : &k_attn_causal_bf<G, false, RB, true>;
   }
-  hipLaunchKernelGGL(k, grid, dim3(512), 0, st, p);
+  hipLaunchKernelGGL(k, grid, dim3(512), 0, st, rope ? p.qkv : p.q, p.k_cache, p.v_cache, p.start, p.M, p.max_seq,
+                     p.key_run, p.runs, p.n_heads, p.n_kv, p);
   return hipGetLastError();
 }
 
