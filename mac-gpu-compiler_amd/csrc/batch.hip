@@ -1121,14 +1121,17 @@ hipError_t launch_lm_head_rows(const MvRowsParams& p, hipStream_t st) {
 }
 
 hipError_t launch_mv_rows(const MvRowsParams& p, bool norm, int epi, hipStream_t st) {
-  if (!p.w || !p.x || !p.out || (norm && !p.gain) || p.M == 0 || p.M > kMvRowsMaxM || p.rows == 0 || p.cols == 0 ||
+  const uint32_t max_m = !norm && epi == kGemmResAdd ? kMvResAddMaxM : kMvRowsMaxM;
+  if (!p.w || !p.x || !p.out || (norm && !p.gain) || p.M == 0 || p.M > max_m || p.rows == 0 || p.cols == 0 ||
       p.cols % 8 || p.cols / 8 > 512 || (epi == kGemmSiluPair ? p.rows % 2 || p.ldo < p.rows / 2 : p.ldo < p.rows))
     return hipErrorInvalidValue;
   switch (p.M) {
     case 1: return launch_mv_rows_nv<1>(p, norm, epi, st);
     case 2: return launch_mv_rows_nv<2>(p, norm, epi, st);
     case 3: return launch_mv_rows_nv<3>(p, norm, epi, st);
-    default: return launch_mv_rows_nv<4>(p, norm, epi, st);
+    case 4: return launch_mv_rows_nv<4>(p, norm, epi, st);
+    case 5: return launch_mv_rows_cols<5, false, kGemmResAdd>(p, st);
+    default: return launch_mv_rows_cols<6, false, kGemmResAdd>(p, st);
   }
 }
 

@@ -1007,7 +1007,9 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
     // q|k|v and gate|up (many rows of W, few columns) are faster on the k-sliced GEMM from 3 rows: 1.324
     // ms vs 1.366 per k = 4 verify at 2048, 1.164 vs 1.200 at 3 rows and 700; o_proj and down are not
     // (1.448 at 4 rows)
-    if (mv && lda == K && W != m->lm_head && !(gain && M >= 3)) {
+    // (K % 32: widths that only the matvec takes)
+    const bool by_rows = gain || epi != qe::kGemmResAdd ? M < 3 || (mv && K % 32) : M <= qe::kMvResAddMaxM;
+    if (m->mv_rows && by_rows && lda == K && W != m->lm_head) {
       qe::MvRowsParams r{W, A, gain, C, M, N, K, ldc, eps};
       HIP_TRY(qe::launch_mv_rows(r, gain != nullptr, epi, s));
       return QE_OK;

@@ -67,3 +67,12 @@ def test_scores_that_grow_over_the_tiles(gpu, tmp_path):
     model.prefill(ids[:640], 0, c, want_logits=False)
     rows = [model.verify(ids[640 + i:660 + i], 640 + i, c) for i in (0, 20, 40)]
     assert np.max(np.abs(rows[2][-1] - ref)) < 5e-3
+
+
+def test_short_chunks_of_widths_that_only_the_matvec_takes(gpu, tmp_path):
+    """hidden and intermediate sizes that are no multiple of 32: chunks of up to 3 tokens"""
+    model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 3, qe.Config(264, 520, 2, 4, 2, 128, 1000,
+                                                                                      1e-6, 1e6, 999)))
+    ids = qe.random_prompt(5, 21, 1000)
+    a, b = qe.KVCache(model, 24), qe.KVCache(model, 24)
+    assert np.max(np.abs(model.prefill_batch(ids, 0, a, chunk=3) - model.prefill(ids, 0, b))) < 1e-3
