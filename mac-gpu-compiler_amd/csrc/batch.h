@@ -45,9 +45,8 @@ constexpr int kGemmNormMaxK = 4096;
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
 // token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
 // own products and lane reductions to every wave of that matvec, so past a few rows the k-sliced GEMM
-// on the matrix cores is faster: with a norm from 3 rows (enqueue_batch), with a residual from 7, where
-// the GEMM's 64 workgroups of 16 columns leave most CUs idle (verify at 700, us, matvec / GEMM: 5 rows
-// 1220 / 1262, 6 rows 1274 / 1297).
+// on the matrix cores is faster: with a residual from 7, where the GEMM's 64 workgroups of 16 columns
+// leave most CUs idle (verify at 700, us, matvec / GEMM: 5 rows 1220 / 1262, 6 rows 1274 / 1297).
 constexpr uint32_t kMvRowsMaxM = 4;
 constexpr uint32_t kMvResAddMaxM = 6;  // with a residual and no norm (o_proj, down)
 struct MvRowsParams {

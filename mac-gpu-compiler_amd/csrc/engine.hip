@@ -997,18 +997,19 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   // norm within and adds residuals in its epilogue. Past that, what the GEMMs read is written split
   // into bf16 halves by whatever computes it: bxs holds the current norm of x, from the reduction
   // that finishes each split o_proj / down (residual add + the next norm in one pass).
-  // Up to kMvRowsMaxM rows the projections are matvecs over the M token rows: each weight is
-  // loaded once per pass, the norm is computed per row in the kernel and the residual is added in
-  // its epilogue (the lm_head of a verify stays on the k-sliced GEMM).
+  // Up to kMvRowsMaxM rows (gate|up: 3; o_proj and down: kMvResAddMaxM) the projections are matvecs
+  // over the M token rows: each weight is loaded once per pass, the norm is computed per row in the
+  // kernel and the residual is added in its epilogue. The lm_head is a matvec up to kMvRowsMaxM rows.
   const bool wide = M > qe::kGemmSliceMaxM && H % 64 == 0 && I % 64 == 0 && QD % 64 == 0;
   const bool mv = m->mv_rows && M <= qe::kMvRowsMaxM;
   auto gemm = [&](const float* A, uint32_t lda, const uint16_t* gain, const uint16_t* W, uint32_t N, uint32_t K,
                   float* C, uint32_t ldc, int epi) -> int {
-    // q|k|v and gate|up (many rows of W, few columns) are faster on the k-sliced GEMM from 3 rows: 1.324
-    // ms vs 1.366 per k = 4 verify at 2048, 1.164 vs 1.200 at 3 rows and 700; o_proj and down are not
-    // (1.448 at 4 rows)
-    // (K % 32: widths that only the matvec takes)
-    const bool by_rows = gain || epi != qe::kGemmResAdd ? M < 3 || (mv && K % 32) : M <= qe::kMvResAddMaxM;
+    // A pass of few rows multiplies in f32, as a decode step does; the k-sliced GEMM holds each activation
+    // as two bf16 halves (about 16 mantissa bits), so its time alone moves no projection there. gate|up of
+    // 4 rows runs there (K % 32: widths that only the matvec takes).
+    const bool by_rows = epi == qe::kGemmResAdd  ? M <= qe::kMvResAddMaxM
+                         : epi == qe::kGemmSiluPair ? M < 4 || (mv && K % 32)
+                                                    : mv;
     if (m->mv_rows && by_rows && lda == K && W != m->lm_head) {
       qe::MvRowsParams r{W, A, gain, C, M, N, K, ldc, eps};
       HIP_TRY(qe::launch_mv_rows(r, gain != nullptr, epi, s));
@@ -1076,9 +1077,9 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       if (rows_per_kv == 8) r.row_split = 2;
       if (m->l2_prefetch && mv) {
         // as in the decode step: the attention is latency-bound, so extra workgroups load this
-        // layer's gate|up (up to 2 tokens: as the multi-row matvec reads it) and
+        // layer's gate|up (up to 3 tokens: as the multi-row matvec reads it) and
         // down weights into the L2 of the XCDs that will read them
-        if (M < 3) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
+        if (M < 4) r.pf[0] = qe::l2_prefetch_target(w.w_gu, 2 * I, H, qe::kNorm, qe::kSiluPair);
         r.pf[1] = qe::l2_prefetch_target(w.w_down, H, I, qe::kCopy, qe::kResAdd);
         r.pf_slots = qe::l2_prefetch_slots(r.pf, qe::kMaxPrefetch);
       }

@@ -1,0 +1,68 @@
+"""Verify passes of 3 and 4 rows multiply in f32 as a decode step does: what they compute differs from
+the same tokens one by one by f32 sums in another order, not by activations held as bf16 halves (gate|up
+of 4 rows and the attention of 3 run on the matrix cores, so the checkpoints leave those out of what is
+compared)."""
+import json
+
+import numpy as np
+import pytest
+
+import qe
+
+pytestmark = pytest.mark.gpu
+
+CFG = qe.Config(256, 512, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999)
+
+
+def load(path, edits):
+    """the seeded checkpoint with edits: tensor name -> bf16 bits by a function of them"""
+    file = qe.write_random_checkpoint(str(path), 7, CFG)
+    raw = np.memmap(file, dtype=np.uint8, mode="r+")
+    n = int(raw[:8].view(np.uint64)[0])
+    for name, t in json.loads(bytes(raw[8:8 + n])).items():
+        for part, f in edits.items():
+            if part in name:
+                a, b = t["data_offsets"]
+                bits = raw[8 + n + a:8 + n + b].view(np.uint16)
+                bits[:] = f(bits)
+    raw.flush()
+    del raw
+    return qe.Model.load_model(file)
+
+
+def times16(bits):  # attention's part of the residual is most of it
+    return bits + np.uint16(4 << 7)
+
+
+def zero(bits):
+    return np.uint16(0)
+
+
+def rel(x, y):
+    return float(np.linalg.norm(x - y) / np.linalg.norm(y))
+
+
+# f32 sums of up to 512 products and f32 softmax in two layers: 2e-7 measured over three seeds;
+# activations held in 16 bits (2^-17 each) give 1.4e-6 to 2.8e-6
+BOUND = 6e-7
+
+
+def test_four_rows_project_in_f32(gpu, tmp_path):
+    model = load(tmp_path, {"down_proj": zero, "o_proj": times16})
+    ids = qe.random_prompt(5, 5, 1000)
+    a, b = qe.KVCache(model, 8), qe.KVCache(model, 8)
+    rows = model.verify(ids[:4], 0, a)
+    for i in range(4):
+        assert rel(rows[i], model.forward(int(ids[i]), i, b)) < BOUND, f"row {i}"
+    assert rel(model.forward(int(ids[4]), 4, a), model.forward(int(ids[4]), 4, b)) < BOUND
+
+
+def test_three_rows_project_in_f32(gpu, tmp_path):
+    # the second layer's K/V rows come from the first layer's MLP alone
+    model = load(tmp_path, {"layers.0.self_attn.o_proj": zero, "layers.1.self_attn.o_proj": times16})
+    ids = qe.random_prompt(5, 4, 1000)
+    a, b = qe.KVCache(model, 8), qe.KVCache(model, 8)
+    model.verify(ids[:3], 0, a)
+    for i in range(3):
+        model.forward(int(ids[i]), i, b)
+    assert rel(model.forward(int(ids[3]), 3, a), model.forward(int(ids[3]), 3, b)) < BOUND
