@@ -222,7 +222,9 @@ int qe_op_gemm_bf16(const float* a, const void* w, float* c, uint64_t m, uint64_
  * [n_kv_heads][kv_stride][128] f32, attending positions 0..n_pos-1; out [n_heads*128].
  * The positions are split into n_splits runs (1..128; 0 picks runs of 64 positions), each
  * attended by one workgroup per KV head, and a second kernel merges the runs' partial softmax
- * sums. With n_splits = 0, up to 256 positions and 2 q heads per KV head, one kernel does it all. `work` (partials, overwritten by every call) must hold qe_op_attention_work_bytes(...)
+ * sums; with n_splits = 0, up to 256 positions and 1 or 2 q heads per KV head, one kernel does
+ * both unless out overlaps q, k or v (it may, in either form: they are read before it is
+ * written). `work` (partials, overwritten by every call) must hold qe_op_attention_work_bytes(...)
  * bytes of device memory. */
 uint64_t qe_op_attention_work_bytes(uint64_t n_heads, uint64_t n_kv_heads, uint64_t n_pos);
 int qe_op_attention(const float* q, const float* k, const float* v, float* out, uint64_t n_pos,

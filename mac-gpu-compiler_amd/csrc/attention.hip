@@ -434,6 +434,12 @@ __global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q_
 // 3.9 / 6.6, 128 4.2 / 6.6, 197 5.4 / 6.5, 256 5.3 / 6.5, but 300 (eight passes) 7.9 / 6.6.
 constexpr uint32_t kAttnShortMax = 256;
 
+// floats a[0 .. na) and b[0 .. nb) share no byte
+bool apart(const void* a, size_t na, const void* b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x + na * sizeof(float) <= y || y + nb * sizeof(float) <= x;
+}
+
 template <int G>
 hipError_t launch_short(const AttnParams& p, float* out, hipStream_t s) {
   const dim3 grid(p.n_kv, 4);
@@ -520,10 +526,12 @@ hipError_t launch_attention_op(const AttnParams& p, uint32_t n_splits, float* ou
     return hipErrorInvalidValue;
   const uint32_t chunk = ceil_div(p.n_pos_fixed, splits);
   if (!attn_args_ok(p, splits, chunk, p.n_pos_fixed) || p.kv_bf16 || p.row_split > 1) return hipErrorInvalidValue;
-  // (workgroups read q while others write out: only apart)
-  const float* q_end = p.qkv + size_t(p.n_heads) * kHeadDim;
-  const bool apart = out >= q_end || out + size_t(p.n_heads) * kHeadDim <= p.qkv;
-  if (n_splits == 0 && p.n_pos_fixed <= kAttnShortMax && p.n_heads <= 2 * p.n_kv && apart)
+  // k_attn_short's workgroups write out while others still read q, k and v: only where out lies apart from
+  // all three. Of the two launches the merge writes out, after every read of them.
+  const size_t n_q = size_t(p.n_heads) * kHeadDim, n_cache = size_t(p.n_kv) * p.max_seq * kHeadDim;
+  const bool alone = apart(out, n_q, p.qkv, n_q) && apart(out, n_q, p.k_cache, n_cache) &&
+                     apart(out, n_q, p.v_cache, n_cache);
+  if (n_splits == 0 && p.n_pos_fixed <= kAttnShortMax && p.n_heads <= 2 * p.n_kv && alone)
     return p.n_heads == p.n_kv ? launch_short<1>(p, out, s) : launch_short<2>(p, out, s);
   hipError_t e = launch_split<false>(p, splits, chunk, s);
   if (e != hipSuccess) return e;

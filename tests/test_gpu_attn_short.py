@@ -1,6 +1,6 @@
 """qe_op_attention's single launch over a short context: every number of passes, positions on both sides
 of a pass and of the longest context it takes, one and two q heads per KV head, rows past the context
-that hold NaN, and an output that overwrites q (which takes the runs)."""
+that hold NaN, and an output that overwrites q, or rows of k or v in use (which takes the runs)."""
 import numpy as np
 import pytest
 
@@ -28,3 +28,23 @@ def test_short_context_matches_float64(gpu, n_pos, n_heads, n_kv, in_place):
     ref = (s @ v[:, :n_pos].double()).reshape(-1)
     # f32 scores of 128 products (|s| < 8: 2^-19 absolute), weights and sums of n_pos terms
     assert float((out.cpu().double() - ref).abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("n_pos", [64, 200, 256])
+@pytest.mark.parametrize("over,row", [("k", 0), ("k", -1), ("v", 0), ("v", -1)])
+def test_out_over_rows_in_use_equals_out_apart(gpu, n_pos, over, row):
+    """out over the first used rows of the cache, or over its end (partly past the used rows): the merge
+    writes it after every read of k and v, so the result is the runs' own, bit for bit"""
+    import torch
+    n_heads, n_kv = 16, 8
+    g = torch.Generator().manual_seed(n_pos)
+    q, stride = torch.randn(n_heads * 128, generator=g).cuda(), n_pos + 3
+    k, v = (torch.randn(n_kv, stride, 128, generator=g).cuda() for _ in range(2))
+    work = torch.empty(qe.op_attention_work_bytes(n_heads, n_kv, n_pos), dtype=torch.uint8, device="cuda")
+    want = torch.empty_like(q)
+    qe.op_attention(q, k, v, want, n_pos, n_heads, n_kv, work, n_splits=(n_pos + 63) // 64)
+    flat = {"k": k, "v": v}[over].view(-1)
+    out = flat[:n_heads * 128] if row == 0 else flat[-n_heads * 128:]
+    qe.op_attention(q, k, v, out, n_pos, n_heads, n_kv, work)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
