@@ -82,7 +82,8 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 constexpr uint32_t kBatchDefaultChunk = 512;  // tokens per chunk of qe_prefill_batch (chunk = 0)
 constexpr uint32_t kBatchMaxChunk = 2048;
-constexpr uint32_t kRowSlots = 8;  // pinned logits rows a verify pass keeps in flight to the host
+constexpr uint32_t kCopySlots = 8;  // pinned pieces of a verify pass's logits in flight to the host
+constexpr size_t kCopyPiece = size_t(640) << 10;
 constexpr uint32_t kVerifyMaxTokens = 64;  // tokens of one qe_verify call
 static_assert(kVerifyMaxTokens <= qe::kIdsByValue, "verify ids travel in a kernel argument");
 
@@ -219,9 +220,9 @@ struct qe_model {
   float* blogits = nullptr;
   uint32_t* ids_dev = nullptr;  // the token ids of one qe_prefill_batch / qe_verify call
   uint64_t ids_cap = 0;
-  // pinned slots that a verify pass's logits rows travel through (copy_logit_rows), made on first use
-  float* h_rows = nullptr;
-  hipEvent_t row_ev[kRowSlots] = {};
+  // pinned slots that a verify pass's logits travel through (copy_logit_rows), made on first use
+  uint8_t* h_pieces = nullptr;
+  hipEvent_t piece_ev[kCopySlots] = {};
 
   ~qe_model() {  // teardown errors have nowhere to go; the handle is gone either way
     if (stream) (void)hipStreamSynchronize(stream);
@@ -239,8 +240,8 @@ struct qe_model {
     if (vstage_ev) (void)hipEventDestroy(vstage_ev);
     if (ids_dev) (void)hipFree(ids_dev);
     if (h_logits) (void)hipHostFree(h_logits);
-    if (h_rows) (void)hipHostFree(h_rows);
-    for (hipEvent_t e : row_ev)
+    if (h_pieces) (void)hipHostFree(h_pieces);
+    for (hipEvent_t e : piece_ev)
       if (e) (void)hipEventDestroy(e);
     if (h_small) (void)hipHostFree(h_small);
     if (stream) (void)hipStreamDestroy(stream);
@@ -1659,27 +1660,47 @@ int check_verify_args(qe_model* model, const uint32_t* ids, uint64_t k, uint64_t
   return QE_OK;
 }
 
-// The pass's `rows` logits rows to the caller's memory, once the stream has computed them: each row
-// travels through a pinned slot, so that it is copied out while the next ones are on their way. (A
-// copy straight into pageable memory goes a megabyte at a time, with nothing in flight while the host
-// copies it: verify of 5 rows at 700 1366 -> 1325 us together with the lm_head's tile, of 40 rows 2775 -> 2440.)
+// The pass's `rows` logits rows to the caller's memory, once the stream has computed them. Pageable memory:
+// in pieces through pinned slots, so that a piece is copied out while the next ones are on their way (a
+// copy straight into it goes a megabyte at a time, with nothing in flight while the host copies). Verify at
+// 300 with 151,936 logits a row, us, straight / pieces of 512 KiB / about 640 KiB / 1 MiB: 2 rows 642, 630, 626,
+// 637; 16 rows 1781, 1673, 1640, 1613; 64 rows into new pages 5260, 4409, 4198, 4510; with 8,000 a row, 40 rows
+// 430, 418, 417, 428 (913 with a copy and an event for every row).
+// Memory that the runtime knows (pinned, managed, a device's) is written by the copy itself: 16 rows 1391
+// into pinned memory, 1647 through the slots.
 int copy_logit_rows(qe_model* m, uint32_t rows, float* out) {
-  const size_t V = m->cfg.vocab_size;
-  if (!m->h_rows) HIP_TRY(hipHostMalloc(&m->h_rows, kRowSlots * V * 4, hipHostMallocDefault));
-  for (hipEvent_t& e : m->row_ev)
+  const size_t total = size_t(rows) * m->cfg.vocab_size * 4;
+  constexpr size_t P = kCopyPiece;
+  hipPointerAttribute_t at{};
+  bool staged = hipPointerGetAttributes(&at, out) != hipSuccess || at.type == hipMemoryTypeUnregistered;
+  if (staged && !m->h_pieces &&
+      hipHostMalloc(&m->h_pieces, kCopySlots * P, hipHostMallocDefault) != hipSuccess) {
+    m->h_pieces = nullptr;  // no memory to pin: straight
+    staged = false;
+  }
+  (void)hipGetLastError();  // (an unknown pointer is an error to some runtimes)
+  if (!staged) {
+    HIP_TRY(hipMemcpyAsync(out, m->blogits, total, hipMemcpyDeviceToHost, m->stream));
+    HIP_TRY(hipStreamSynchronize(m->stream));
+    return QE_OK;
+  }
+  for (hipEvent_t& e : m->piece_ev)
     if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  auto send = [&](uint32_t r) -> hipError_t {
-    const uint32_t s = r % kRowSlots;
-    if (hipError_t e = hipMemcpyAsync(m->h_rows + s * V, m->blogits + r * V, V * 4, hipMemcpyDeviceToHost, m->stream))
+  const size_t pieces = (total + P - 1) / P;
+  auto bytes = [&](size_t i) { return std::min(P, total - i * P); };
+  auto send = [&](size_t i) -> hipError_t {
+    const size_t s = i % kCopySlots;
+    if (hipError_t e = hipMemcpyAsync(m->h_pieces + s * P, reinterpret_cast<uint8_t*>(m->blogits) + i * P, bytes(i),
+                                      hipMemcpyDeviceToHost, m->stream))
       return e;
-    return hipEventRecord(m->row_ev[s], m->stream);
+    return hipEventRecord(m->piece_ev[s], m->stream);
   };
   hipError_t e = hipSuccess;
-  for (uint32_t r = 0; r < rows && r < kRowSlots && e == hipSuccess; r++) e = send(r);
-  for (uint32_t r = 0; r < rows && e == hipSuccess; r++) {
-    if ((e = hipEventSynchronize(m->row_ev[r % kRowSlots])) != hipSuccess) break;
-    memcpy(out + r * V, m->h_rows + (r % kRowSlots) * V, V * 4);
-    if (r + kRowSlots < rows) e = send(r + kRowSlots);
+  for (size_t i = 0; i < pieces && i < kCopySlots && e == hipSuccess; i++) e = send(i);
+  for (size_t i = 0; i < pieces && e == hipSuccess; i++) {
+    if ((e = hipEventSynchronize(m->piece_ev[i % kCopySlots])) != hipSuccess) break;
+    memcpy(reinterpret_cast<uint8_t*>(out) + i * P, m->h_pieces + (i % kCopySlots) * P, bytes(i));
+    if (i + kCopySlots < pieces) e = send(i + kCopySlots);
   }
   if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // nothing queued outlives the call
   HIP_TRY(e);

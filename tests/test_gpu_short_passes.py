@@ -1,4 +1,5 @@
-"""Verify passes of 3 and 4 rows multiply in f32 as a decode step does: what they compute differs from
+"""Short verify passes: what they multiply in, and the way of their logits to the host.
+Passes of 3 and 4 rows multiply in f32 as a decode step does: what they compute differs from
 the same tokens one by one by f32 sums in another order, not by activations held as bf16 halves (gate|up
 of 4 rows and the attention of 3 run on the matrix cores, so the checkpoints leave those out of what is
 compared)."""
@@ -66,3 +67,24 @@ def test_three_rows_project_in_f32(gpu, tmp_path):
     for i in range(3):
         model.forward(int(ids[i]), i, b)
     assert rel(model.forward(int(ids[3]), 3, a), model.forward(int(ids[3]), 3, b)) < BOUND
+
+
+@pytest.mark.parametrize("k", [1, 4, 5, 33, 64])
+def test_logits_arrive_whole_in_pageable_and_pinned_memory(gpu, tmp_path, k):
+    """40,002 logits a row: one, two, nine and sixteen pieces (the slots taken again) through pinned slots into
+    pageable memory; pinned memory is written directly"""
+    import ctypes
+
+    import torch
+    V = 40002
+    model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 7, qe.Config(256, 512, 1, 2, 2, 128, V, 1e-6,
+                                                                                       1e6, 999)))
+    ids = np.ascontiguousarray(qe.random_prompt(5, k, V))
+    cache = qe.KVCache(model, k)
+    pinned = torch.full((k * V + 1,), float("nan"), pin_memory=True)
+    paged = np.full(k * V + 1, np.nan, dtype=np.float32)
+    for at in (pinned.data_ptr(), paged.ctypes.data):
+        qe._check(qe.lib().qe_verify(model._h, ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), k, 0, cache._h,
+                                     ctypes.cast(at, ctypes.POINTER(ctypes.c_float))))
+    np.testing.assert_array_equal(paged, pinned.numpy())
+    assert np.isfinite(paged[:-1]).all() and np.isnan(paged[-1])
