@@ -45,10 +45,13 @@ constexpr int kGemmNormMaxK = 4096;
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
 // token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
 // own products and lane reductions to every wave of that matvec, so past a few rows the k-sliced GEMM
-// on the matrix cores is faster: with a residual from 7, where the GEMM's 64 workgroups of 16 columns
-// leave most CUs idle (verify at 700, us, matvec / GEMM: 5 rows 1220 / 1262, 6 rows 1274 / 1297).
+// on the matrix cores is faster. With a residual and few weight rows (o_proj and down at a hidden size
+// of up to 1024) that is from 7 rows, as the GEMM has at most 64 workgroups of 16 columns for 256 CUs
+// (us, matvec / GEMM: qe_verify_greedy of 5 and 6 rows, hidden 1024 and 28 layers 1031 / 1069 and 1059 /
+// 1080; 8 layers 303 / 315, 311 / 318; hidden 512 247 / 251, 249 / 255), with more of them from 5 (hidden
+// 1536 283 / 264, 296 / 267; 2048 329 / 291, 341 / 295; 4096 378 / 299, 408 / 301).
 constexpr uint32_t kMvRowsMaxM = 4;
-constexpr uint32_t kMvResAddMaxM = 6;  // with a residual and no norm (o_proj, down)
+constexpr uint32_t kMvResAddMaxM = 6, kMvResAddMaxN = 1024;  // with a residual and no norm
 struct MvRowsParams {
   const uint16_t* w;     // bf16 [rows][cols], row-major
   const float* x;        // [M][cols]
@@ -114,7 +117,7 @@ hipError_t launch_resadd_norm_split(float* x, const float* part, uint32_t splits
 // out[m][r] (=, +=) sum_c W[r][c] x'[m][c] for m < M (kGemmStore / kGemmResAdd), or
 // out[m][i] = silu(gate_i) * up_i over the interleaved gate/up rows (kGemmSiluPair, ldo >= rows/2);
 // x' = x, or RMSNorm(x_m) * gain with `norm`. f32 FMA on bf16 weights, as the decode matvec.
-// cols % 8 == 0, cols <= 4096, 1 <= M <= kMvRowsMaxM; out must not alias x.
+// cols % 8 == 0, cols <= 4096, 1 <= M <= kMvRowsMaxM (kMvResAddMaxM with a residual and no norm); out must not alias x.
 hipError_t launch_mv_rows(const MvRowsParams& p, bool norm, int epi, hipStream_t st);
 // final RMSNorm (gain) + lm_head of M <= kMvRowsMaxM token rows: out[m][row], each row's logits
 // equal to the decode step's lm_head's for that hidden state (its layout and summation order).

@@ -998,7 +998,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   // norm within and adds residuals in its epilogue. Past that, what the GEMMs read is written split
   // into bf16 halves by whatever computes it: bxs holds the current norm of x, from the reduction
   // that finishes each split o_proj / down (residual add + the next norm in one pass).
-  // Up to kMvRowsMaxM rows (gate|up: 3; o_proj and down: kMvResAddMaxM) the projections are matvecs
+  // Up to kMvRowsMaxM rows (gate|up: 3; o_proj and down into few columns: kMvResAddMaxM) the projections are matvecs
   // over the M token rows: each weight is loaded once per pass, the norm is computed per row in the
   // kernel and the residual is added in its epilogue. The lm_head is a matvec up to kMvRowsMaxM rows.
   const bool wide = M > qe::kGemmSliceMaxM && H % 64 == 0 && I % 64 == 0 && QD % 64 == 0;
@@ -1008,7 +1008,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
     // A pass of few rows multiplies in f32, as a decode step does; the k-sliced GEMM holds each activation
     // as two bf16 halves (about 16 mantissa bits), so its time alone moves no projection there. gate|up of
     // 4 rows runs there (K % 32: widths that only the matvec takes).
-    const bool by_rows = epi == qe::kGemmResAdd  ? M <= qe::kMvResAddMaxM
+    const bool by_rows = epi == qe::kGemmResAdd  ? mv || (M <= qe::kMvResAddMaxM && N <= qe::kMvResAddMaxN)
                          : epi == qe::kGemmSiluPair ? M < 4 || (mv && K % 32)
                                                     : mv;
     if (m->mv_rows && by_rows && lda == K && W != m->lm_head) {

@@ -88,3 +88,18 @@ def test_logits_arrive_whole_in_pageable_and_pinned_memory(gpu, tmp_path, k):
                                      ctypes.cast(at, ctypes.POINTER(ctypes.c_float))))
     np.testing.assert_array_equal(paged, pinned.numpy())
     assert np.isfinite(paged[:-1]).all() and np.isnan(paged[-1])
+
+
+@pytest.mark.parametrize("hidden", [1024, 1056])
+@pytest.mark.parametrize("k", [4, 5, 6, 7])
+def test_rows_on_both_sides_of_the_residual_rule(gpu, tmp_path, hidden, k):
+    """o_proj and down of 5 and 6 rows: the matvec up to 1024 weight rows, the GEMM past that"""
+    model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 7, qe.Config(hidden, 512, 2, 4, 2, 128, 1000,
+                                                                                       1e-6, 1e6, 999)))
+    ids = qe.random_prompt(5, 20 + k, 1000)
+    a, b = qe.KVCache(model, 20 + k), qe.KVCache(model, 20 + k)
+    for c in (a, b):
+        model.prefill(ids[:20], 0, c, want_logits=False)
+    rows = model.verify(ids[20:], 20, a)
+    for i in range(k):  # activations in 16 bits, two layers and the lm_head: some 2^-17 each
+        assert rel(rows[i], model.forward(int(ids[20 + i]), 20 + i, b)) < 4e-5, f"row {i}"
