@@ -1172,16 +1172,21 @@ hipError_t launch_kslice_t(const GemmParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// (the last four: many columns, as an lm_head's, where a wide tile has fewer bytes of A beside its W)
+constexpr uint32_t kSliceTiles[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64},  {48, 64},
+                                       {64, 64}, {16, 128}, {32, 128}, {48, 128}, {64, 128}};
+int slice_tile(const GemmParams& p) {
+  int best = 0;
+  for (int i = 1; i < 11; i++)
+    if (tile_cost(p, kSliceTiles[i][0], kSliceTiles[i][1]) < tile_cost(p, kSliceTiles[best][0], kSliceTiles[best][1]))
+      best = i;
+  return best;
+}
+
 template <bool NORM, int EPI>
 hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
   if (NORM && p.K > uint32_t(kGemmNormMaxK)) return hipErrorInvalidValue;
-  // (the last four: many columns, as an lm_head's, where a wide tile has fewer bytes of A beside its W)
-  const uint32_t tile[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64},  {48, 64},
-                              {64, 64}, {16, 128}, {32, 128}, {48, 128}, {64, 128}};
-  int best = 0;
-  for (int i = 1; i < 11; i++)
-    if (tile_cost(p, tile[i][0], tile[i][1]) < tile_cost(p, tile[best][0], tile[best][1])) best = i;
-  switch (best) {
+  switch (slice_tile(p)) {
     case 0: return launch_kslice_t<NORM, EPI, 1, 1, 8, 4>(p, st);
     case 1: return launch_kslice_t<NORM, EPI, 1, 2, 8, 2>(p, st);
     case 2: return launch_kslice_t<NORM, EPI, 2, 2, 8, 2>(p, st);
@@ -1202,9 +1207,13 @@ struct WideTile {
 };
 constexpr WideTile kWideTiles[] = {{64, 128}, {64, 192}, {128, 128}, {128, 192}, {128, 256}};
 
-// Clocks of a launch over bm x bn tiles: rounds of 256 workgroups, each K / 32 phases of the longer
-// of its MFMAs (16 clocks each, per SIMD) and its LDS traffic (128 bytes a clock: the fragments four
-// waves read and the block that is written), plus what a workgroup costs besides (fill and drain).
+// What the tiles of a launch are ranked by: rounds of 256 workgroups, each K / 32 phases of the longer of
+// its MFMAs (16 clocks each, per SIMD) and its LDS traffic (128 bytes a clock: the fragments four waves
+// read and the block that is written), plus what a workgroup costs besides (fill and drain). The clocks
+// are about half of those measured; the tile is the best of the five within 0.3% on average over 143
+// shapes of 65 to 2048 rows (us, in the order of kWideTiles: 512 x 6144 x 1024 24.8, 18.1, 22.0, 26.7, 32.6;
+// 1024 x 6144 x 1024 38.4, 34.2, 42.1, 29.6, 33.8; 2048 x 4096 x 1024 51.4, 48.7, 45.7, 52.3, 37.5), at worst
+// 13% above it (700 x 8192 x 4096 119 on 64 x 192, 105 on 128 x 256).
 uint64_t wide_cost(uint32_t M, uint32_t N, uint32_t kz, uint32_t splits, uint32_t bm, uint32_t bn) {
   const uint64_t wgs = uint64_t((uint64_t(M) + bm - 1) / bm) * ((uint64_t(N) + bn - 1) / bn) * splits;
   const uint32_t mt = bm / 32, nt = bn / 32;
@@ -1260,11 +1269,15 @@ hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st) 
   if (norm && epi == kGemmSiluPair) return launch_kslice<true, kGemmSiluPair>(p, st);
   if (!norm && epi == kGemmResAdd) return launch_kslice<false, kGemmResAdd>(p, st);
   if (norm || epi != kGemmStore) return hipErrorInvalidValue;
-  // the k-sliced kernel up to two rounds of its smaller tiles, the wide one past that
-  uint64_t slice = ~uint64_t(0);
-  for (uint32_t bm : {32u, 48u, 64u}) slice = std::min(slice, tile_cost(p, bm, 64));
-  const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM &&
-                    std::min({tile_cost(p, 64, 128), tile_cost(p, 64, 192), tile_cost(p, 128, 256)}) < slice;
+  // More than 64 rows: the k-sliced kernel while its largest tile makes one round of 256 workgroups (us, it and
+  // the wide one, each on its own tile: 130 x 6144 x 1024 9.5 and 12.8, 333 x 4096 x 1024 11.1 and 13.0; past it
+  // 512 x 6144 x 1024 24.2 and 18.1, 333 x 6144 x 1024 18.8 and 16.2), but its two largest tiles only over a K that
+  // makes up for their sums through LDS (48 x 128: K = 320 8.0 and 7.2, 1024 11.2 and 13.2; 64 x 128: 96 6.7 and
+  // 5.5, 1024 17.1 and 15.3, 1664 21.5 and 19.7, 2048 26.7 and 28.3, 3040 30.4 and 34.4).
+  const auto& tile = kSliceTiles[slice_tile(p)];
+  const uint32_t area = tile[0] * tile[1], deep = area >= 64 * 128 ? 2048 : area >= 48 * 128 ? 672 : 0;
+  const bool rounds = (uint64_t(p.M) + 63) / 64 * ((uint64_t(p.N) + 127) / 128) > 256;
+  const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM && (rounds || p.K < deep);
   return wide ? launch_wide<kGemmStore, false>(p, 1, BatchAttnParams{}, st) : launch_kslice<false, kGemmStore>(p, st);
 }
 

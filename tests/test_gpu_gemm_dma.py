@@ -1,6 +1,6 @@
 """The GEMMs that load their operands straight into LDS (qe_op_gemm_bf16) at the edges of their
-tiles: every k-sliced tile (16 x 16 .. 64 x 128) and every wide one (64 x 128, 64 x 192 with three
-and two slots, 128 x 256), ragged rows and columns, k of one 32-deep step, an odd number of steps,
+tiles: every k-sliced tile (16 x 16 .. 64 x 128) and every wide one (64 x 128, 64 x 192, 128 x 128,
+128 x 192, 128 x 256), both sides of the choice between the two kernels, ragged rows and columns, k of one 32-deep step, an odd number of steps,
 fewer 64-deep blocks than waves, and an output whose rows are not 16-byte aligned."""
 import numpy as np
 import pytest
@@ -17,6 +17,8 @@ SHAPES = [
     (8, 1024, 3072), (3, 1022, 96), (7, 6146, 1056), (5, 80002, 288), (8, 65538, 32),
     # k-sliced over many columns: 16 x 128, 32 x 128, 48 x 128, 64 x 128
     (12, 70002, 288), (24, 40002, 96), (40, 40002, 96), (64, 40002, 64),
+    # the longest K on a wide tile of one round, the shortest on the k-sliced kernel's 64 x 128
+    (512, 4094, 1984), (512, 4094, 2048),
     # wide
     (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 128), (1025, 6146, 320), (2047, 4098, 64),
 ]
