@@ -1048,21 +1048,22 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
     const bool split_attn =
         m->rows_split_attn && (rows_per_kv == 1 || rows_per_kv == 2 || rows_per_kv == 4 || rows_per_kv == 8);
     // input_layernorm + q|k|v (cpu_inference.rs:129-132); long chunks do the q/k norm, RoPE and K/V
-    // append in the GEMM's epilogue, the others in the attention launch (or k_qk_rope before the
-    // split kernel)
+    // append in the GEMM's epilogue, passes of 5 to 64 rows in the attention launch, the others in
+    // k_qk_rope (in the attention launch every token block would do it again for all the keys before it:
+    // +3 to 8% of a prefill of 65 to 512 tokens at widths that are no multiple of 64)
+    const bool attn_appends = M <= qe::kGemmSliceMaxM && !split_attn;
     if (wide) {
       const qe::GemmParams g{bxs, H, nullptr, w.w_qkv, M, QD + 2 * KD, H, bqkv, QD + 2 * KD, eps, 0};
       HIP_TRY(qe::launch_gemm_qk_rope(g, a, s));
     } else {
       if ((rc = gemm(bx, H, w.w_in, w.w_qkv, QD + 2 * KD, H, bqkv, QD + 2 * KD, qe::kGemmStore))) return rc;
-      if (split_attn) HIP_TRY(qe::launch_qk_rope(a, s));
+      if (!attn_appends) HIP_TRY(qe::launch_qk_rope(a, s));
     }
     // multi-stream prefill: the attention reads the previous chunks' K/V rows of this layer,
     // appended on other streams. The event is recorded after this chunk's own wait, so that it
     // stands for the K/V rows of this chunk and of every chunk before it (chunk i waits for
     // chunk i-1 only, whatever the number of streams).
     if (cs && cs->wait_kv) HIP_TRY(hipStreamWaitEvent(s, cs->wait_kv[l], 0));
-    const bool attn_appends = !wide && !split_attn;  // the attention launch itself appends the K/V rows
     if (cs && cs->kv_done && !attn_appends) HIP_TRY(hipEventRecord(cs->kv_done[l], s));
     uint32_t merge_splits = 0;  // > 0: o_proj merges this many attention runs in its prologue
     if (split_attn) {
