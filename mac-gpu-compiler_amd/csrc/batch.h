@@ -24,7 +24,7 @@ constexpr int kBatchMaxRuns = 32;
 // eps; K <= kGemmNormMaxK) when the launch asks for the norm. kGemmSiluPair: W rows 2i / 2i+1 are
 // gate_i / up_i and C[m][i] = silu(gate) * up. N even, K % 32 == 0, lda % 4 == 0.
 // The launches of a chunk (launch_gemm_split, launch_gemm_silu_split, launch_gemm_qk_rope) take A as split rows:
-// every f32 value as hi + lo bf16, 8 hi then 8 lo (16 bytes each) per 8 values. K % 64 == 0.
+// every f32 value as hi + lo bf16, 8 hi then 8 lo (16 bytes each) per 8 values.
 struct GemmParams {
   const float* A;
   uint32_t lda;
@@ -40,6 +40,12 @@ struct GemmParams {
 // Verify passes and chunks of up to kGemmSliceMaxM rows run the projections on k_gemm_kslice over
 // f32 rows, norms and residuals within; longer chunks on k_gemm_wide over split rows.
 constexpr uint32_t kGemmSliceMaxM = 64;
+// Whether a chunk of M rows takes split rows and k_gemm_wide (H, I: hidden and intermediate size). At widths
+// that are no multiple of 64 that is from 320 tiles of 64 x 128 of gate|up (prefill, us, k_gemm_kslice / split
+// rows: hidden 1056 / intermediate 3104 350 tokens 818 / 889, 400 912 / 918, 450 939 / 867; 544 / 1568 600 566 /
+// 617, 800 720 / 669; 2080 / 4064 256 509 / 579, 350 625 / 620, 400 720 / 656; 1056 / 3104 in one chunk of 2048 4180 /
+// 2380), otherwise from 65 rows.
+bool chunk_on_split_rows(uint32_t M, uint32_t H, uint32_t I);
 constexpr int kGemmNormMaxK = 4096;
 
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their

@@ -1239,14 +1239,15 @@ template <int EPI, bool SPLIT, int BM, int BN, int NS>
 hipError_t launch_wide_t(const GemmParams& p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
   const uint64_t wgs = (uint64_t(p.M) + BM - 1) / BM * ((uint64_t(p.N) + BN - 1) / BN) * splits;
   if (hipError_t e = check_grid(wgs, 512)) return e;
-  hipLaunchKernelGGL((k_gemm_wide<EPI, SPLIT, BM, BN, NS>), dim3(uint32_t(wgs)), dim3(512), 0, st, p.A, p.W, p.gain, p.C,
-                     p.lda, p.M, p.N, p.K, p.ldc, p.kz, qa);
+  auto* k = p.kz % 64 ? &k_gemm_wide<EPI, SPLIT, BM, BN, NS, true> : &k_gemm_wide<EPI, SPLIT, BM, BN, NS, false>;
+  hipLaunchKernelGGL(k, dim3(uint32_t(wgs)), dim3(512), 0, st, p.A, p.W, p.gain, p.C, p.lda, p.M, p.N, p.K, p.ldc, p.kz,
+                     qa);
   return hipGetLastError();
 }
 
 template <int EPI, bool SPLIT>
 hipError_t launch_wide(GemmParams p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
-  if (splits == 0 || p.K % (64 * splits)) return hipErrorInvalidValue;
+  if (splits == 0 || p.K % splits || p.K / splits % (splits == 1 ? 32 : 64)) return hipErrorInvalidValue;
   p.kz = p.K / splits;
   const WideTile t = wide_tile(p.M, p.N, p.kz, splits, EPI == kGemmQkRope);
   if (t.bm == 64 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 64, 128, 4>(p, splits, qa, st);
@@ -1277,8 +1278,13 @@ hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st) 
   const auto& tile = kSliceTiles[slice_tile(p)];
   const uint32_t area = tile[0] * tile[1], deep = area >= 64 * 128 ? 2048 : area >= 48 * 128 ? 672 : 0;
   const bool rounds = (uint64_t(p.M) + 63) / 64 * ((uint64_t(p.N) + 127) / 128) > 256;
-  const bool wide = p.K % 64 == 0 && p.M > kGemmSliceMaxM && (rounds || p.K < deep);
+  const bool wide = p.M > kGemmSliceMaxM && (rounds || p.K < deep);
   return wide ? launch_wide<kGemmStore, false>(p, 1, BatchAttnParams{}, st) : launch_kslice<false, kGemmStore>(p, st);
+}
+
+bool chunk_on_split_rows(uint32_t M, uint32_t H, uint32_t I) {
+  if (M <= kGemmSliceMaxM || H % 32 || I % 32) return false;
+  return (H % 64 == 0 && I % 64 == 0) || ceil_div(M, 64) * ceil_div(2 * I, 128) > 320;
 }
 
 uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K) {

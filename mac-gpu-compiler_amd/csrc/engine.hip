@@ -994,14 +994,14 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
   const size_t layer_kv = size_t(c.num_key_value_heads) * kv->max_seq * D * el;
   hipStream_t s = xb ? xb->stream : m->stream;
   const float eps = c.rms_norm_eps;
-  // Up to kGemmSliceMaxM rows (or widths that are no multiples of 64) the k-sliced GEMM computes each
-  // norm within and adds residuals in its epilogue. Past that, what the GEMMs read is written split
+  // In short passes (chunk_on_split_rows) the k-sliced GEMM computes each norm within and adds
+  // residuals in its epilogue. In longer ones, what the GEMMs read is written split
   // into bf16 halves by whatever computes it: bxs holds the current norm of x, from the reduction
   // that finishes each split o_proj / down (residual add + the next norm in one pass).
   // Up to kMvRowsMaxM rows (gate|up: 3; o_proj and down into few columns: kMvResAddMaxM) the projections are matvecs
   // over the M token rows: each weight is loaded once per pass, the norm is computed per row in the
   // kernel and the residual is added in its epilogue. The lm_head is a matvec up to kMvRowsMaxM rows.
-  const bool wide = M > qe::kGemmSliceMaxM && H % 64 == 0 && I % 64 == 0 && QD % 64 == 0;
+  const bool wide = qe::chunk_on_split_rows(M, H, I);
   const bool mv = m->mv_rows && M <= qe::kMvRowsMaxM;
   auto gemm = [&](const float* A, uint32_t lda, const uint16_t* gain, const uint16_t* W, uint32_t N, uint32_t K,
                   float* C, uint32_t ldc, int epi) -> int {

@@ -289,9 +289,12 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_kslice(QE_GEMM_ARGS, float eps
 }
 
 // ---------------------------------------------------------------------------------------------
-// GEMM for many rows: tile BM (m) x BN (n), K a multiple of 64, eight waves as 2 x 2 (a quarter of the
-// tile each) x the two 32-deep halves of every 64-deep stage. The stages of both operands are loaded
-// straight into a ring of NS LDS slots, NS - 1 ahead, one barrier per stage, in whole 128-byte lines
+// GEMM for many rows: tile BM (m) x BN (n), eight waves as 2 x 2 (a quarter of the tile each) x the two
+// 32-deep halves of every 64-deep stage. TAIL: K is an odd number of halves and the last stage has one (its
+// upper places are filled with the lower half again, which nothing reads; as a test in every stage of one
+// kernel it cost the other shapes 2 to 5%). 2048 x 6144 x 1056: 61 us, 82 k-sliced; 2048 x 6144 x 96 18.7, 31.
+// The stages of both operands are loaded straight into a ring of NS LDS slots, NS - 1 ahead, one barrier per
+// stage, in whole 128-byte lines
 // (with every CU loading, L2 gives a CU 115 B/ns in lines and 70 in halves of them): A rows of 256
 // bytes (chunk c of 16 bytes at place (c & 8) | ((c ^ row) & 7)), then W rows of 128 bytes (chunk c at
 // place c ^ (row & 7)).
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_kslice(QE_GEMM_ARGS, float eps
 // power). Two other schedules of the same tiles (the two halves in antiphase; fragments read a stage
 // ahead) ran at the same rate per stage and started 0.6 - 1.1 us later.
 // ---------------------------------------------------------------------------------------------
-template <int EPI, bool SPLIT, int BM, int BN, int NS>
+template <int EPI, bool SPLIT, int BM, int BN, int NS, bool TAIL>
 __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, BatchAttnParams qa) {
   const GemmParams p{A, lda, gain, W, M, N, K, C, ldc, 0.f, kz};
   constexpr int MT = BM / 32, NT = BN / 32;
@@ -322,7 +325,7 @@ __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, Ba
   const int grp = wave >> 2, wm = wave & 1, wn = (wave >> 1) & 1;
   const uint32_t ncol = ceil_div(p.N, uint32_t(BN)), tiles = ncol * ceil_div(p.M, uint32_t(BM));
   const uint32_t z = blockIdx.x / tiles, t = blockIdx.x % tiles, m0 = t / ncol * BM, n0 = t % ncol * BN;
-  const uint32_t nst = p.kz / 64, lds0 = lds_address(smem);
+  const uint32_t nst = TAIL ? p.kz / 64 + 1 : p.kz / 64, lds0 = lds_address(smem);
   // tile column of fragment j's first column
   auto col = [&](int j) __attribute__((always_inline)) {
     return HALF_HEADS ? 64 * (j / (NT / 2)) + 32 * wn + 16 * (j % (NT / 2)) : 16 * (wn * NT + j);
@@ -339,8 +342,14 @@ __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, Ba
     const uint32_t r = 8 * (wave + 8 * i) + (lane >> 3), lc = (lane & 7) ^ (r & 7);
     wsrc[i] = reinterpret_cast<const uint8_t*>(p.W + size_t(min(n0 + r, p.N - 1)) * p.K + size_t(z) * p.kz) + lc * 16;
   }
-  auto issue = [&](uint32_t slot) __attribute__((always_inline)) {
+  auto issue = [&](uint32_t s, uint32_t slot) __attribute__((always_inline)) {
     const uint32_t l = lds0 + slot * SBYTES;
+    if (TAIL && s == nst - 1) {  // lanes of the upper half (lc & 8, lc & 4 above) stay within the row
+#pragma unroll
+      for (int i = 0; i < AI; i++) asrc[i] -= lane & 8 ? 128 : 0;
+#pragma unroll
+      for (int i = 0; i < WI; i++) wsrc[i] -= (lane ^ (lane >> 3)) & 4 ? 64 : 0;
+    }
 #pragma unroll
     for (int i = 0; i < AI; i++) {
       dma16(l + uint32_t(wave + 8 * i) * 1024, asrc[i]);
@@ -363,7 +372,7 @@ __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, Ba
   const uint32_t w0 = ABYTES + li * 128 + ((4 * grp + kg) ^ (li & 7)) * 16;
 #pragma unroll
   for (int i = 0; i < NS - 1; i++)
-    if (uint32_t(i) < nst) issue(i);
+    if (uint32_t(i) < nst) issue(i, i);
   uint32_t slot = 0;
   for (uint32_t s = 0; s < nst; s++) {
     // this wave's loads of stage s have landed and its reads of the previous stage have returned;
@@ -372,6 +381,7 @@ __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, Ba
     wait_lds();
     __builtin_amdgcn_s_barrier();
     asm volatile("" : : : "memory");
+    if (TAIL && s == nst - 1 && grp) break;  // (the last stage: nothing is left to issue)
     const uint8_t* sp = smem + slot * SBYTES;
     f32x4 x[MT], y[MT];
     bf16x8 w[NT];
@@ -382,7 +392,7 @@ __global__ __launch_bounds__(512) void k_gemm_wide(QE_GEMM_ARGS, uint32_t kz, Ba
     }
 #pragma unroll
     for (int j = 0; j < NT; j++) w[j] = *reinterpret_cast<const bf16x8*>(sp + w0 + col(j) * 128);
-    if (s + NS - 1 < nst) issue(slot == 0 ? NS - 1 : slot - 1);
+    if (s + NS - 1 < nst) issue(s + NS - 1, slot == 0 ? NS - 1 : slot - 1);
 #pragma unroll
     for (int i = 0; i < MT; i++) {
       bf16x8 hi, lo;

@@ -1,7 +1,7 @@
 """Chunks of more than 64 tokens: their GEMMs on split rows (norm, attention and SwiGLU outputs held
 as bf16 halves) against the same prompt token by token, at ragged rows, odd numbers of 64-deep
 stages, a last column tile that holds one of its two heads, and widths that are no multiple of 64
-(the k-sliced GEMMs at any number of rows)."""
+(the k-sliced GEMMs up to 576 rows of "half_stages", then a half stage at the end of every product)."""
 import numpy as np
 import pytest
 
@@ -13,12 +13,15 @@ CONFIGS = {
     "tiny": qe.Config(256, 512, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999),
     "odd_stages": qe.Config(320, 448, 2, 4, 4, 128, 1000, 1e-6, 1e6, 999),
     "half_stage": qe.Config(288, 480, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999),
+    "half_stages": qe.Config(288, 2080, 2, 4, 2, 128, 1000, 1e-6, 1e6, 999),
     "93_heads": qe.Config(256, 512, 1, 31, 31, 128, 1000, 1e-6, 1e6, 999),
 }
 
 
 @pytest.mark.parametrize("name,n,kv", [("tiny", 65, "f32"), ("tiny", 129, "bf16"), ("tiny", 1025, "f32"),
                                        ("odd_stages", 200, "f32"), ("half_stage", 150, "f32"),
+                                       ("half_stages", 576, "f32"), ("half_stages", 577, "f32"),
+                                       ("half_stages", 1100, "bf16"), ("half_stages", 2047, "f32"),
                                        ("93_heads", 2001, "f32")])
 def test_chunk_matches_token_by_token(gpu, tmp_path, name, n, kv):
     model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 7, CONFIGS[name]))

@@ -21,6 +21,8 @@ SHAPES = [
     (512, 4094, 1984), (512, 4094, 2048),
     # wide
     (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 128), (1025, 6146, 320), (2047, 4098, 64),
+    # wide with a half stage at the end (k no multiple of 64), from the only one to one past the ring
+    (449, 4096, 32), (512, 6144, 32), (513, 6142, 96), (1025, 6146, 160), (2047, 4098, 288), (512, 12290, 1056),
 ]
 
 
