@@ -1249,6 +1249,19 @@ template <int EPI, bool SPLIT>
 hipError_t launch_wide(GemmParams p, uint32_t splits, const BatchAttnParams& qa, hipStream_t st) {
   if (splits == 0 || p.K % splits || p.K / splits % (splits == 1 ? 32 : 64)) return hipErrorInvalidValue;
   p.kz = p.K / splits;
+  if constexpr (EPI == kGemmStore) {
+    // A short K where even the largest tile makes more than one round: two workgroups a CU (rings of two
+    // slots), so that one writes its block while the other loads and multiplies; of 64 x 128 and 64 x 192 the
+    // one with the fewer columns for the busiest CU. us, one workgroup a CU / two: 2048 x 6144 x 256 27.0 / 22.1,
+    // x 384 32.9 / 27.3, x 96 18.7 / 16.2, 2048 x 5110 x 256 26.8 / 19.9; with 256 tiles of 128 x 256 2048 x 4096 x
+    // 256 16.7 / 17.3.
+    const uint64_t rows = (uint64_t(p.M) + 63) / 64, t128 = rows * ((uint64_t(p.N) + 127) / 128),
+                   t192 = rows * ((uint64_t(p.N) + 191) / 192);
+    if (p.kz <= 512 && (uint64_t(p.M) + 127) / 128 * ((uint64_t(p.N) + 255) / 256) > 256)
+      return (t128 + 255) / 256 * 128 < (t192 + 255) / 256 * 192
+                 ? launch_wide_t<EPI, SPLIT, 64, 128, 2>(p, splits, qa, st)
+                 : launch_wide_t<EPI, SPLIT, 64, 192, 2>(p, splits, qa, st);
+  }
   const WideTile t = wide_tile(p.M, p.N, p.kz, splits, EPI == kGemmQkRope);
   if (t.bm == 64 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 64, 128, 4>(p, splits, qa, st);
   if (t.bm == 128 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 128, 128, 3>(p, splits, qa, st);

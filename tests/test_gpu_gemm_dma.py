@@ -1,6 +1,6 @@
 """The GEMMs that load their operands straight into LDS (qe_op_gemm_bf16) at the edges of their
 tiles: every k-sliced tile (16 x 16 .. 64 x 128) and every wide one (64 x 128, 64 x 192, 128 x 128,
-128 x 192, 128 x 256), both sides of the choice between the two kernels, ragged rows and columns, k of one 32-deep step, an odd number of steps,
+128 x 192, 128 x 256, and the first two with rings of two slots), both sides of the choice between the two kernels, ragged rows and columns, k of one 32-deep step, an odd number of steps,
 fewer 64-deep blocks than waves, and an output whose rows are not 16-byte aligned."""
 import numpy as np
 import pytest
@@ -20,9 +20,12 @@ SHAPES = [
     # the longest K on a wide tile of one round, the shortest on the k-sliced kernel's 64 x 128
     (512, 4094, 1984), (512, 4094, 2048),
     # wide
-    (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 128), (1025, 6146, 320), (2047, 4098, 64),
+    (65, 12290, 64), (449, 4096, 192), (512, 6144, 1024), (513, 6142, 576), (1025, 6146, 640), (2047, 4098, 576),
+    # two workgroups a CU over a short k: 64 x 128 and 64 x 192
+    (2000, 5110, 64), (1025, 7426, 512), (1500, 6144, 512), (2047, 8194, 64),
     # wide with a half stage at the end (k no multiple of 64), from the only one to one past the ring
-    (449, 4096, 32), (512, 6144, 32), (513, 6142, 96), (1025, 6146, 160), (2047, 4098, 288), (512, 12290, 1056),
+    (449, 4096, 32), (449, 4096, 288), (512, 6144, 32), (512, 6144, 416), (513, 6142, 544), (1025, 6146, 1056),
+    (2047, 4098, 608), (2000, 5110, 32), (2000, 5110, 96), (1500, 6144, 32), (1500, 6144, 160),
 ]
 
 
