@@ -82,6 +82,9 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 constexpr uint32_t kBatchDefaultChunk = 512;  // tokens per chunk of qe_prefill_batch (chunk = 0)
 constexpr uint32_t kBatchMaxChunk = 2048;
+// chunks of qe_prefill_batch above this many tokens go over several streams (one stream / two, ms: 2048 tokens
+// in chunks of 64 42.8 / 34.0, of 48 55.7 / 41.9, of 33 76.5 / 57.6; 130 in chunks of 64 3.36 / 2.89)
+constexpr uint32_t kStreamMinChunk = 32;
 constexpr uint32_t kCopySlots = 8;  // pinned pieces of a verify pass's logits in flight to the host
 constexpr size_t kCopyPiece = size_t(640) << 10;
 constexpr uint32_t kVerifyMaxTokens = 64;  // tokens of one qe_verify call
@@ -1604,11 +1607,11 @@ int qe_prefill_batch(qe_model* model, const uint32_t* ids, uint64_t n, uint64_t 
     if (ids[i] >= model->cfg.vocab_size) return fail(QE_ERR_ARG, "token %u at %llu >= vocab", ids[i], (unsigned long long)i);
   int rc = ensure_batch(model, chunk, 0);
   if (rc) return rc;
-  // chunks of more than kGemmSliceMaxM tokens go round-robin over up to prefill_streams streams
+  // chunks of more than kStreamMinChunk tokens go round-robin over up to prefill_streams streams
   // and buffer sets: chunk i's layer-l attention waits for chunk i-1's layer-l K/V rows, and
   // otherwise the chunks' launches overlap (each chunk runs the same kernels as on one stream)
   const uint64_t n_chunks = (n + chunk - 1) / chunk;
-  const int S = chunk > qe::kGemmSliceMaxM ? int(std::min<uint64_t>(model->prefill_streams, n_chunks)) : 1;
+  const int S = chunk > kStreamMinChunk ? int(std::min<uint64_t>(model->prefill_streams, n_chunks)) : 1;
   if (S > 1 && (rc = ensure_streams(model, chunk, S))) return rc;
   if ((rc = upload_ids(model, ids, n))) return rc;
   auto stream_of = [&](int set) { return set ? model->extra[set - 1].stream : model->stream; };

@@ -36,3 +36,23 @@ def test_chunk_matches_token_by_token(gpu, tmp_path, name, n, kv):
     for i in range(2):  # the K/V rows of every position are what the next steps attend to
         d = np.max(np.abs(model.forward(int(ids[i]), n + i, a) - model.forward(int(ids[i]), n + i, b)))
         assert d < tol, f"step {i}: {d}"
+
+
+# chunks whose attention launch appends their K/V rows (33 and 64 tokens), chunks on the k-sliced GEMMs with
+# k_qk_rope (widths that are no multiple of 64), and chunks on split rows with a half stage
+@pytest.mark.parametrize("name,n,chunk", [("tiny", 500, 33), ("tiny", 600, 64), ("half_stage", 600, 64),
+                                          ("half_stage", 600, 96), ("half_stage", 700, 128), ("half_stages", 2000, 640)])
+def test_streams_change_no_result(gpu, tmp_path, monkeypatch, name, n, chunk):
+    path = qe.write_random_checkpoint(str(tmp_path), 7, CONFIGS[name])
+    ids = qe.random_prompt(5, n, 1000)
+
+    def run(streams):
+        monkeypatch.setenv("QE_PREFILL_STREAMS", streams)  # read when the model loads
+        model = qe.Model.load_model(path)
+        cache = qe.KVCache(model, n + 2)
+        return model.prefill_batch(ids, 0, cache, chunk=chunk), model.forward(int(ids[0]), n, cache)
+
+    one = run("1")
+    for streams in ("2", "3", "4"):
+        for got, want in zip(run(streams), one):
+            np.testing.assert_array_equal(got, want, err_msg=f"{streams} streams")
