@@ -158,7 +158,7 @@ __global__ __launch_bounds__(512) void k_attn_causal_bf(const float* q_in, const
   const int rw = wave & 3, kh = wave >> 2;
   const uint32_t g = blockIdx.x, mb = blockIdx.y * TOK, run = blockIdx.z;
   if (run >= runs) {  // a prefetch workgroup (whole workgroup, before any load)
-    l2_prefetch_tiles(p.pf.pf, (run - runs) * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + g,
+    l2_prefetch_tiles<512>(p.pf.pf, (run - runs) * gridDim.x * gridDim.y + blockIdx.y * gridDim.x + g,
                       reinterpret_cast<uint32_t*>(p.att));
     return;
   }

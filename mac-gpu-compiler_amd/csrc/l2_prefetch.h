@@ -61,11 +61,12 @@ __device__ __forceinline__ void l2_prefetch(const L2Prefetch (&pf)[kMaxPrefetch]
 // For consumers that each read more than one prefetch workgroup loads (a GEMM's column tile j,
 // whose row tiles and K splits all run on XCD j % 8): the chunks of consumers j = x, x + 8,
 // x + 16, ... of each target (x = this XCD) form one list, and prefetch workgroup q loads piece
-// q / 8 of it, 256 x 16 chunks. A launch carries 8 x tile_prefetch_slots() such workgroups at
+// q / 8 of it, 4096 chunks (4096 / THREADS per thread). A launch carries 8 x tile_prefetch_slots() such workgroups at
 // consecutive linear ids, so each XCD gets every piece once.
+template <uint32_t THREADS>
 __device__ __forceinline__ void l2_prefetch_tiles(const L2Prefetch (&pf)[kMaxPrefetch], uint32_t q,
                                                   uint32_t* sink) {
-  constexpr uint32_t KMAX = 16;
+  constexpr uint32_t KMAX = 4096 / THREADS;
   const uint32_t x = xcc_id(), tid = threadIdx.x;
   uint32_t span[kMaxPrefetch], tot = 0;
 #pragma unroll
@@ -73,12 +74,12 @@ __device__ __forceinline__ void l2_prefetch_tiles(const L2Prefetch (&pf)[kMaxPre
     span[t] = pf[t].w && x < pf[t].n_cwg ? ceil_div(pf[t].n_cwg - x, 8u) * pf[t].cw_chunks : 0;
     tot += span[t];
   }
-  const uint32_t base = (q / 8) * 256 * KMAX;
+  const uint32_t base = (q / 8) * 4096;
   if (base >= tot) return;
   uint4 v[KMAX];
 #pragma unroll
   for (uint32_t k = 0; k < KMAX; k++) {
-    uint32_t i = min(base + tid + 256 * k, tot - 1);
+    uint32_t i = min(base + tid + THREADS * k, tot - 1);
     const uint16_t* w = pf[0].w;
     uint32_t cw = pf[0].cw_chunks, nc = pf[0].n_chunks, sp = span[0];
 #pragma unroll
