@@ -5,6 +5,7 @@
 
 #include <cstdint>
 
+#include "gemm_choice.h"
 #include "kernels.h"
 
 namespace qe {
@@ -37,15 +38,6 @@ struct GemmParams {
   uint32_t kz;  // the depth of one K split (set by the launches)
 };
 
-// Verify passes and chunks of up to kGemmSliceMaxM rows run the projections on k_gemm_kslice over
-// f32 rows, norms and residuals within; longer chunks on k_gemm_wide over split rows.
-constexpr uint32_t kGemmSliceMaxM = 64;
-// Whether a chunk of M rows takes split rows and k_gemm_wide (H, I: hidden and intermediate size). At widths
-// that are no multiple of 64 that is from 320 tiles of 64 x 128 of gate|up (prefill, us, k_gemm_kslice / split
-// rows: hidden 1056 / intermediate 3104 350 tokens 818 / 889, 400 912 / 918, 450 939 / 867; 544 / 1568 600 566 /
-// 617, 800 720 / 669; 2080 / 4064 256 509 / 579, 350 625 / 620, 400 720 / 656; 1056 / 3104 in one chunk of 2048 4180 /
-// 2380), otherwise from 65 rows.
-bool chunk_on_split_rows(uint32_t M, uint32_t H, uint32_t I);
 constexpr int kGemmNormMaxK = 4096;
 
 // Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
@@ -103,8 +95,6 @@ struct BatchAttnParams {
 
 hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st);
 // ---- a chunk's GEMMs: A as split rows (see GemmParams) ----
-// K splits for launch_gemm_split: enough workgroups to fill the chip (1 when K does not split)
-uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K);
 // partial sums of `splits` K ranges: C[z][m][n], z < splits, ldc = N
 hipError_t launch_gemm_split(const GemmParams& p, uint32_t splits, hipStream_t st);
 // C[m] = split row of silu(gate) * up over the interleaved gate/up rows of W (ldc >= N / 2)

@@ -1137,21 +1137,6 @@ hipError_t launch_mv_rows(const MvRowsParams& p, bool norm, int epi, hipStream_t
 
 namespace {
 
-// The tile of a k-sliced launch: the workgroups are dealt over 256 CUs, so its time goes with the
-// bytes the busiest CU loads (rounds of 256 x one workgroup's), plus what a workgroup costs besides
-// its loads, worth about 60 KB of them. Measured (us, M x N x K): 9 x 6144 x 1024 on 16 x 32 tiles
-// 3.5, 16 x 48 4.0; 64 x 6144 x 1024 on 32 x 48 5.8, 32 x 64 6.0, 16 x 32 7.3; 130 x 1024 x 3072 on
-// 32 x 32 7.5, 32 x 64 9.0, 16 x 32 9.5; 130 x 4096 x 1024 on 48 x 64 7.3, 64 x 64 7.9, 32 x 64 10.1;
-// 512 x 1024 x 3072 on 32 x 64 15.1, 48 x 64 17.6, 64 x 64 20.4. N = 151936, K = 1024 (an lm_head): 5 rows
-// on 16 x 128 54.7, 64 x 128 76.5; 12 rows 56.6 and 77.9; 24 rows on 32 x 128 67.1, 64 x 128 79.7; 40 rows on
-// 48 x 128 80.7, 64 x 128 84.8. Deeper rings (all of a wave's steps in flight) were slower: down of 5 rows
-// 7.3 against 6.2 traced.
-uint64_t tile_cost(const GemmParams& p, uint32_t bm, uint32_t bn) {
-  const uint64_t wgs = (uint64_t(p.M) + bm - 1) / bm * ((uint64_t(p.N) + bn - 1) / bn);
-  const uint32_t rows = bm == 16 && p.M <= 8 ? 8 : bm;  // (HALF)
-  return (wgs + 255) / 256 * (uint64_t(4 * rows + 2 * bn) * p.K + 60 * 1024);
-}
-
 hipError_t check_grid(uint64_t wgs, uint32_t threads) {
   return wgs * threads < (uint64_t(1) << 32) ? hipSuccess : hipErrorInvalidValue;
 }
@@ -1172,21 +1157,10 @@ hipError_t launch_kslice_t(const GemmParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// (the last four: many columns, as an lm_head's, where a wide tile has fewer bytes of A beside its W)
-constexpr uint32_t kSliceTiles[][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 48}, {32, 64},  {48, 64},
-                                       {64, 64}, {16, 128}, {32, 128}, {48, 128}, {64, 128}};
-int slice_tile(const GemmParams& p) {
-  int best = 0;
-  for (int i = 1; i < 11; i++)
-    if (tile_cost(p, kSliceTiles[i][0], kSliceTiles[i][1]) < tile_cost(p, kSliceTiles[best][0], kSliceTiles[best][1]))
-      best = i;
-  return best;
-}
-
 template <bool NORM, int EPI>
 hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
   if (NORM && p.K > uint32_t(kGemmNormMaxK)) return hipErrorInvalidValue;
-  switch (slice_tile(p)) {
+  switch (slice_tile(p.M, p.N, p.K)) {
     case 0: return launch_kslice_t<NORM, EPI, 1, 1, 8, 4>(p, st);
     case 1: return launch_kslice_t<NORM, EPI, 1, 2, 8, 2>(p, st);
     case 2: return launch_kslice_t<NORM, EPI, 2, 2, 8, 2>(p, st);
@@ -1199,40 +1173,6 @@ hipError_t launch_kslice(const GemmParams& p, hipStream_t st) {
     case 9: return launch_kslice_t<NORM, EPI, 3, 8, 4, 2>(p, st);
     default: return launch_kslice_t<NORM, EPI, 4, 8, 4, 2>(p, st);
   }
-}
-
-// ---- k_gemm_wide: the tile ----
-struct WideTile {
-  uint32_t bm, bn;
-};
-constexpr WideTile kWideTiles[] = {{64, 128}, {64, 192}, {128, 128}, {128, 192}, {128, 256}};
-
-// What the tiles of a launch are ranked by: rounds of 256 workgroups, each K / 32 phases of the longer of
-// its MFMAs (16 clocks each, per SIMD) and its LDS traffic (128 bytes a clock: the fragments four waves
-// read and the block that is written), plus what a workgroup costs besides (fill and drain). The clocks
-// are about half of those measured; the tile is the best of the five within 0.3% on average over 143
-// shapes of 65 to 2048 rows (us, in the order of kWideTiles: 512 x 6144 x 1024 24.8, 18.1, 22.0, 26.7, 32.6;
-// 1024 x 6144 x 1024 38.4, 34.2, 42.1, 29.6, 33.8; 2048 x 4096 x 1024 51.4, 48.7, 45.7, 52.3, 37.5), at worst
-// 13% above it (700 x 8192 x 4096 119 on 64 x 192, 105 on 128 x 256).
-uint64_t wide_cost(uint32_t M, uint32_t N, uint32_t kz, uint32_t splits, uint32_t bm, uint32_t bn) {
-  const uint64_t wgs = uint64_t((uint64_t(M) + bm - 1) / bm) * ((uint64_t(N) + bn - 1) / bn) * splits;
-  const uint32_t mt = bm / 32, nt = bn / 32;
-  const uint32_t mfma = mt * nt * 2 * 16, lds = 32 * (2 * mt + nt) + bm + bn / 2;
-  return (wgs + 255) / 256 * (uint64_t(kz / 32) * std::max(mfma, lds) + 7000);
-}
-
-WideTile wide_tile(uint32_t M, uint32_t N, uint32_t kz, uint32_t splits, bool heads) {
-  WideTile best{};
-  uint64_t cost = ~uint64_t(0);
-  for (const WideTile& t : kWideTiles) {
-    if (heads && t.bn % kHeadDim) continue;
-    const uint64_t c = wide_cost(M, N, kz, splits, t.bm, t.bn);
-    if (c < cost) {
-      cost = c;
-      best = t;
-    }
-  }
-  return best;
 }
 
 template <int EPI, bool SPLIT, int BM, int BN, int NS>
@@ -1250,19 +1190,11 @@ hipError_t launch_wide(GemmParams p, uint32_t splits, const BatchAttnParams& qa,
   if (splits == 0 || p.K % splits || p.K / splits % (splits == 1 ? 32 : 64)) return hipErrorInvalidValue;
   p.kz = p.K / splits;
   if constexpr (EPI == kGemmStore) {
-    // A short K where even the largest tile makes more than one round: two workgroups a CU (rings of two
-    // slots), so that one writes its block while the other loads and multiplies; of 64 x 128 and 64 x 192 the
-    // one with the fewer columns for the busiest CU. us, one workgroup a CU / two: 2048 x 6144 x 256 27.0 / 22.1,
-    // x 384 32.9 / 27.3, x 96 18.7 / 16.2, 2048 x 5110 x 256 26.8 / 19.9; with 256 tiles of 128 x 256 2048 x 4096 x
-    // 256 16.7 / 17.3.
-    const uint64_t rows = (uint64_t(p.M) + 63) / 64, t128 = rows * ((uint64_t(p.N) + 127) / 128),
-                   t192 = rows * ((uint64_t(p.N) + 191) / 192);
-    if (p.kz <= 512 && (uint64_t(p.M) + 127) / 128 * ((uint64_t(p.N) + 255) / 256) > 256)
-      return (t128 + 255) / 256 * 128 < (t192 + 255) / 256 * 192
-                 ? launch_wide_t<EPI, SPLIT, 64, 128, 2>(p, splits, qa, st)
-                 : launch_wide_t<EPI, SPLIT, 64, 192, 2>(p, splits, qa, st);
+    const GemmTile two = wide_pair_tile(p.M, p.N, p.K);
+    if (two.bn == 128) return launch_wide_t<EPI, SPLIT, 64, 128, 2>(p, splits, qa, st);
+    if (two.bn == 192) return launch_wide_t<EPI, SPLIT, 64, 192, 2>(p, splits, qa, st);
   }
-  const WideTile t = wide_tile(p.M, p.N, p.kz, splits, EPI == kGemmQkRope);
+  const GemmTile t = wide_tile(p.M, p.N, p.kz, splits, EPI == kGemmQkRope);
   if (t.bm == 64 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 64, 128, 4>(p, splits, qa, st);
   if (t.bm == 128 && t.bn == 128) return launch_wide_t<EPI, SPLIT, 128, 128, 3>(p, splits, qa, st);
   if (t.bm == 128 && t.bn == 256) return launch_wide_t<EPI, SPLIT, 128, 256, 2>(p, splits, qa, st);
@@ -1283,29 +1215,8 @@ hipError_t launch_gemm(const GemmParams& p, bool norm, int epi, hipStream_t st) 
   if (norm && epi == kGemmSiluPair) return launch_kslice<true, kGemmSiluPair>(p, st);
   if (!norm && epi == kGemmResAdd) return launch_kslice<false, kGemmResAdd>(p, st);
   if (norm || epi != kGemmStore) return hipErrorInvalidValue;
-  // More than 64 rows: the k-sliced kernel while its largest tile makes one round of 256 workgroups (us, it and
-  // the wide one, each on its own tile: 130 x 6144 x 1024 9.5 and 12.8, 333 x 4096 x 1024 11.1 and 13.0; past it
-  // 512 x 6144 x 1024 24.2 and 18.1, 333 x 6144 x 1024 18.8 and 16.2), but its two largest tiles only over a K that
-  // makes up for their sums through LDS (48 x 128: K = 320 8.0 and 7.2, 1024 11.2 and 13.2; 64 x 128: 96 6.7 and
-  // 5.5, 1024 17.1 and 15.3, 1664 21.5 and 19.7, 2048 26.7 and 28.3, 3040 30.4 and 34.4).
-  const auto& tile = kSliceTiles[slice_tile(p)];
-  const uint32_t area = tile[0] * tile[1], deep = area >= 64 * 128 ? 2048 : area >= 48 * 128 ? 672 : 0;
-  const bool rounds = (uint64_t(p.M) + 63) / 64 * ((uint64_t(p.N) + 127) / 128) > 256;
-  const bool wide = p.M > kGemmSliceMaxM && (rounds || p.K < deep);
-  return wide ? launch_wide<kGemmStore, false>(p, 1, BatchAttnParams{}, st) : launch_kslice<false, kGemmStore>(p, st);
-}
-
-bool chunk_on_split_rows(uint32_t M, uint32_t H, uint32_t I) {
-  if (M <= kGemmSliceMaxM || H % 32 || I % 32) return false;
-  return (H % 64 == 0 && I % 64 == 0) || ceil_div(M, 64) * ceil_div(2 * I, 128) > 320;
-}
-
-uint32_t gemm_splits(uint32_t M, uint32_t N, uint32_t K) {
-  // 64 x 128 tiles: split while that leaves CUs without one
-  const uint32_t tiles = ceil_div(N, 128) * ceil_div(M, 64);
-  uint32_t z = 1;
-  while (z < 8 && tiles * z < 256 && K % (128 * z) == 0) z *= 2;
-  return z;
+  return gemm_on_wide(p.M, p.N, p.K) ? launch_wide<kGemmStore, false>(p, 1, BatchAttnParams{}, st)
+                                     : launch_kslice<false, kGemmStore>(p, st);
 }
 
 hipError_t launch_gemm_split(const GemmParams& p, uint32_t splits, hipStream_t st) {
