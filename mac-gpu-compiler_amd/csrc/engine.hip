@@ -1079,7 +1079,7 @@ int enqueue_batch(qe_model* m, qe_kv* kv, uint32_t M, uint32_t start, const uint
       // 8 rows (4 tokens): two workgroups of 4 rows per KV head halve each one's score and
       // P.V work for a second read of the K/V runs, mostly from L2 (verify of 4 tokens at
       // position 2048: 1.321 -> 1.261 ms; 4 workgroups of 2 rows: 1.399 ms; 4 rows: no change)
-      if (rows_per_kv == 8) r.row_split = 2;
+      if (rows_per_kv == 8 && M > 1) r.row_split = 2;  // (a workgroup holds whole tokens)
       if (m->l2_prefetch && mv) {
         // as in the decode step: the attention is latency-bound, so extra workgroups load this
         // layer's gate|up (up to 3 tokens: as the multi-row matvec reads it) and

@@ -103,3 +103,13 @@ def test_rows_on_both_sides_of_the_residual_rule(gpu, tmp_path, hidden, k):
     rows = model.verify(ids[20:], 20, a)
     for i in range(k):  # activations in 16 bits, two layers and the lm_head: some 2^-17 each
         assert rel(rows[i], model.forward(int(ids[20 + i]), 20 + i, b)) < 4e-5, f"row {i}"
+
+
+def test_single_rows_at_eight_q_heads_per_kv_head(gpu, tmp_path):
+    """a verify of one token, and a chunk's last token alone, where its 8 q heads are all rows of a KV head"""
+    model = qe.Model.load_model(qe.write_random_checkpoint(str(tmp_path), 7, qe.Config(256, 512, 1, 8, 1, 128, 1000,
+                                                                                       1e-6, 1e6, 999)))
+    ids = qe.random_prompt(5, 66, 1000)
+    a, b = qe.KVCache(model, 66), qe.KVCache(model, 66)
+    assert rel(model.prefill_batch(ids[:65], 0, a, chunk=64), model.prefill(ids[:65], 0, b)) < 4e-5
+    assert rel(model.verify(ids[65:], 65, a)[0], model.forward(int(ids[65]), 65, b)) < 4e-5
