@@ -16,10 +16,10 @@
 //                         16 MiB chunk, for the same chunk every launch, 8 rotating chunks
 //                         (128 MiB, within the MALL) and 48 (768 MiB): whether L2 keeps lines
 //                         from one launch to the next
-//   qe_stage_pmc --gemm   the chunked prefill's GEMM instead (launch_gemm, no norm, plain store),
-//                         3 launches at each of M x N x K = 2048 x 4096 x 1024 (q|k|v of a
-//                         2048-token chunk: k_gemm_wide), 512 x 6144 x 1024 and 512 x 4096 x 1024
-//                         (gate|up and q|k|v of a 512-token chunk: k_gemm_wide), for the
+//   qe_stage_pmc --gemm   the products of a 512-token and of a 2048-token chunk instead, as the
+//                         prefill launches them (split rows: q|k|v with the q/k norm, RoPE and K/V
+//                         append, gate|up with silu, of 512 rows the partials of down), 3 launches
+//                         each, then the op's (launch_gemm, f32 rows, plain store) 512 x 6144 x 1024, for the
 //                         matrix-core counters (SQ_INSTS_MFMA, SQ_VALU_MFMA_BUSY_CYCLES, ...);
 //                         --reps R launches per shape instead of 3, --random fills A and W with
 //                         hashed values in [-1, 1) and [-1/64, 1/64) instead of constants (the
@@ -169,27 +169,54 @@ int main(int argc, char** argv) {
     CK(hipSetDevice(0));
     hipStream_t gs;
     CK(hipStreamCreate(&gs));
-    const uint32_t shapes[3][3] = {{2048, 4096, 1024}, {512, 6144, 1024}, {512, 4096, 1024}};
+    enum { kQkv, kGateUp, kDown, kOp };
+    const char* const names[] = {"q|k|v", "gate|up", "down", "op"};
+    const uint32_t shapes[6][4] = {{kQkv, 512, 4096, 1024},  {kGateUp, 512, 6144, 1024},  {kDown, 512, 1024, 3072},
+                                   {kQkv, 2048, 4096, 1024}, {kGateUp, 2048, 6144, 1024}, {kOp, 512, 6144, 1024}};
+    // q|k|v: q rows, one layer's f32 cache, RoPE rows and norm gains (any finite values)
+    const uint32_t GH = 16, GKV = 8, GD = qe::kHeadDim, top = 2048;
+    qe::BatchAttnParams a{};
+    a.q = dalloc<float>(size_t(top) * GH * GD);
+    float* cache = dalloc<float>(2 * size_t(GKV) * top * GD);
+    float* rope = dalloc<float>(size_t(top) * GD);
+    uint16_t* gains = dalloc<uint16_t>(2 * GD);
+    k_fill_f32<<<1024, 256, 0, gs>>>(rope, size_t(top) * GD, 0.5f);
+    k_fill_f32<<<1, 256, 0, gs>>>(reinterpret_cast<float*>(gains), GD, 0.0078125f);
+    a.k_cache = cache;
+    a.v_cache = cache + size_t(GKV) * top * GD;
+    a.rope = rope;
+    a.q_norm = gains;
+    a.k_norm = gains + GD;
+    a.max_seq = top;
+    a.n_heads = GH;
+    a.n_kv = GKV;
+    a.eps = 1e-6f;
     for (const auto& sh : shapes) {
-      const uint32_t M = sh[0], N = sh[1], K = sh[2];
+      const uint32_t what = sh[0], M = sh[1], N = sh[2], K = sh[3], z = what == kDown ? qe::gemm_splits(M, N, K) : 1;
       float* A = dalloc<float>(size_t(M) * K);
       uint16_t* W = dalloc<uint16_t>(size_t(N) * K);
-      float* C = dalloc<float>(size_t(M) * N);
+      float* C = dalloc<float>(size_t(z) * M * N);
       if (random) {
-        k_fill_hash_f32<<<1024, 256, 0, gs>>>(A, size_t(M) * K, 1.0f);
+        if (what == kOp) k_fill_hash_f32<<<1024, 256, 0, gs>>>(A, size_t(M) * K, 1.0f);
+        else k_fill_hash_bf16<<<1024, 256, 0, gs>>>(reinterpret_cast<uint16_t*>(A), 2 * size_t(M) * K, 1.0f);
         k_fill_hash_bf16<<<1024, 256, 0, gs>>>(W, size_t(N) * K, 1.0f / 64);
       } else {
         k_fill_f32<<<1024, 256, 0, gs>>>(A, size_t(M) * K, 0.5f);
         // bf16 pairs (0, 0.0078125): any finite values give the same matrix-core work
         k_fill_f32<<<1024, 256, 0, gs>>>(reinterpret_cast<float*>(W), size_t(N) * K / 2, 0.0078125f);
       }
-      const qe::GemmParams g{A, K, nullptr, W, M, N, K, C, N, 1e-6f, 0};
-      for (int r = 0; r < reps; r++) CK(qe::launch_gemm(g, false, qe::kGemmStore, gs));
+      const qe::GemmParams g{A, K, nullptr, W, M, N, K, C, what == kGateUp ? N / 2 : N, 1e-6f, 0};
+      a.M = M;
+      for (int r = 0; r < reps; r++)
+        CK(what == kQkv      ? qe::launch_gemm_qk_rope(g, a, gs)
+           : what == kGateUp ? qe::launch_gemm_silu_split(g, gs)
+           : what == kDown   ? qe::launch_gemm_split(g, z, gs)
+                             : qe::launch_gemm(g, false, qe::kGemmStore, gs));
       CK(hipStreamSynchronize(gs));
       CK(hipFree(A));
       CK(hipFree(W));
       CK(hipFree(C));
-      std::printf("gemm %u x %u x %u: %d launches%s\n", M, N, K, reps, random ? " (hashed operands)" : "");
+      std::printf("%s %u x %u x %u: %d launches%s\n", names[what], M, N, K, reps, random ? " (hashed operands)" : "");
     }
     return 0;
   }
