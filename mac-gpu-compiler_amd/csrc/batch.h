@@ -13,7 +13,7 @@ namespace qe {
 // kGemmPartial: split over K; split z writes its partial sums to C + z M ldc (launch_gemm_split)
 // kGemmQkRope (launch_gemm_qk_rope): the q|k|v projection of a chunk with the per-head q/k
 // RMSNorm, RoPE and the K/V append of k_qk_rope in its epilogue
-// kGemmSiluSplit (launch_gemm_split_rows): kGemmSiluPair written as split rows
+// kGemmSiluSplit (launch_gemm_silu_split): kGemmSiluPair written as split rows
 enum GemmEpilogue {
   kGemmStore = 0, kGemmResAdd = 1, kGemmSiluPair = 2, kGemmPartial = 3, kGemmQkRope = 4, kGemmSiluSplit = 5
 };
@@ -40,8 +40,8 @@ struct GemmParams {
 
 constexpr int kGemmNormMaxK = 4096;
 
-// Verify passes and chunks of up to kMvRowsMaxM tokens run the projections as a matvec over their
-// token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
+// Verify passes and chunks of up to kMvRowsMaxM tokens run the projections (gate|up: of up to 3) as a
+// matvec over their token rows: out[m][.] for m < M from x [M][cols] (see launch_mv_rows). Each further row adds its
 // own products and lane reductions to every wave of that matvec, so past a few rows the k-sliced GEMM
 // on the matrix cores is faster. With a residual and few weight rows (o_proj and down at a hidden size
 // of up to 1024) that is from 7 rows, as the GEMM has at most 64 workgroups of 16 columns for 256 CUs

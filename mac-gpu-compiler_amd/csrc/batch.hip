@@ -6,7 +6,7 @@
 //   GEMMs          C[m][n] = sum_k A'[m][k] W[n][k], A' = A or an RMSNorm of its rows, split into
 //                  hi + lo bf16 so the products keep ~16 mantissa bits (gemm_dma.h); epilogues store /
 //                  residual add / silu(gate)*up / q-k norm + RoPE + K/V append (cpu_inference.rs:225-257):
-//                  k_gemm_kslice (<= 64 rows), k_gemm_wide (more); k_mv_rows (<= 4 rows, f32 FMA)
+//                  k_gemm_kslice (<= 64 rows), k_gemm_wide (more: gemm_choice.h); k_mv_rows (few rows, f32 FMA)
 //   k_resadd_norm_split  residual add of a split GEMM, then the next norm, split for the next GEMM
 //   k_qk_rope      per token and head: q/k RMSNorm + RoPE, K/V append   (cpu_inference.rs:134-141)
 //   k_attn_causal_bf  token m attends positions 0..start+m, split bf16 MFMA (cpu_inference.rs:144-162)
@@ -677,8 +677,8 @@ __global__ __launch_bounds__(256) void k_embed_rows_v(const uint16_t* __restrict
 }
 
 // ---------------------------------------------------------------------------------------------
-// Matvec over the NV = M token rows of a short verify pass or chunk (M <= kMvRowsMaxM): the
-// decode step's matvec layout. A row group of TPR threads covers one weight row in 8-column
+// Matvec over the NV = M token rows of a short verify pass or chunk (M <= kMvRowsMaxM, with a residual
+// kMvResAddMaxM): the decode step's matvec layout. A row group of TPR threads covers one weight row in 8-column
 // chunks (CPT per thread) and RR rows per group; each weight chunk is loaded once (128-bit) and
 // multiplied by the NV token rows in f32 FMA, so the weights stream once per pass as in a decode
 // step. With NORM every row group computes the sum of squares of each token row over its own
@@ -1267,8 +1267,10 @@ hipError_t launch_qk_rope(const BatchAttnParams& p, hipStream_t st) {
 }
 
 // Row blocks per wave of k_attn_causal_bf: two (each LDS fragment feeds twice the MFMAs, each staged
-// tile twice the rows) once that leaves a workgroup for every second CU. 2048 tokens in one chunk 7.62 ms
-// with two, 7.89 with one; in chunks of 512 9.47 and 9.29; 333 tokens 2.35 and 2.26.
+// tile twice the rows) from 1024 rows, whatever the heads (prefill from position 0, two / one block: 700 rows
+// 1.00 to 1.02, 1024 0.98 to 1.004, 2048 0.92 to 0.98, over 8 to 32 q heads on 1 to 16 KV heads; 16 over 8, us: 512
+// rows 2426 / 2370, 1024 3850 / 3897, 2048 7270 / 7530). After 2048 cached positions two would pay from 512
+// rows at 16 q heads (3024 / 3203), not at 8.
 uint32_t attn_row_blocks(uint32_t M) { return M >= 1024 ? 2 : 1; }
 
 template <int G, int RB>

@@ -177,7 +177,8 @@ struct qe_model {
   // decode attention launches also load the next weights into L2 (QE_L2_PREFETCH=0 turns it off)
   bool l2_prefetch = true;
   // verify passes and chunks of up to kMvRowsMaxM tokens run their projections as multi-row
-  // matvecs (QE_MV_ROWS=0: on the k-sliced GEMM)
+  // matvecs (gate|up of up to 3 tokens, o_proj and down into up to kMvResAddMaxN columns of up to
+  // kMvResAddMaxM; QE_MV_ROWS=0: on the k-sliced GEMM)
   bool mv_rows = true;
   // passes of at most 8 / (q heads per KV head) tokens (a verify of up to 4 rows) attend on the
   // decode step's split kernel, all their q heads of a KV head sharing one read of its K/V
@@ -186,7 +187,7 @@ struct qe_model {
   // and their o_proj merges those runs in its prologue when they are few (QE_MV_MERGE=0: a
   // merge launch of its own)
   bool mv_merge = true;
-  // chunks of more than 64 tokens: the causal attention launch also loads o_proj's weights into the
+  // chunks on split rows (of more than 64 tokens): the causal attention launch also loads o_proj's weights into the
   // L2 of the XCDs that will read them (QE_PREFILL_PREFETCH=0 turns it off)
   bool prefill_prefetch = true;
   // ... and their lm_head is the decode step's matvec over all their rows, each row's logits

@@ -142,7 +142,7 @@ __device__ __forceinline__ void emit4(const GemmParams& p, uint32_t m, uint32_t 
 // HALF (M <= 8): rows 8 .. 15 of the A tile are not loaded and have no place in the slot. Their lanes
 // multiply what lies there (W), which reaches only the sums of those rows, and those are not written.
 // Bound: at these sizes the bytes each CU pulls from L2 (about 50 B/ns with all CUs loading); the
-// tile is the one with the fewest on the busiest CU (launch_kslice).
+// tile is the one with the fewest on the busiest CU (slice_tile).
 // ---------------------------------------------------------------------------------------------
 template <bool NORM, int EPI, int MT, int NT, int NW, int NS, bool HALF>
 __global__ __launch_bounds__(64 * NW) void k_gemm_kslice(QE_GEMM_ARGS, float eps) {

@@ -24,12 +24,9 @@ def bf16_round(a: np.ndarray) -> np.ndarray:
     return u.astype(np.uint16)
 
 
-# m <= 32 runs the skinny (split over k) kernel: one m-tile on 16 or 8 waves, or two m-tiles;
-# m <= 64 the LDS-tiled 64 x 64 kernel (k % 64 == 0) or the register-only one (k = 96); larger m
-# the 64-row kernel up to 1024 rows (192-column tiles where that fills the CUs more evenly: 512 x
-# 6144, 1000 x 6144), then the 128-row tile kernel with 64 columns per tile, or 128 once that gives
-# 256 tiles (2048 x 6144);
-# odd stage counts (k = 32, 96), ragged rows and columns (n = 1000) included
+# m <= 64 runs the k-sliced kernel; larger m the k-sliced or the wide one (512 x 6144, 513 x 6144, 1000 x
+# 6144 and 2048 x 6144 on 64 x 192 to 128 x 256 tiles); odd stage counts (k = 32, 96), ragged rows and columns
+# (n = 1000) included. tests/test_gpu_gemm_dma.py goes through the tiles.
 @pytest.mark.parametrize("m,n,k", [(1, 64, 32), (5, 128, 64), (64, 1024, 1024), (100, 4096, 1024),
                                    (512, 1024, 3072), (37, 6144, 1024), (4, 32768, 1024), (3, 1000, 256),
                                    (16, 2048, 1024), (8, 4096, 3072), (17, 6144, 1024), (32, 1024, 3072),
@@ -79,12 +76,12 @@ def test_tiny_prefill_batch_matches_oracle(gpu, tiny_ckpt, n_prompt, chunk):
         assert toks[i] == tok
 
 
-# k <= 4: the projections are multi-row matvecs over the k token rows; k = 5, 9, 17: the skinny
-# GEMM; "skinny": k = 4 with the multi-row matvec switched off
+# k <= 4: the projections are multi-row matvecs over the k token rows (gate|up of 4 on the GEMM); k = 5: o_proj
+# and down; k = 9, 17: the k-sliced GEMM; "gemm": k = 4 with the multi-row matvec switched off
 @pytest.mark.parametrize("k,path", [(1, "rows"), (2, "rows"), (3, "rows"), (4, "rows"), (5, "rows"), (9, "rows"),
-                                    (17, "rows"), (4, "skinny")])
+                                    (17, "rows"), (4, "gemm")])
 def test_tiny_verify_matches_oracle(gpu, tiny_ckpt, k, path, monkeypatch):
-    if path == "skinny":
+    if path == "gemm":
         monkeypatch.setenv("QE_MV_ROWS", "0")  # read when the model loads
     m = qe.Model.load_model(tiny_ckpt)
     om = oracle.Model(tiny_ckpt)
