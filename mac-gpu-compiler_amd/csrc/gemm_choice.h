@@ -105,7 +105,9 @@ inline bool gemm_on_wide(uint32_t M, uint32_t N, uint32_t K) {
 // that are no multiple of 64 that is from 320 tiles of 64 x 128 of gate|up (prefill, us, k_gemm_kslice / split
 // rows: hidden 1056 / intermediate 3104 350 tokens 818 / 889, 400 912 / 918, 450 939 / 867; 544 / 1568 600 566 /
 // 617, 800 720 / 669; 2080 / 4064 256 509 / 579, 350 625 / 620, 400 720 / 656; 1056 / 3104 in one chunk of 2048 4180 /
-// 2380), otherwise from 65 rows.
+// 2380), otherwise from 65 rows (1024 / 3072, 28 layers: 200 tokens 1927 / 1841, 256 2063 / 1952, 333 2543 / 2244;
+// below that the other way round, 65 1429 / 1653, 100 1545 / 1743, 130 1751 / 1786: one more block of 64 rows would
+// pay on k_gemm_kslice).
 inline bool chunk_on_split_rows(uint32_t M, uint32_t H, uint32_t I) {
   if (M <= kGemmSliceMaxM || H % 32 || I % 32) return false;
   return (H % 64 == 0 && I % 64 == 0) || gemm_tiles(M, 64) * gemm_tiles(2 * uint64_t(I), 128) > 320;
